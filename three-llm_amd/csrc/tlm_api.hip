@@ -103,7 +103,7 @@ struct tlm_linear {
   uint4* w = nullptr;
   uint16_t* s = nullptr;
   GemvPlan plan;
-  float* part = nullptr;  // op-level partials [splits][N]
+  float* part = nullptr;  // op-level scratch [N]: the gated MLP's h, a result whose y overlaps x
   // paired layout (fused MLP gate|up, N = 2I): canonical gate row i sits in
   // tile i / 32, lane i % 32; up row I + i in the same tile, lane 32 + i % 32
   int pair_half = 0;  // I when paired, else 0
@@ -589,7 +589,7 @@ int tlm_linear_create(tlm_ctx* ctx, int fmt, int n_out, int k_in, const void* we
   int rc = linear_alloc(ctx, fmt, n_out, k_in, false, &L);
   if (rc) return rc;
   rc = linear_write_rows(L, 0, n_out, weights, scales);
-  if (rc == TLM_OK && hipMalloc(&L->part, sizeof(float) * (size_t)L->plan.splits * L->N) != hipSuccess)
+  if (rc == TLM_OK && hipMalloc(&L->part, sizeof(float) * (size_t)L->N) != hipSuccess)
     rc = fail(TLM_ERR_OOM, "TLMLinear: partials allocation failed");
   if (rc) {
     tlm_linear_destroy(L);
@@ -622,18 +622,37 @@ int tlm_linear_dequant(tlm_linear* L, float* host_out) {
   return TLM_OK;
 }
 
+static OpGemvArgs op_gemv_args(const tlm_linear* L, const float* x, const float* bias, float* y) {
+  OpGemvArgs a;
+  memset(&a, 0, sizeof a);
+  a.w = L->w;
+  a.s = L->s;
+  a.N = L->N;
+  a.C = L->C;
+  a.K = L->K;
+  a.x = x;
+  a.bias = bias;
+  a.y = y;
+  return a;
+}
+
+// Whether [p, p + n) and [q, q + m) share an address.
+static bool overlap(const float* p, size_t n, const float* q, size_t m) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a < b + m * sizeof(float) && b < a + n * sizeof(float);
+}
+
 int tlm_op_linear(tlm_linear* L, const float* x, const float* bias, float* y) {
   if (!L || !x || !y) return fail(TLM_ERR_INVALID, "TLMLinear: null argument");
-  GemvArgs a;
-  const bool direct = L->plan.splits == 1;
-  fill_gemv_args(a, L, direct ? y : L->part);
-  a.in = x;
-  a.bias = direct ? bias : nullptr;
-  if (!launch_linear(L, PRO_COPY, a, L->ctx->stream))
+  hipStream_t st = L->ctx->stream;
+  // y may be (part of) x: every block reads all of x, so y is then written afterwards
+  const bool apart = !overlap(x, L->K, y, L->N);
+  if (!launch_op_gemv(wfmt(L->fmt), false, op_gemv_args(L, x, apart ? bias : nullptr, apart ? y : L->part),
+                      L->ctx->cus, st))
     return fail(TLM_ERR_STATE, "TLMLinear: no kernel variant for this shape");
   CHECK_LAUNCH("TLMLinear");
-  if (!direct) {
-    launch_reduce(L->part, L->plan.splits, L->N, bias, L->N, y, L->ctx->stream);
+  if (!apart) {
+    launch_reduce(L->part, 1, L->N, bias, L->N, y, st);
     CHECK_LAUNCH("TLMLinear");
   }
   return TLM_OK;
@@ -686,27 +705,15 @@ int tlm_op_gated_mlp(tlm_linear* gu, tlm_linear* down, const float* x, float* y)
   if (gu->N != 2 * down->K || gu->K != down->N)
     return fail(TLM_ERR_INVALID, "TLMGatedMLP: gate/up %dx%d does not match down %dx%d", gu->N, gu->K, down->N,
                 down->K);
+  // gate|up with SwiGLU, then down: h (fp32, in the gate|up linear's scratch)
+  // is all that passes between the two launches
   hipStream_t st = gu->ctx->stream;
-  GemvArgs a;
-  fill_gemv_args(a, gu, gu->part);
-  a.in = x;
-  if (!launch_linear(gu, PRO_COPY, a, st))
+  if (!launch_op_gemv(wfmt(gu->fmt), true, op_gemv_args(gu, x, nullptr, gu->part), gu->ctx->cus, st))
     return fail(TLM_ERR_STATE, "TLMGatedMLP: no kernel variant for this shape");
   CHECK_LAUNCH("TLMGatedMLP");
-  GemvArgs b;
-  const bool direct = down->plan.splits == 1;
-  fill_gemv_args(b, down, direct ? y : down->part);
-  b.pin = gu->part;
-  b.n_pin = gu->plan.splits;
-  b.pin_stride = gu->N;
-  b.up_off = down->K;
-  if (!launch_linear(down, PRO_SWIGLU, b, st))
+  if (!launch_op_gemv(wfmt(down->fmt), false, op_gemv_args(down, gu->part, nullptr, y), gu->ctx->cus, st))
     return fail(TLM_ERR_STATE, "TLMGatedMLP: no kernel variant for this shape");
   CHECK_LAUNCH("TLMGatedMLP");
-  if (!direct) {
-    launch_reduce(down->part, down->plan.splits, down->N, nullptr, down->N, y, st);
-    CHECK_LAUNCH("TLMGatedMLP");
-  }
   return TLM_OK;
 }
 

@@ -32,7 +32,6 @@ enum WeightFmt { WF_F16 = 1, WF_Q4 = 2 };
 enum Prologue {
   PRO_COPY = 0,    // x = in
   PRO_RMS = 1,     // x = rmsnorm(base + sum_j pin[j]) * w
-  PRO_SWIGLU = 2,  // x = silu(sum_j pin[j][k]) * (sum_j pin[j][up_off + k])
   PRO_ATTN = 3,    // x = flash-decoding combine of the attention chunk partials
   PRO_RMS2 = 4,    // PRO_RMS for K up to 8 elements per thread (chosen by launch_gemv)
   PRO_RMSF = 5,    // x = rmsnorm(sum of the kRep fixed-point replicas acc_in) * w
@@ -88,12 +87,11 @@ struct GemvArgs {
   unsigned long long* zero_ptr;      // optional: the grid zeroes zero_ptr[0, zero_n)
   int zero_n;
   const int* ctrl;
-  const float* pin;    // partials to add (RMS) / gate|up partials (SWIGLU)
+  const float* pin;    // partials to add (RMS)
   int n_pin, pin_stride;
   const float* norm_w;
   float eps;
   float* xout;         // block (0,0) stores base + sum pin here (residual stream)
-  int up_off;          // SWIGLU: offset of the up rows in pin
   // PRO_ATTN: chunk partials of the attention kernel
   const float* pacc;   // [Hq][nsplit][D]
   const float* pml;    // [Hq][nsplit][2]
@@ -152,10 +150,24 @@ struct AttnArgs {
   int gqa;              // long windows: the matrix-core kernel (one block per kv head and chunk)
 };
 
+// One vector through a linear in one launch (tlm_ops.hip).
+struct OpGemvArgs {
+  const uint4* w;      // [T][C][64] 16-byte chunks, plain row order
+  const uint16_t* s;   // q4 scales [T][C][64]
+  int N, C, K;
+  const float* x;      // fp32 [K]
+  const float* bias;   // [N] or null
+  float* y;            // [N] (SWIGLU: [N / 2])
+  int cps, x_vec;      // set by the launcher: chunks per slice of x in LDS; x can be read 16 bytes at a time
+};
+
 // launchers (stream-ordered, graph-capturable: no memset, no host sync)
 // launchers return false when no compiled variant matches (nothing is launched)
 // waves in {4, 8}; nch in {1, 2, 4, 8}: chunks per wave and load batch
 bool launch_gemv(int fmt, int pro, int waves, int nch, dim3 grid, const GemvArgs& a, hipStream_t st);
+// one vector through a linear in one launch; swiglu: gate rows [0, N / 2), up
+// rows [N / 2, N), y = silu(gate x) * (up x)
+bool launch_op_gemv(int fmt, bool swiglu, const OpGemvArgs& a, int cus, hipStream_t st);
 // fused MLP: kMlpWaves waves, one block per 32 intermediate indices; nch: gate|up
 // chunks per wave, ndb: down (tile, chunk) items per wave per batch (1, 2, 4)
 bool launch_mlp(int fmt, int nch, int ndb, int blocks, const MlpArgs& a, hipStream_t st);

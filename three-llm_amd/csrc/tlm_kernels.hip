@@ -22,21 +22,6 @@ namespace tlm {
 
 // ------------------------------------------------------------------ GEMV --
 
-// Sum of n <= kMaxPart partial vectors at element k.  The loads are
-// unconditional (indices clamped to valid rows) and only the adds are masked,
-// so all of them are in flight before the first use: a consumer pays one
-// memory round trip however many splits its producer used.  n == 0 reads nothing.
-__device__ __forceinline__ float sum_parts(const float* p, int n, int stride, int k) {
-  if (n <= 0) return 0.f;
-  float v[kMaxPart];
-#pragma unroll
-  for (int j = 0; j < kMaxPart; j++) v[j] = p[(size_t)min(j, n - 1) * stride + k];
-  float s = 0.f;
-#pragma unroll
-  for (int j = 0; j < kMaxPart; j++) s += j < n ? v[j] : 0.f;
-  return s;
-}
-
 __device__ __forceinline__ float4 f4add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 
 // Flash-decoding combine of one output element (query head `row`, dim d) over
@@ -102,7 +87,7 @@ struct GemvPrologue {
   static constexpr int R = (PRO == PRO_RMS2 || PRO == PRO_RMSF2 || PRO == PRO_RMSF2H) ? 2 : 1;  // float4s of the residual row per thread
   float4 x[R], w[R];
   ulonglong2 fx[kRmsF ? R : 1][NREP][2];  // RMSF: the 4 elements' replicas
-  float4 p[2][kMaxPart];  // RMS: partials per float4 (R rows); SWIGLU: [0] gate, [1] up partials
+  float4 p[2][kMaxPart];  // RMS: partials per float4 (R rows)
   static constexpr int kSlotLanes = 8;  // ATTN: lanes sharing one float4, splitting its chunk slots
   static constexpr bool kAttn = PRO == PRO_ATTN || PRO == PRO_ATTN3;
   // chunk slots per lane: 16 per float4 and round trip, or 32 for the long-
@@ -134,9 +119,6 @@ struct GemvPrologue {
     const int kc = min(k0 + 4 * min(f, n4 - 1), a.K - 4);
     if (PRO == PRO_COPY) {
       x[0] = *reinterpret_cast<const float4*>(a.in + kc);
-    } else if (PRO == PRO_SWIGLU) {
-      load_parts(a.pin, a.n_pin, a.pin_stride, kc, p[0]);
-      load_parts(a.pin + a.up_off, a.n_pin, a.pin_stride, kc, p[1]);
     } else if (kAttn) {
       // slots jb + (lane & 7) + 8u of the float4 at f
       const int row = kc / a.att_D, d = kc % a.att_D;
@@ -194,18 +176,6 @@ struct GemvPrologue {
       // (slots past the active count are masked in attn_finish)
       load_slice4(a, kAttn ? tid / kSlotLanes : tid, k0, klen_pad / 4, 0, a.att_nsplit);
     }
-  }
-
-  // silu(gate) * up (TSLSiLUMul.ts:15-29) or the flash-decoding combine of the
-  // attention chunk partials for the float4 loaded by load_slice4.
-  __device__ __forceinline__ float4 value4(const GemvArgs& a, int f, int k0, int n4) {
-    if (PRO == PRO_COPY) return x[0];
-    if (PRO == PRO_SWIGLU) {
-      const float4 g = sum_loaded(p[0], a.n_pin), u = sum_loaded(p[1], a.n_pin);
-      return make_float4(g.x / (1.f + __expf(-g.x)) * u.x, g.y / (1.f + __expf(-g.y)) * u.y,
-                         g.z / (1.f + __expf(-g.z)) * u.z, g.w / (1.f + __expf(-g.w)) * u.w);
-    }
-    return x[0];  // not reached for the attention prologues (attn_finish)
   }
 
   // Flash-decoding combine of the attention chunk partials: eight lanes share
@@ -335,9 +305,6 @@ struct GemvPrologue {
         if (k < a.K) {
           if (PRO == PRO_COPY) {
             y = a.in[k];
-          } else if (PRO == PRO_SWIGLU) {
-            const float g = sum_parts(a.pin, a.n_pin, a.pin_stride, k);
-            y = g / (1.f + __expf(-g)) * sum_parts(a.pin + a.up_off, a.n_pin, a.pin_stride, k);
           } else {
             y = attn_combine_elem(a.pacc, a.pml, k / a.att_D, k % a.att_D, a.att_D, a.att_nsplit, nact);
           }
@@ -351,7 +318,7 @@ struct GemvPrologue {
       for (int fb = 0; fb < n4; fb += nt) {
         const int f = fb + tid;
         if (fb > 0) load_slice4(a, f, k0, n4, 0, 1);
-        float4 y = value4(a, f, k0, n4);
+        float4 y = x[0];
         if (!(f < n4 && k0 + 4 * f < a.K)) y = make_float4(0.f, 0.f, 0.f, 0.f);
         put4<FMT>(xl, xsum, 4 * f, y, f < n4);
       }
@@ -693,22 +660,18 @@ bool launch_gemv(int fmt, int pro, int waves, int nch, dim3 grid, const GemvArgs
   }
 #define GEMV_N(F, P, Wv) GEMV_CASE(F, P, Wv, 1) GEMV_CASE(F, P, Wv, 2) GEMV_CASE(F, P, Wv, 4) GEMV_CASE(F, P, Wv, 8)
 #define GEMV_W(F, P) GEMV_N(F, P, 4) GEMV_N(F, P, 8)
-  GEMV_W(WF_Q4, PRO_COPY)
   GEMV_W(WF_Q4, PRO_RMSF)
   GEMV_W(WF_Q4, PRO_RMSF2)
   GEMV_W(WF_Q4, PRO_RMSFH)
   GEMV_W(WF_Q4, PRO_RMSF2H)
-  GEMV_W(WF_Q4, PRO_SWIGLU)
   GEMV_W(WF_Q4, PRO_ATTN)
   GEMV_W(WF_F16, PRO_ATTN)
   GEMV_W(WF_Q4, PRO_ATTN3)
   GEMV_W(WF_F16, PRO_ATTN3)
-  GEMV_W(WF_F16, PRO_COPY)
   GEMV_W(WF_F16, PRO_RMSF)
   GEMV_W(WF_F16, PRO_RMSF2)
   GEMV_W(WF_F16, PRO_RMSFH)
   GEMV_W(WF_F16, PRO_RMSF2H)
-  GEMV_W(WF_F16, PRO_SWIGLU)
 #undef GEMV_W
 #undef GEMV_N
 #undef GEMV_CASE
