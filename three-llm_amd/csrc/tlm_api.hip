@@ -133,7 +133,6 @@ struct tlm_attn {
   float* pacc = nullptr;
   float* pml = nullptr;
   float* zero_bias = nullptr;  // stands in for an absent QKV bias
-  int* ctrl = nullptr;
 };
 
 struct Layer {
@@ -798,8 +797,8 @@ static int attn_init(tlm_ctx* ctx, const tlm_attn_desc* d, tlm_attn* A, bool own
     HIP_TRY(hipMalloc(&A->vc, cache));
     HIP_TRY(hipMemset(A->kc, 0, cache));
     HIP_TRY(hipMemset(A->vc, 0, cache));
-    HIP_TRY(hipMalloc(&A->ctrl, sizeof(int) * 8));
-    HIP_TRY(hipMemset(A->ctrl, 0, sizeof(int) * 8));
+    if (!attention_one_prepare(d->kv_fmt == TLM_FMT_F32, D))
+      return fail(TLM_ERR_HIP, "TLMAttention: the one-call kernel's LDS was refused");
   }
   return TLM_OK;
 }
@@ -813,7 +812,6 @@ static void attn_free(tlm_attn* A, bool own_cache) {
   if (own_cache) {
     hipFree(A->kc);
     hipFree(A->vc);
-    hipFree(A->ctrl);
   }
 }
 
@@ -879,11 +877,27 @@ int tlm_op_attention(tlm_attn* A, const float* qkv, int position, float* out) {
   if (position < 0 || position >= A->d.max_tokens)
     return fail(TLM_ERR_RANGE, "TLMAttention: position %d outside [0, %d)", position, A->d.max_tokens);
   hipStream_t st = A->ctx->stream;
-  launch_set_ctrl(A->ctrl, 0, position, 0, 0, 0, EmbStage{}, st);
-  const int total = (A->d.heads + 2 * A->d.kv_heads) * A->d.head_dim;
-  const bool lw = long_window(A, position);
-  AttnArgs a = attn_args(A, qkv, 1, total, nullptr, A->ctrl, A->kc, A->vc, out, lw);
-  if (!launch_attention(A->d.kv_fmt == TLM_FMT_F32, A->gmax, a, true, lw, st))
+  const int total = (A->d.heads + 2 * A->d.kv_heads) * A->d.head_dim, D = A->d.head_dim;
+  const bool f32 = A->d.kv_fmt == TLM_FMT_F32;
+  const int n = A->d.sliding_window > 0 ? std::min(position + 1, A->d.sliding_window) : position + 1;
+  // One launch as long as one block per head (or per kv head, on the matrix
+  // cores) is faster than chunks and the kernel that combines them.  us a call,
+  // Llama-3.2-1B heads (head_dim 64) / Llama-3.2-3B (128), with the position in
+  // the launch instead of in a control word that a kernel of its own writes:
+  //   block per head        32 positions 3.4 / 4.9   101 4.8 / 6.5   512 7.7 / 10.5
+  //   block per kv head     32 positions 4.4 / 5.9   101 4.5 / 6.1   512 5.7 / 8.6   701 7.3 / 11.2   1001 8.5 / 14.0
+  //   chunks and a combine  1501 positions 8.3 / 9.7 (as many up to 4 chunks fewer)
+  // Without the matrix-core kernel (fp32 cache, other head_dims) the block per
+  // head serves windows of one pass per wave.
+  const bool per_head = n <= (A->gqa ? 64 : attention_one_positions(f32, D));
+  const bool per_kv_head = !per_head && A->gqa && n <= (D == 64 ? 768 : 512);
+  const bool lw = A->gqa || long_window(A, position);
+  AttnArgs a = attn_args(A, qkv, 1, total, nullptr, nullptr, A->kc, A->vc, out, lw);
+  a.pos = position;
+  if (per_head || per_kv_head) a.nsplit = 1;
+  if (!(per_head      ? launch_attention_one(f32, a, st)
+        : per_kv_head ? launch_gqa_attention_one(a, st)
+                      : launch_attention(f32, A->gmax, a, true, lw, st)))
     return fail(TLM_ERR_STATE, "TLMAttention: no kernel variant for this shape");
   CHECK_LAUNCH("TLMAttention");
   return TLM_OK;

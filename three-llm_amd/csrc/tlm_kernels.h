@@ -9,6 +9,7 @@ constexpr int kTile = 64;      // output rows per tile: one row per lane of a wa
 constexpr int kMaxChunks = 8;  // most 16-byte chunks a wave keeps in flight per batch
 constexpr int kMaxPart = 8;    // partial vectors a consumer folds in with one round trip
 constexpr int kAttnWaves = 4;  // decode attention: waves per block, each a quarter of the block's chunk
+constexpr int kOneWaves = 12;  // one-call decode attention (short windows): most waves per block
 constexpr int kGqaWaves = 8;   // matrix-core decode attention (long windows): waves per block
 constexpr int kGqaTile = 32;   // its positions per wave tile
 constexpr int kGqaPro = 3;     // its q|k|v elements per thread: (G + 2) head_dim <= 3 * 64 kGqaWaves
@@ -136,7 +137,8 @@ struct AttnArgs {
   const float* src;     // q|k|v partial sums [n_src][src_stride]
   int n_src, src_stride;
   const float* bias;    // [(Hq + 2Hkv) D] or null
-  const int* ctrl;      // position at ctrl[C_POS]
+  const int* ctrl;      // position at ctrl[C_POS]; null: pos
+  int pos;
   void* kc;             // [Hkv][max_tokens][D] (this layer)
   void* vc;
   const float* rope_cos;  // [max_tokens][rd/2], attention factor folded in
@@ -183,6 +185,14 @@ constexpr int kMlpWaves = 16;
 bool launch_lm_head(int fmt, int pro, int waves, int nch, dim3 grid, const GemvArgs& a, hipStream_t st);
 // attention chunk partials; with `combine` also the combine kernel writing a.out
 bool launch_attention(bool kv_f32, int gmax, const AttnArgs& a, bool combine, bool long_win, hipStream_t st);
+// the whole window of position a.pos in one launch, one block per query head
+// (n_src 1, nsplit 1; windows up to attention_one_positions); prepare: once per head_dim and
+// cache type, outside stream capture, allows the kernel its LDS
+int attention_one_positions(bool kv_f32, int D);
+bool attention_one_prepare(bool kv_f32, int D);
+bool launch_attention_one(bool kv_f32, const AttnArgs& a, hipStream_t st);
+// the same on the matrix cores, one block per kv head (what gqa_attention_fits covers)
+bool launch_gqa_attention_one(const AttnArgs& a, hipStream_t st);
 // long windows, fp16 cache, head_dim 64 or 128, G <= 16: grid Hkv x nsplit
 bool launch_gqa_attention(const AttnArgs& a, hipStream_t st);
 size_t gemv_smem_bytes(int fmt, int cps, int waves);

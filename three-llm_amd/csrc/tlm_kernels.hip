@@ -847,10 +847,13 @@ int attn_lpp(int D, bool kv_f32) { return head_tiling(attn_dt(D), kv_f32 ? 4 : 2
 
 // LDS of a head_kernel block: one wave region per wave, then (long windows)
 // the merge area [kAttnWaves][2 + DT] (max, sum, unnormalised output of each wave).
+static size_t head_smem_bytes(int D, bool kv_f32, int nw) {
+  const int dt = attn_dt(D), esz = kv_f32 ? 4 : 2;
+  return sizeof(float) * ((size_t)nw * head_wave_floats(dt, esz) + (nw > 1 ? (size_t)nw * (2 + dt) : 0));
+}
 size_t attn_smem_bytes(int gmax, int D, bool kv_f32, bool long_win) {
   (void)gmax;
-  const int dt = attn_dt(D), esz = kv_f32 ? 4 : 2, nw = long_win ? kAttnWaves : 1;
-  return sizeof(float) * ((size_t)nw * head_wave_floats(dt, esz) + (long_win ? (size_t)nw * (2 + dt) : 0));
+  return head_smem_bytes(D, kv_f32, long_win ? kAttnWaves : 1);
 }
 
 
@@ -862,6 +865,10 @@ size_t attn_smem_bytes(int gmax, int D, bool kv_f32, bool long_win) {
 // merge (max, sum, output) in LDS at the end, so the combine downstream folds
 // kAttnWaves times fewer partials, and the block numbering is XCD-aware
 // (below).  The host captures one graph per mode and picks it per position.
+// One call (ONE: tlm_op_attention over a short window): block b = head b with
+// the whole window, spread over as many waves as it holds passes (up to
+// kOneWaves); wave 0's merge writes the output itself, so no combine kernel and
+// no control word are needed, and q|k|v come as one vector.
 // Each wave
 //   * forms its q head and the KV head's new k and v from the QKV partial sums
 //     + bias and applies RoPE (rotate-half, TSLAttention.ts:168-250),
@@ -872,8 +879,8 @@ size_t attn_smem_bytes(int gmax, int D, bool kv_f32, bool long_win) {
 //   * writes (max, sum, unnormalised output) for the combine.
 // All global loads of the first pass are unconditional and issued before the
 // first use; until the merge a wave touches only its own LDS region.
-template <typename KT, int DT, bool LONG>
-__global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(AttnArgs a) {
+template <typename KT, int DT, bool LONG, bool ONE = false>
+__global__ __launch_bounds__(64 * (ONE ? kOneWaves : LONG ? kAttnWaves : 1)) void head_kernel(AttnArgs a) {
   extern __shared__ float sm[];
   constexpr int ESZ = sizeof(KT);
   constexpr HeadTiling TL = head_tiling(DT, ESZ);
@@ -883,7 +890,9 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
   constexpr int KW = DL * ESZ / 4;            // K dwords per lane
   // fp16 cache, head_dim 128: the output dims of a lane are adjacent (P.V)
   constexpr bool PAIRD = !GEN && ESZ == 2 && DT == 128;
-  constexpr int NW = LONG ? kAttnWaves : 1;
+  constexpr int NSRC = ONE ? 1 : kMaxPart;    // q|k|v vectors to add
+  // waves per block (ONE: the launch's choice)
+  const int NW = ONE ? blockDim.x >> 6 : LONG ? kAttnWaves : 1;
   const int G = a.G, b = blockIdx.x;
   int hk, c, h, g;
   if (LONG) {
@@ -904,16 +913,16 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
     hk = h / G;
     g = h % G;
   }
-  const int lane = threadIdx.x & 63, wv = LONG ? threadIdx.x >> 6 : 0;
+  const int lane = threadIdx.x & 63, wv = LONG || ONE ? threadIdx.x >> 6 : 0;
   const int D = GEN ? a.D : DT;
-  const int pos = a.ctrl[C_POS];
+  const int pos = ONE ? a.pos : a.ctrl ? a.ctrl[C_POS] : a.pos;
   if (pos < 0 || pos >= a.max_tokens) return;
   const ChunkPlan cp = chunk_plan(pos, a.window, a.nsplit, a.chmin);
   if (c >= cp.nact) return;
   // the block's chunk [b0, b1), split over nwu <= kAttnWaves waves of at least
   // 32 positions (block-uniform); this wave's part [t0, t1) may be empty
   const int b0 = cp.first + c * cp.chunk, b1 = min(b0 + cp.chunk, pos + 1);
-  const int nwu = LONG ? min(NW, (b1 - b0 + 31) / 32) : 1;
+  const int nwu = ONE ? NW : LONG ? min(NW, (b1 - b0 + 31) / 32) : 1;
   if (nwu == 1 && wv != 0) return;  // one wave does the whole chunk, no merge
   const int sc = (b1 - b0 + nwu - 1) / nwu;
   const int t0 = min(b0 + wv * sc, b1), t1 = min(t0 + sc, b1);
@@ -931,7 +940,7 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
 
   // q (row 0), new k (row 1), new v (row 2): partial sums + bias, element d = lane + 64 e
   const int QS = a.Hq * D, KS = a.Hkv * D;
-  float gp[3][EPL][kMaxPart], gb[3][EPL];
+  float gp[3][EPL][NSRC], gb[3][EPL];
 #pragma unroll
   for (int r = 0; r < 3; r++) {
     const int base = r == 0 ? h * D : r == 1 ? QS + hk * D : QS + KS + hk * D;
@@ -939,7 +948,7 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
     for (int e = 0; e < EPL; e++) {
       const int col = base + min(lane + 64 * e, D - 1);
 #pragma unroll
-      for (int j = 0; j < kMaxPart; j++)
+      for (int j = 0; j < NSRC; j++)
         gp[r][e][j] = a.src[(size_t)max(min(j, a.n_src - 1), 0) * a.src_stride + col];
       gb[r][e] = a.bias[col];
     }
@@ -967,7 +976,7 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
     for (int e = 0; e < EPL; e++) {
       float s = gb[r][e];
 #pragma unroll
-      for (int j = 0; j < kMaxPart; j++) s = fmaf(gp[r][e][j], j < a.n_src ? 1.f : 0.f, s);
+      for (int j = 0; j < NSRC; j++) s = fmaf(gp[r][e][j], j < a.n_src ? 1.f : 0.f, s);
       const int d = lane + 64 * e;
       if (d < D) raw[r * DT + d] = s;
     }
@@ -1065,6 +1074,14 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
     wave_lds_sync();
   }
   const size_t row = (size_t)h * a.nsplit + c;
+  if (nwu == 1 && ONE) {
+#pragma unroll
+    for (int e = 0; e < EPL; e++) {
+      const int d = PAIRD ? 2 * lane + e : lane + 64 * e;
+      if (d < D) a.out[(size_t)h * D + d] = o[e] / l;
+    }
+    return;
+  }
   if (nwu == 1) {  // wave 0 alone: its result is the chunk's partial
 #pragma unroll
     for (int e = 0; e < EPL; e++) {
@@ -1091,41 +1108,121 @@ __global__ __launch_bounds__(64 * (LONG ? kAttnWaves : 1)) void head_kernel(Attn
   }
   __syncthreads();  // every wave of the block reaches this once
   if (wv != 0) return;
+  constexpr int NWM = ONE ? kOneWaves : LONG ? kAttnWaves : 1;
   float M = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < NW; w++) M = fmaxf(M, mg[w * (2 + DT)]);
-  float wsc[NW], L = 0.f;
+  for (int w = 0; w < NWM; w++) M = w < NW ? fmaxf(M, mg[w * (2 + DT)]) : M;
+  float wsc[NWM], L = 0.f;
 #pragma unroll
-  for (int w = 0; w < NW; w++) {
-    const float mw = mg[w * (2 + DT)];
+  for (int w = 0; w < NWM; w++) {
+    const float mw = w < NW ? mg[w * (2 + DT)] : -INFINITY;
     wsc[w] = mw == -INFINITY ? 0.f : __expf(mw - M);
-    L = fmaf(mg[w * (2 + DT) + 1], wsc[w], L);
+    L = w < NW ? fmaf(mg[w * (2 + DT) + 1], wsc[w], L) : L;
   }
   for (int d = lane; d < D; d += 64) {
     float od = 0.f;
 #pragma unroll
-    for (int w = 0; w < NW; w++) od = fmaf(mg[w * (2 + DT) + 2 + d], wsc[w], od);
-    a.pacc[row * D + d] = od;
+    for (int w = 0; w < NWM; w++) od = w < NW ? fmaf(mg[w * (2 + DT) + 2 + d], wsc[w], od) : od;
+    if (ONE) a.out[(size_t)h * D + d] = od / L;
+    else a.pacc[row * D + d] = od;
   }
-  if (lane == 0) {
+  if (!ONE && lane == 0) {
     a.pml[row * 2] = M;
     a.pml[row * 2 + 1] = L;
   }
 }
 
+// The chunk partials of one query head, combined (one block).  Groups of DT
+// threads take every (256 / DT)th chunk, so 32 chunks are one round trip, and
+// merge in LDS.
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
-  const int row = blockIdx.x;
-  const int pos = a.ctrl[C_POS];
+  __shared__ float mo[256], mm[8], ml[8];
+  const int row = blockIdx.x, dt = a.D <= 32 ? 32 : a.D, ng = 256 / dt;
+  const int g = threadIdx.x / dt, d = threadIdx.x % dt;
+  const int pos = a.ctrl ? a.ctrl[C_POS] : a.pos;
   if (pos < 0 || pos >= a.max_tokens) return;
   const ChunkPlan cp = chunk_plan(pos, a.window, a.nsplit, a.chmin);
-  for (int d = threadIdx.x; d < a.D; d += blockDim.x)
-    a.out[(size_t)row * a.D + d] = attn_combine_elem(a.pacc, a.pml, row, d, a.D, a.nsplit, cp.nact);
+  const float* pml = a.pml + (size_t)row * a.nsplit * 2;
+  const float* ac = a.pacc + (size_t)row * a.nsplit * a.D + min(d, a.D - 1);
+  float M = -INFINITY, L = 0.f, O = 0.f;
+  for (int jb = g; g < ng && jb < cp.nact; jb += 16 * ng) {
+    float m[16], l[16], o[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int j = min(jb + u * ng, cp.nact - 1);
+      m[u] = pml[2 * j];
+      l[u] = pml[2 * j + 1];
+      o[u] = ac[(size_t)j * a.D];
+    }
+    float Mb = M;
+#pragma unroll
+    for (int u = 0; u < 16; u++) Mb = fmaxf(Mb, m[u]);
+    const float sc = M == -INFINITY ? 0.f : __expf(M - Mb);
+    L *= sc;
+    O *= sc;
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const float e = (jb + u * ng < cp.nact && m[u] != -INFINITY) ? __expf(m[u] - Mb) : 0.f;
+      L = fmaf(l[u], e, L);
+      O = fmaf(o[u], e, O);
+    }
+    M = Mb;
+  }
+  mo[threadIdx.x] = O;
+  if (d == 0 && g < ng) {
+    mm[g] = M;
+    ml[g] = L;
+  }
+  __syncthreads();
+  if (g || d >= a.D) return;
+  for (int k = 1; k < ng; k++) M = fmaxf(M, mm[k]);
+  L = O = 0.f;
+  for (int k = 0; k < ng; k++) {
+    const float e = mm[k] == -INFINITY ? 0.f : __expf(mm[k] - M);
+    L = fmaf(ml[k], e, L);
+    O = fmaf(mo[k * dt + d], e, O);
+  }
+  a.out[(size_t)row * a.D + d] = O / L;
 }
+
+int attention_one_positions(bool kv_f32, int D) { return kOneWaves * head_tiling(attn_dt(D), kv_f32 ? 4 : 2).sub; }
+
+#define ONE_CASES(X) \
+  X(float, 32, true) X(float, 64, true) X(float, 128, true) X(uint16_t, 32, false) X(uint16_t, 64, false) \
+  X(uint16_t, 128, false)
+
+bool attention_one_prepare(bool kv_f32, int D) {
+  const size_t smem = head_smem_bytes(D, kv_f32, kOneWaves);
+#define ONE_PREP(KT, DTV, F32)                                                                              \
+  if (attn_dt(D) == DTV && kv_f32 == F32)                                                                   \
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&head_kernel<KT, DTV, false, true>),           \
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess;
+  ONE_CASES(ONE_PREP)
+#undef ONE_PREP
+  return true;  // a head_dim without a kernel: the launch refuses it
+}
+
+bool launch_attention_one(bool kv_f32, const AttnArgs& a, hipStream_t st) {
+  // a wave for each pass of the window
+  const int n = a.window > 0 ? std::min(a.pos + 1, a.window) : a.pos + 1;
+  const int sub = attention_one_positions(kv_f32, a.D) / kOneWaves, nw = (n + sub - 1) / sub;
+  if (nw > kOneWaves) return false;
+  const size_t smem = head_smem_bytes(a.D, kv_f32, nw);
+#define ONE_LAUNCH(KT, DTV, F32)                                                                            \
+  if (attn_dt(a.D) == DTV && kv_f32 == F32) {                                                               \
+    hipLaunchKernelGGL((head_kernel<KT, DTV, false, true>), dim3(a.Hq), dim3(64 * nw), smem, st, a);        \
+    return true;                                                                                            \
+  }
+  ONE_CASES(ONE_LAUNCH)
+#undef ONE_LAUNCH
+  return false;
+}
+#undef ONE_CASES
 
 bool launch_attention(bool kv_f32, int gmax, const AttnArgs& a, bool combine, bool long_win, hipStream_t st) {
   if (long_win && a.gqa) {
     const bool ok = !kv_f32 && launch_gqa_attention(a, st);
-    if (ok && combine) hipLaunchKernelGGL(attn_combine_kernel, dim3(a.Hq), dim3(128), 0, st, a);
+    if (ok && combine) hipLaunchKernelGGL(attn_combine_kernel, dim3(a.Hq), dim3(256), 0, st, a);
     return ok;
   }
   // long windows: XCD-aware numbering, groups of 8 (kv head, chunk) pairs x G heads
@@ -1146,7 +1243,7 @@ bool launch_attention(bool kv_f32, int gmax, const AttnArgs& a, bool combine, bo
     HEAD_CASE(uint16_t, 32) HEAD_CASE(uint16_t, 64) HEAD_CASE(uint16_t, 128)
   }
 #undef HEAD_CASE
-  if (ok && combine) hipLaunchKernelGGL(attn_combine_kernel, dim3(a.Hq), dim3(128), 0, st, a);
+  if (ok && combine) hipLaunchKernelGGL(attn_combine_kernel, dim3(a.Hq), dim3(256), 0, st, a);
   return ok;
 }
 
