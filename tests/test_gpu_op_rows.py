@@ -1,0 +1,59 @@
+"""tlm_op_linear_rows at the edges of its tiles and split counts, against the
+float64 product of the fp16 operands the matrix cores see (weights rounded to
+fp16 once, activations fp16).  fp32 sums of K products: an error bound of
+2e-6 of the sum of magnitudes, as for any order of the same additions."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+import three_llm_amd.tlm as tlm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = tlm.Context(0)
+    yield c
+    c.close()
+
+
+def make_linear(ctx, fmt, w):
+    if fmt == tlm.FMT_Q4:
+        packed, scales = orc.q4_quantize(w)
+        return tlm.Linear(ctx, fmt, packed, scales), orc.q4_dequant(packed, scales)
+    h = w.astype(np.float16)
+    return tlm.Linear(ctx, fmt, np.ascontiguousarray(h.view(np.uint16))), h.astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt,M,N,K,bias", [
+    # four waves splitting K on 32 x 64 tiles: a wave without steps, a ring that
+    # is never full, ragged rows and columns
+    (tlm.FMT_F16, 1, 256, 32, True), (tlm.FMT_F16, 31, 65, 96, False), (tlm.FMT_F16, 33, 64, 416, True),
+    (tlm.FMT_F16, 129, 1000, 1056, True),
+    # the same in K slices that a second kernel adds; N % 4 != 0 there too
+    (tlm.FMT_F16, 33, 192, 4096, True), (tlm.FMT_F16, 33, 195, 2080, True), (tlm.FMT_Q4, 31, 130, 4096, False),
+    (tlm.FMT_Q4, 257, 300, 8192, True),
+    # 128 x 128 tiles, whole and in slices
+    (tlm.FMT_F16, 1030, 4100, 1024, True), (tlm.FMT_F16, 512, 2048, 4096, False), (tlm.FMT_F16, 700, 10000, 320, True),
+    # 256 x 256 tiles: rows and columns past the last whole one, an odd step count
+    (tlm.FMT_F16, 513, 15000, 608, True),
+])
+def test_rows_at_tile_edges(ctx, fmt, M, N, K, bias):
+    print(f"[rows] fmt {fmt}, {M} x {N} x {K}", flush=True)
+    rng = np.random.default_rng(M * 7 + N + K)
+    w = (rng.standard_normal((N, K), dtype=np.float32) * 0.02).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32).astype(np.float16)
+    b = (rng.standard_normal(N) * 0.1).astype(np.float32)
+    L, wd = make_linear(ctx, fmt, w)
+    # two calls: the second finds the slices' buffer as the first left it
+    out = ctx.array(np.full((M, N), np.nan, np.float32))
+    for _ in range(2):
+        y = L.rows(ctx.array(x.view(np.uint16)), M, out, ctx.array(b) if bias else None).read().reshape(M, N)
+    L.close()
+    xh, wh = x.astype(np.float64), wd.astype(np.float16).astype(np.float64)
+    ref, mag = xh @ wh.T, np.abs(xh) @ np.abs(wh).T
+    if bias:
+        ref, mag = ref + b, mag + np.abs(b)
+    excess = np.abs(y - ref) - (2e-6 * mag + 1e-7)
+    assert excess.max() <= 0, f"max excess {excess.max()}"

@@ -88,7 +88,10 @@ struct tlm_ctx {
   float* topk_v = nullptr;
   int* topk_i = nullptr;
   void* scratch = nullptr;  // this device's copy of `scratch` (device address)
+  float* part = nullptr;    // split-K slices of tlm_op_linear_rows (kPartFloats)
+  std::mutex part_mu;
 };
+constexpr size_t kPartFloats = (size_t)8 << 20;  // 32 MiB
 constexpr size_t kTopkWork = 32768;
 
 struct GemvPlan {
@@ -498,6 +501,7 @@ int tlm_open(int device, tlm_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->arg_idx, 4096 * sizeof(int));
   if (e == hipSuccess) e = hipMalloc(&c->topk_v, 2 * kTopkWork * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&c->topk_i, 2 * kTopkWork * sizeof(int));
+  if (e == hipSuccess) e = hipMalloc(&c->part, kPartFloats * sizeof(float));
   if (e != hipSuccess) {
     tlm_close(c);
     return fail(TLM_ERR_HIP, "TLMContext: setup failed: %s", hipGetErrorString(e));
@@ -518,6 +522,7 @@ void tlm_close(tlm_ctx* ctx) {
   hipFree(ctx->arg_idx);
   hipFree(ctx->topk_v);
   hipFree(ctx->topk_i);
+  hipFree(ctx->part);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -676,9 +681,19 @@ int tlm_op_linear_rows(tlm_linear* L, const uint16_t* x, int32_t rows, const flo
   g.ldc = L->N;
   if (L->fmt == TLM_FMT_Q4 && L->smax > 0x6FFF)
     return fail(TLM_ERR_INVALID, "TLMLinear: q4 scale above 8188 overflows the fp16 GEMM operand");
-  const GemmShape sh = gemm_shape(wfmt(L->fmt), GEMM_STORE, rows, L->N, L->K, L->ctx->cus);
-  if (!launch_gemm(wfmt(L->fmt), GEMM_STORE, sh, g, L->ctx->stream))
+  tlm_ctx* ctx = L->ctx;
+  const GemmShape sh = gemm_shape(wfmt(L->fmt), GEMM_STORE, rows, L->N, L->K, ctx->cus, kPartFloats);
+  const bool split = sh.splits > 1;
+  // the slices live in the context's buffer from the GEMM to the fold: another
+  // thread's pair of launches on the same stream goes wholly before or after
+  std::unique_lock<std::mutex> lock(ctx->part_mu, std::defer_lock);
+  if (split) {
+    lock.lock();
+    g.Cf = ctx->part;
+  }
+  if (!launch_gemm(wfmt(L->fmt), split ? GEMM_PART : GEMM_STORE, sh, g, ctx->stream))
     return fail(TLM_ERR_STATE, "TLMLinear: no batched kernel variant for %d x %d", L->N, L->K);
+  if (split) launch_fold_rows(ctx->part, sh.splits, bias, rows, L->N, y, ctx->stream);
   CHECK_LAUNCH("TLMLinear");
   return TLM_OK;
 }
@@ -1883,7 +1898,7 @@ static int prefill_plan(tlm_model* m, int M, PfPlan* pp) {
   // small chunks (the K-wave QKV GEMM), head_dim 64, full rotary: RoPE and the
   // cache append run in the QKV GEMM's epilogue (no split-K slices, no rope_kv)
   pp->sr = gemm_shape(lf, GEMM_ROPE, M, m->Nqkv, H, cus);
-  pp->rope_epi = pp->sr.ring && pp->sr.kw && D == 64 && d.rotary_dim == 64;
+  pp->rope_epi = lf == WF_Q4 && pp->sr.tile == GT_KW && D == 64 && d.rotary_dim == 64;
   pp->so = gemm_shape(lf, GEMM_PART, M, H, m->QS, cus);
   pp->sg = gemm_shape(lf, GEMM_SWIGLU, M, L0.gu->T * kTile, H, cus);
   pp->sd = gemm_shape(lf, GEMM_PART, M, H, I, cus);
@@ -1895,7 +1910,7 @@ static int prefill_plan(tlm_model* m, int M, PfPlan* pp) {
   // kernel between them drops out (127-row Qwen2.5-0.5B chunk: its 24
   // launches were 3.6 us each; the unsplit O GEMM costs 0.4 us more).
   pp->sf = gemm_shape(lf, GEMM_FOLD, M, H, m->QS, cus);
-  pp->fold = g_pf_fold && lf == WF_Q4 && pp->sf.ring && pp->sf.kw && pp->sg.ring && pp->sg.kw && H % kTile == 0 &&
+  pp->fold = g_pf_fold && lf == WF_Q4 && pp->sf.tile == GT_KW && pp->sg.tile == GT_KW && H % kTile == 0 &&
              H / kTile <= 32;
   const size_t part = std::max({(size_t)pp->sq.splits * M * m->Nqkv, (size_t)pp->so.splits * M * H,
                                 (size_t)pp->sd.splits * M * H});

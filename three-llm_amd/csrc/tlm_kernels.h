@@ -387,13 +387,16 @@ struct GemmArgs {
   int ss_ld, n_norm;
   float eps;
 };
+// Tile of a GEMM block: GT_KW one 64-column weight tile and 32 rows whose K
+// range the block's four waves share; the others rows x columns of a block
+// whose waves share its K steps.
+enum GemmTile { GT_KW = 0, GT_128x256, GT_128x128, GT_256x256 };
+inline int gemm_tile_rows(int t) { return t == GT_KW ? 32 : t == GT_256x256 ? 256 : 128; }
+inline int gemm_tile_cols(int t) { return t == GT_KW ? 64 : t == GT_128x128 ? 128 : 256; }
 // Tile and split-K choice of one GEMM (gemm_shape is the only planner, so the
 // host sizes the slice buffers from the same numbers the launch uses).
 struct GemmShape {
-  int ring;  // 1: the q4 LDS-ring kernel (wn waves over 64 wn columns, 32 mt rows)
-  int kw;    // 1 (with ring): four waves split K on one 64-column tile
-  int wn;
-  int mt, nb, gx, gy, spc, splits;
+  int tile, gx, gy, spc, splits;
 };
 // Rows of the residual stream: X[m] += sum of n_part slices part[s][m]
 // (slice stride pstride floats, rows of H), then Y[m] = fp16(rmsnorm(X[m]) w)
@@ -441,8 +444,12 @@ struct RopeKvArgs {
   int* ovf;             // set to 1 when an fp16 q, k or v is not finite; may be null
   const int* ctrl;      // non-null: the first row's position is ctrl[C_POS] instead of p0
 };
-GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus);
+// part: floats the caller has for the slices of a result it can add up itself
+// (GEMM_STORE; splits > 1 then means GEMM_PART and launch_fold_rows)
+GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part = 0);
 bool launch_gemm(int fmt, int epi, const GemmShape& sh, const GemmArgs& g, hipStream_t st);
+// y[m][n] = bias[n] + the sum of n_part slices part[s][m][n]
+void launch_fold_rows(const float* part, int n_part, const float* bias, int M, int N, float* y, hipStream_t st);
 void launch_rms_rows(const RowsArgs& a, int M, hipStream_t st);
 void launch_rope_kv(const RopeKvArgs& a, hipStream_t st);
 bool launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st);

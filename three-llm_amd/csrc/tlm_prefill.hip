@@ -45,8 +45,6 @@ __device__ __forceinline__ half8_t dequant8(uint32_t w, half2_t s2) {
   return r;
 }
 
-__device__ __forceinline__ half8_t as_half8(uint4 v) { return __builtin_bit_cast(half8_t, v); }
-
 // silu(g) * u for a result rounded to fp16: the hardware reciprocal (1 ulp)
 // instead of a full-precision division; g -> -inf gives exp = inf, rcp = 0.
 __device__ __forceinline__ float silu_mul(float g, float u) {
@@ -87,215 +85,31 @@ __device__ __forceinline__ float block_sum_f(float v, float* scratch) {
 
 }  // namespace
 
-// Global loads of one 32-k step: the thread's A pieces and the lane's weight
-// chunks (q4: one 16-byte chunk + scale; fp16: the two 8-k chunks of its half).
-template <int FMT, int MT, int NB>
-struct GemmPtrs {
-  const uint16_t* asrc[MT];
-  const uint4* wp[NB];
-  const uint16_t* sp[NB];
-};
-// Registers of one step in flight; members are named, not arrays, so that the
-// compiler keeps every stage of the ring in registers.
-template <int FMT, int MT, int NB>
-struct GemmStage {
-  static_assert(MT <= 2 && NB <= 2, "stage registers are spelled out for MT, NB <= 2");
-  uint4 a0, a1;      // A pieces (a1 when MT == 2)
-  uint4 w0, w1;      // column group 0: q4 chunk, or the two fp16 chunks
-  uint4 v0, v1;      // column group 1 (NB == 2)
-  uint16_t s0, s1;   // q4 scales of the groups
-  __device__ __forceinline__ void load(const GemmPtrs<FMT, MT, NB>& p, int c, int kh) {
-    a0 = *reinterpret_cast<const uint4*>(p.asrc[0] + c * 32);
-    if constexpr (MT > 1) a1 = *reinterpret_cast<const uint4*>(p.asrc[1] + c * 32);
-    if constexpr (FMT == WF_Q4) {
-      w0 = p.wp[0][(size_t)c * kTile];
-      s0 = p.sp[0][(size_t)c * kTile];
-      if constexpr (NB > 1) {
-        v0 = p.wp[1][(size_t)c * kTile];
-        s1 = p.sp[1][(size_t)c * kTile];
-      }
-    } else {
-      w0 = p.wp[0][(size_t)(4 * c + kh) * kTile];
-      w1 = p.wp[0][(size_t)(4 * c + 2 + kh) * kTile];
-      if constexpr (NB > 1) {
-        v0 = p.wp[1][(size_t)(4 * c + kh) * kTile];
-        v1 = p.wp[1][(size_t)(4 * c + 2 + kh) * kTile];
-      }
-    }
-  }
-  // B operands of column group j for the two 16-k halves of the step
-  __device__ __forceinline__ void operands(int j, int kh, half8_t& b1, half8_t& b2) const {
-    const uint4& x = j ? v0 : w0;
-    if constexpr (FMT == WF_Q4) {
-      const _Float16 s = __builtin_bit_cast(_Float16, j ? s1 : s0);
-      const half2_t s2 = {s, s};
-      b1 = dequant8(kh ? x.y : x.x, s2);
-      b2 = dequant8(kh ? x.w : x.z, s2);
-    } else {
-      b1 = as_half8(x);
-      b2 = as_half8(j ? v1 : w1);
-    }
-  }
-};
-
-// ----------------------------------------------------------------- GEMM --
-// C = A W^T.  Block: 4 waves as 2 (rows) x 2 (columns); a wave owns 32 MT rows
-// x 32 NB columns as MT x NB MFMA tiles of 32 x 32.  Per 32-k step the block's
-// A rows [64 MT][32] go through LDS (double buffered, one barrier per step)
-// and each lane forms its column's B operand in registers: q4 codes
-// dequantised once per step, fp16 rows loaded as they are.  Global loads run
-// kPf steps ahead of the MFMAs through a ring of register stages (the loop is
-// unrolled by kPf so every stage is a fixed set of registers).
-// Split-K: blockIdx.z takes steps [z spc, (z + 1) spc); GEMM_PART writes each
-// split's sum to its own slice Cf + z M ldc, the consumer adds the slices.
+// ---------------------------------------------------------- GEMM, LDS ring --
+// C = A W^T with the operands streamed by direct global -> LDS loads
+// (global_load_lds: no registers held while the loads are in flight).
 // MFMA 32x32x16 f16 lane layouts: A: lane l holds A[l % 32][8 (l / 32) + 0..7];
 // B: B[8 (l / 32) + 0..7][l % 32]; D: register v of lane l holds
 // D[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].
-// Columns are physical weight rows: with NB = 2 a wave's two groups are the
-// two halves of one 64-row tile, which for the paired gate|up layout are the
-// gate rows 32t.. and the matching up rows, so GEMM_SWIGLU finishes in-lane.
-constexpr int kPf = 4;  // steps in flight (the four stages of gemm_kernel)
-
-template <int FMT, int MT, int NB>
-struct GemmMain {
-  static constexpr int LS = 40;  // LDS halves per A row (32 + 8: conflict-free 16-byte reads)
-  float16_t acc[MT][NB];
-
-  // one step: stage -> LDS buffer and B registers, refill the stage, barrier, MFMAs
-  // returns the stage refilled with step `next` (values, not references: the
-  // ring then stays in registers)
-  __device__ __forceinline__ GemmStage<FMT, MT, NB> step(GemmStage<FMT, MT, NB> st,
-                                                         const GemmPtrs<FMT, MT, NB>& p, _Float16* buf,
-                                                         const int* adst, int next, bool refill, int arow,
-                                                         int kh) {
-    *reinterpret_cast<uint4*>(buf + adst[0]) = st.a0;
-    if constexpr (MT > 1) *reinterpret_cast<uint4*>(buf + adst[1]) = st.a1;
-    half8_t b[NB][2];
-#pragma unroll
-    for (int j = 0; j < NB; j++) st.operands(j, kh, b[j][0], b[j][1]);
-    // the stage's registers are free once the operands are formed: keep the
-    // refill after them so the loads land in the same registers (otherwise the
-    // loop needs copies that wait for the loads)
-    __builtin_amdgcn_sched_barrier(0);
-    if (refill) st.load(p, next, kh);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-      const _Float16* ar = buf + (arow + 32 * i) * LS + 8 * kh;
-      const half8_t a1 = *reinterpret_cast<const half8_t*>(ar);
-      const half8_t a2 = *reinterpret_cast<const half8_t*>(ar + 16);
-#pragma unroll
-      for (int j = 0; j < NB; j++) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b[j][0], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b[j][1], acc[i][j], 0, 0, 0);
-      }
-    }
-    return st;
-  }
-};
-
-template <int FMT, int MT, int NB, int EPI>
-__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-  using Main = GemmMain<FMT, MT, NB>;
-  constexpr int BM = 64 * MT, LS = Main::LS;
-  __shared__ __align__(16) _Float16 as[2][BM * LS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l32 = lane & 31, kh = lane >> 5;
-  const int m0 = blockIdx.y * BM;
-  const int cg0 = (blockIdx.x * 2 + wn) * 32 * NB;
-  const int c0 = blockIdx.z * g.spc, n = min(g.spc, g.K / 32 - c0);
-
-  GemmPtrs<FMT, MT, NB> p;
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    const int r = min(cg0 + 32 * j + l32, g.N - 1);  // clamped: loads stay unconditional
-    const size_t base = (size_t)(r / kTile) * g.C * kTile + r % kTile;
-    p.wp[j] = g.w + base;
-    p.sp[j] = FMT == WF_Q4 ? g.s + base : g.s;
-  }
-  int adst[MT];
-#pragma unroll
-  for (int u = 0; u < MT; u++) {
-    const int q = tid + 256 * u, r = q >> 2, piece = q & 3;
-    p.asrc[u] = g.A + (size_t)min(m0 + r, g.M - 1) * g.lda + piece * 8;
-    adst[u] = r * LS + piece * 8;
-  }
-
-  Main mm;
-#pragma unroll
-  for (int i = 0; i < MT; i++)
-#pragma unroll
-    for (int j = 0; j < NB; j++) mm.acc[i][j] = (float16_t){};
-
-  // four named stages (not an array: the ring must stay in registers)
-  GemmStage<FMT, MT, NB> s0, s1, s2, s3;
-  s0.load(p, c0, kh);
-  s1.load(p, c0 + min(1, n - 1), kh);
-  s2.load(p, c0 + min(2, n - 1), kh);
-  s3.load(p, c0 + min(3, n - 1), kh);
-  const int arow = wm * 32 * MT + l32;
-  const int nfull = n - n % kPf;
-  for (int cb = 0; cb < nfull; cb += kPf) {
-    s0 = mm.step(s0, p, as[0], adst, c0 + min(cb + 4, n - 1), true, arow, kh);
-    s1 = mm.step(s1, p, as[1], adst, c0 + min(cb + 5, n - 1), true, arow, kh);
-    s2 = mm.step(s2, p, as[0], adst, c0 + min(cb + 6, n - 1), true, arow, kh);
-    s3 = mm.step(s3, p, as[1], adst, c0 + min(cb + 7, n - 1), true, arow, kh);
-  }
-  // tail: stage u holds step nfull + u
-  if (nfull < n) mm.step(s0, p, as[0], adst, 0, false, arow, kh);
-  if (nfull + 1 < n) mm.step(s1, p, as[1], adst, 0, false, arow, kh);
-  if (nfull + 2 < n) mm.step(s2, p, as[0], adst, 0, false, arow, kh);
-
-  const int rbase = m0 + wm * 32 * MT + 4 * kh;
-  if (EPI == GEMM_SWIGLU) {
-    const int oi = (cg0 / kTile) * 32 + l32;  // canonical gate index of this lane's column
-    if (oi >= g.n_out) return;
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int row = rbase + 32 * i + 8 * (v >> 2) + (v & 3);
-        if (row < g.M) {
-          const float gt = mm.acc[i][0][v], up = mm.acc[i][NB - 1][v];
-          const _Float16 hv = f16_guard(g.ovf, silu_mul(gt, up));
-          g.Ch[(size_t)row * g.ldc + oi] = __builtin_bit_cast(uint16_t, hv);
-        }
-      }
-    return;
-  }
-  float* out = g.Cf + (EPI == GEMM_PART ? (size_t)blockIdx.z * g.M * g.ldc : 0);
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    const int col = cg0 + 32 * j + l32;
-    if (col >= g.N) continue;
-    const float bias = (EPI == GEMM_STORE && g.bias) ? g.bias[col] : 0.f;
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int row = rbase + 32 * i + 8 * (v >> 2) + (v & 3);
-        if (row < g.M) out[(size_t)row * g.ldc + col] = mm.acc[i][j][v] + bias;
-      }
-  }
-}
-
-// ------------------------------------------------------- q4 GEMM, LDS ring --
-// The q4 GEMM with its operands streamed by direct global -> LDS loads
-// (global_load_lds: no registers held while the loads are in flight).
-// Block: 4 waves side by side over 256 columns (four 64-row weight tiles); a
-// wave owns all 32 MT rows x its 64 columns (MT x 2 MFMA tiles of 32 x 32).
-// Per 32-k step a stage of the LDS ring holds the block's A rows [32 MT][32]
-// (16-byte pieces at a swizzled slot, see a_slot), the 256 weight chunks and
-// their scales.  kRing stages: a step's loads are issued kRing - 1 steps
-// before its MFMAs; every wave issues the same number of loads per stage
-// (small blocks repeat a copy of identical bytes), so one immediate vmcnt
-// bounds the loads still in flight.  Columns: for the paired gate|up layout
-// a wave's two 32-column groups are the gate rows and the matching up rows.
-// The depth is even: the operands of consecutive steps alternate between two
-// register sets (a 6-stage ring measured slower).
-constexpr int kRing = 4;
-static_assert(kRing % 2 == 0, "even ring depth");
+// Columns are physical weight rows: a wave's two 32-column groups are the two
+// halves of one 64-row tile, which for the paired gate|up layout are the gate
+// rows 32t.. and the matching up rows, so GEMM_SWIGLU finishes in-lane.
+// Split-K: blockIdx.z takes steps [z spc, (z + 1) spc); GEMM_PART writes each
+// split's sum to its own slice Cf + z M ldc, the consumer adds the slices.
+// Block: WM x WN waves over 32 MT WM rows and 64 WN columns (64-row weight
+// tiles); a wave owns 32 MT rows x 64 columns (MT x 2 MFMA tiles of 32 x 32).
+// Per 32-k step a stage of the LDS ring holds the block's A rows (16-byte
+// pieces at a swizzled slot, see a_slot) and the weights: q4 chunks and their
+// scales, which each wave dequantises in registers, or fp16 chunks
+// [4][64 rows], which are MFMA operands as they lie.  NS stages: a step's
+// loads are issued NS - 1 steps before its MFMAs; every wave issues the same
+// number of loads per stage (small blocks repeat a copy of identical bytes),
+// so one immediate vmcnt bounds the loads still in flight.  NS is even: the
+// operands of consecutive steps alternate between two register sets.
+// fp16 is bound by the L2's reads where the chip is full: 2048 x 16384 x 2048
+// takes 174 us in 128 x 128 tiles (3.0 GB from the L2), 147 us in 256 x 256
+// (1.9 GB).  A smaller result needs more blocks: 512 x 2048 x 8192 took 96 us
+// as 64 blocks over all of K, 30 us as 128 x 128 tiles in 4 K slices.
 
 // s_waitcnt immediate that waits until at most n vector-memory operations are
 // outstanding (n < 64) and leaves the other counters alone: vmcnt bits 3:0 in
@@ -323,15 +137,20 @@ __device__ __forceinline__ void lds_dma4(const void* base, uint32_t off, uint32_
                : "memory", "m0");
 }
 
-template <int MT, int WN>
+template <int FMT, int MT, int WM, int WN, int NS>
 struct RingLayout {
-  static constexpr int BM = 32 * MT;
-  static constexpr int NA = 2 * MT;             // 1 KiB A copies per stage
-  static constexpr int AW = (NA + WN - 1) / WN; // A copies per wave
-  static constexpr int S_BYTES = WN * 128 > 256 ? WN * 128 : 256;
-  static constexpr int W_OFF = BM * 64, S_OFF = W_OFF + WN * 1024, STAGE = S_OFF + S_BYTES;
-  static constexpr int LPS = AW + 2;            // copies per wave per stage: A, one weight tile, scales
-  static constexpr int NR = kRing;
+  static constexpr int WAVES = WM * WN;
+  static constexpr int BM = 32 * MT * WM;
+  static constexpr int NA = 2 * MT * WM;                // 1 KiB A copies per stage
+  static constexpr int AW = (NA + WAVES - 1) / WAVES;   // A copies per wave
+  static constexpr int NW = FMT == WF_Q4 ? 1 : 4;       // 1 KiB copies of one weight tile per stage
+  static constexpr int CW = NW >= WM ? NW / WM : 1;     // weight copies per wave
+  static constexpr int S_BYTES = FMT != WF_Q4 ? 0 : WN * 128;
+  static constexpr int W_OFF = BM * 64, S_OFF = W_OFF + WN * NW * 1024, STAGE = S_OFF + S_BYTES;
+  static constexpr int LPS = AW + CW + (FMT == WF_Q4);  // copies per wave per stage
+  static constexpr int NR = NS;
+  static_assert(NR % 2 == 0, "even ring depth");
+  static_assert(FMT != WF_Q4 || WN % 2 == 0, "one scale copy covers two tiles");
   static_assert((NR - 1) * LPS <= 63, "copies in flight within vmcnt's range");
 };
 
@@ -341,13 +160,12 @@ struct RingLayout {
 // takes k = 16 kh + 0..7, MFMA 2 k = 16 kh + 8..15 (kh = lane / 32), so a
 // lane's A pieces are 2 kh, 2 kh + 1 and its weight dwords 2 kh, 2 kh + 1
 // (one 8-byte read).
-template <int MT, int WN>
+template <int FMT, int MT, int WM, int WN, int NS>
 struct RingBlock {
-  using RL = RingLayout<MT, WN>;
-  const char* abase;  // A + 32 c halves, weight and scale bases advance per step
-  const char* wbase;
+  using RL = RingLayout<FMT, MT, WM, WN, NS>;
+  const char* abase;  // the block's first row at its first step; 32 c halves further per step
+  const char* wbase;  // likewise this wave's weight tile and scales
   const char* sbase;
-  int a_lds_stride;   // bytes per 32-k step in each operand
   uint32_t agoff[RL::AW], alds[RL::AW];  // global byte offsets / LDS offsets of this wave's A copies
   uint32_t wgoff, sgoff, wlds, slds;
   uint32_t lbase;
@@ -358,12 +176,14 @@ struct RingBlock {
   __device__ __forceinline__ void issue(int stage, int c) {
     const uint32_t sb = lbase + stage * RL::STAGE;
     const char* ab = abase + (size_t)c * 64;
-    const char* wb = wbase + (size_t)c * kTile * 16;
-    const char* sbs = sbase + (size_t)c * kTile * 2;
+    const char* wb = wbase + (size_t)c * RL::NW * kTile * 16;
 #pragma unroll
     for (int u = 0; u < RL::AW; u++) lds_dma16(ab, agoff[u], __builtin_amdgcn_readfirstlane(sb + alds[u]));
-    lds_dma16(wb, wgoff, __builtin_amdgcn_readfirstlane(sb + wlds));
-    lds_dma4(sbs, sgoff, __builtin_amdgcn_readfirstlane(sb + slds));
+#pragma unroll
+    for (int u = 0; u < RL::CW; u++)
+      lds_dma16(wb + u * 1024, wgoff, __builtin_amdgcn_readfirstlane(sb + wlds + u * 1024));
+    if constexpr (FMT == WF_Q4)
+      lds_dma4(sbase + (size_t)c * kTile * 2, sgoff, __builtin_amdgcn_readfirstlane(sb + slds));
   }
 
   // One step's MFMA operands: the A pieces as read from LDS and the weights
@@ -380,6 +200,16 @@ struct RingBlock {
     for (int j = 0; j < 2; j++) {
       w[j] = *reinterpret_cast<const uint2*>(sb + rd_w[j]);
       sc[j] = *reinterpret_cast<const _Float16*>(sb + rd_s[j]);
+    }
+  }
+  // fp16: chunk 2 kh is the B operand of MFMA 1, chunk 2 kh + 1 of MFMA 2
+  template <int S>
+  __device__ __forceinline__ void read_b(const unsigned char* lds, Ops& o) const {
+    const unsigned char* sb = lds + S * RL::STAGE;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      o.b[j][0] = *reinterpret_cast<const half8_t*>(sb + rd_w[j]);
+      o.b[j][1] = *reinterpret_cast<const half8_t*>(sb + rd_w[j] + 1024);
     }
   }
   template <int S>
@@ -403,9 +233,10 @@ struct RingBlock {
   __device__ __forceinline__ void read(const unsigned char* lds, Ops& o) const {
     uint2 w[2];
     _Float16 sc[2];
-    read_w<S>(lds, w, sc);
+    if constexpr (FMT == WF_Q4) read_w<S>(lds, w, sc);
+    else read_b<S>(lds, o);
     read_a<S>(lds, o);
-    dequant(w, sc, o);
+    if constexpr (FMT == WF_Q4) dequant(w, sc, o);
   }
 
   // Step i in stage S; `cur` holds its operands, read and dequantised during
@@ -426,7 +257,8 @@ struct RingBlock {
     __builtin_amdgcn_sched_barrier(0);  // keep each step's MFMAs after its own barrier
     uint2 w[2];
     _Float16 sc[2];
-    read_w<(S + 1) % NR>(lds, w, sc);
+    if constexpr (FMT == WF_Q4) read_w<(S + 1) % NR>(lds, w, sc);
+    else read_b<(S + 1) % NR>(lds, nxt);
     read_a<(S + 1) % NR>(lds, nxt);
     issue((S + NR - 1) % NR, refill_c);
     __builtin_amdgcn_sched_barrier(0);  // the reads and copies go out before the MFMAs
@@ -437,13 +269,15 @@ struct RingBlock {
         acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.a1[t], cur.b[j][0], acc[t][j], 0, 0, 0);
         acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.a2[t], cur.b[j][1], acc[t][j], 0, 0, 0);
       }
-    dequant(w, sc, nxt);
-    // order: a few MFMAs while the weight reads land, then one MFMA per
-    // slice of the dequantisation
-    __builtin_amdgcn_sched_group_barrier(0x008, MT, 0);
+    if constexpr (FMT == WF_Q4) {
+      dequant(w, sc, nxt);
+      // order: a few MFMAs while the weight reads land, then one MFMA per
+      // slice of the dequantisation
+      __builtin_amdgcn_sched_group_barrier(0x008, MT, 0);
 #define RING_MV __builtin_amdgcn_sched_group_barrier(0x002, 8, 0); __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV
+      RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV RING_MV
 #undef RING_MV
+    }
   }
 };
 
@@ -452,67 +286,73 @@ struct RingBlock {
 // left after the last full pass (their stages already hold them).  Even steps
 // take their operands from o0 and read the next step's into o1, odd steps
 // the other way round.
-template <int MT, int WN, int S, int E>
+template <class RB, int S, int E>
 struct RingSteps {
-  using RB = RingBlock<MT, WN>;
   using Ops = typename RB::Ops;
   static __device__ __forceinline__ void full(RB& rb, const unsigned char* lds, int i, int n, Ops& o0, Ops& o1) {
-    const int c = min(i + S + RingLayout<MT, WN>::NR - 1, n - 1);
-    if constexpr (S % 2 == 0) rb.template step<S>(lds, c, o0, o1);
-    else rb.template step<S>(lds, c, o1, o0);
-    RingSteps<MT, WN, S + 1, E>::full(rb, lds, i, n, o0, o1);
+    if constexpr (S < E) {
+      const int c = min(i + S + RB::RL::NR - 1, n - 1);
+      if constexpr (S % 2 == 0) rb.template step<S>(lds, c, o0, o1);
+      else rb.template step<S>(lds, c, o1, o0);
+      RingSteps<RB, S + 1, E>::full(rb, lds, i, n, o0, o1);
+    }
   }
   static __device__ __forceinline__ void tail(RB& rb, const unsigned char* lds, int i, int n, Ops& o0, Ops& o1) {
-    if (i + S < n) {
-      if constexpr (S % 2 == 0) rb.template step<S>(lds, n - 1, o0, o1);
-      else rb.template step<S>(lds, n - 1, o1, o0);
+    if constexpr (S < E) {
+      if (i + S < n) {
+        if constexpr (S % 2 == 0) rb.template step<S>(lds, n - 1, o0, o1);
+        else rb.template step<S>(lds, n - 1, o1, o0);
+      }
+      RingSteps<RB, S + 1, E>::tail(rb, lds, i, n, o0, o1);
     }
-    RingSteps<MT, WN, S + 1, E>::tail(rb, lds, i, n, o0, o1);
   }
 };
-template <int MT, int WN, int E>
-struct RingSteps<MT, WN, E, E> {
-  using Ops = typename RingBlock<MT, WN>::Ops;
-  static __device__ __forceinline__ void full(RingBlock<MT, WN>&, const unsigned char*, int, int, Ops&, Ops&) {}
-  static __device__ __forceinline__ void tail(RingBlock<MT, WN>&, const unsigned char*, int, int, Ops&, Ops&) {}
-};
 
-template <int MT, int WN, int EPI>
-__global__ __launch_bounds__(64 * WN) __attribute__((amdgpu_waves_per_eu(2))) void gemm_q4_ring_kernel(GemmArgs g) {
-  using RL = RingLayout<MT, WN>;
+template <int FMT, int MT, int WM, int WN, int NS, int EPI>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ring_kernel(GemmArgs g) {
+  using RB = RingBlock<FMT, MT, WM, WN, NS>;
+  using RL = typename RB::RL;
   constexpr int NR = RL::NR;
   __shared__ __align__(16) unsigned char lds[NR * RL::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wm = wave / WN;
   const int l32 = lane & 31, kh = lane >> 5;
   const int m0 = blockIdx.y * RL::BM, t0 = blockIdx.x * WN, T = (g.N + kTile - 1) / kTile;
   const int c0 = blockIdx.z * g.spc, n = min(g.spc, g.K / 32 - c0);
 
-  RingBlock<MT, WN> rb;
+  RB rb;
   rb.lbase = (uint32_t)(uintptr_t)lds;
-  rb.abase = reinterpret_cast<const char*>(g.A) + (size_t)c0 * 64;
-  rb.wbase = reinterpret_cast<const char*>(g.w) + (size_t)c0 * kTile * 16;
-  rb.sbase = reinterpret_cast<const char*>(g.s) + (size_t)c0 * kTile * 2;
+  rb.abase = reinterpret_cast<const char*>(g.A) + ((size_t)m0 * g.lda + (size_t)c0 * 32) * 2;
+  // this wave's copies of its weight tile: CW of the NW (each wave row of the block its own)
+  const int wc = RL::NW > 1 ? wm * RL::CW : 0;
+  rb.wbase = reinterpret_cast<const char*>(g.w) +
+             ((size_t)min(t0 + wn, T - 1) * g.C + (size_t)c0 * RL::NW) * kTile * 16 + wc * 1024;
+  rb.wgoff = (uint32_t)lane * 16;
+  rb.wlds = RL::W_OFF + (wn * RL::NW + wc) * 1024;
 #pragma unroll
   for (int u = 0; u < RL::AW; u++) {
     const int ai = (wave * RL::AW + u) % RL::NA, sl = ai * 64 + lane, r = sl >> 2;
-    rb.agoff[u] = (uint32_t)(((size_t)min(m0 + r, g.M - 1) * g.lda + 8 * ((sl & 3) ^ a_swz(r))) * 2);
+    rb.agoff[u] = (uint32_t)(((size_t)min(r, g.M - 1 - m0) * g.lda + 8 * ((sl & 3) ^ a_swz(r))) * 2);
     rb.alds[u] = ai * 1024;
   }
-  rb.wgoff = (uint32_t)(((size_t)min(t0 + wave, T - 1) * g.C * kTile + lane) * 16);
-  const int sidx = WN >= 4 ? wave % (WN / 2) : 0;  // one scale copy covers two tiles
-  rb.sgoff = (uint32_t)(((size_t)min(t0 + 2 * sidx + (lane >> 5), T - 1) * g.C * kTile + 2 * (lane & 31)) * 2);
-  rb.wlds = RL::W_OFF + wave * 1024;
-  rb.slds = RL::S_OFF + sidx * 256;
+  if constexpr (FMT == WF_Q4) {
+    const int sidx = wave % (WN / 2);  // one scale copy covers two tiles
+    const int st = min(t0 + 2 * sidx + (lane >> 5), T - 1) - t0;
+    rb.sbase = reinterpret_cast<const char*>(g.s) + ((size_t)t0 * g.C + c0) * kTile * 2;
+    rb.sgoff = (uint32_t)(((size_t)st * g.C * kTile + 2 * (lane & 31)) * 2);
+    rb.slds = RL::S_OFF + sidx * 256;
+  }
 #pragma unroll
   for (int t = 0; t < MT; t++) {
-    const int r = 32 * t + l32;
+    const int r = 32 * (wm * MT + t) + l32;
     rb.rd_a1[t] = a_slot(r, 2 * kh) * 16;
     rb.rd_a2[t] = a_slot(r, 2 * kh + 1) * 16;
   }
 #pragma unroll
   for (int j = 0; j < 2; j++) {
-    const int cc = wave * 64 + 32 * j + l32;
-    rb.rd_w[j] = RL::W_OFF + cc * 16 + 8 * kh;
+    const int cc = wn * 64 + 32 * j + l32;
+    rb.rd_w[j] = FMT == WF_Q4 ? RL::W_OFF + cc * 16 + 8 * kh
+                              : RL::W_OFF + wn * 4096 + 2 * kh * 1024 + (32 * j + l32) * 16;
     rb.rd_s[j] = RL::S_OFF + cc * 2;
   }
 #pragma unroll
@@ -521,19 +361,19 @@ __global__ __launch_bounds__(64 * WN) __attribute__((amdgpu_waves_per_eu(2))) vo
   // steps are relative to c0 from here on
 #pragma unroll
   for (int st = 0; st < NR - 1; st++) rb.issue(st, min(st, n - 1));
-  typename RingBlock<MT, WN>::Ops o0, o1;
+  typename RB::Ops o0, o1;
   __builtin_amdgcn_s_waitcnt(waitcnt_vm((NR - 2) * RL::LPS));  // step 0 has landed (this wave's copies)
   asm volatile("s_barrier" ::: "memory");                        // ... and every wave's
   rb.template read<0>(lds, o0);
   int i = 0;
-  for (; i + NR <= n; i += NR) RingSteps<MT, WN, 0, NR>::full(rb, lds, i, n, o0, o1);
-  RingSteps<MT, WN, 0, NR - 1>::tail(rb, lds, i, n, o0, o1);
+  for (; i + NR <= n; i += NR) RingSteps<RB, 0, NR>::full(rb, lds, i, n, o0, o1);
+  RingSteps<RB, 0, NR - 1>::tail(rb, lds, i, n, o0, o1);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the clamped trailing copies land before the block exits
 
-  const int cg0 = (t0 + wave) * kTile;
-  const int rbase = m0 + 4 * kh;
+  const int cg0 = (t0 + wn) * kTile;
+  const int rbase = m0 + 32 * MT * wm + 4 * kh;
   if (EPI == GEMM_SWIGLU) {
-    const int oi = (t0 + wave) * 32 + l32;
+    const int oi = (t0 + wn) * 32 + l32;
     if (oi >= g.n_out) return;
 #pragma unroll
     for (int t = 0; t < MT; t++)
@@ -564,7 +404,7 @@ __global__ __launch_bounds__(64 * WN) __attribute__((amdgpu_waves_per_eu(2))) vo
   }
 }
 
-// ------------------------------------------------ q4 GEMM, waves split K --
+// --------------------------------------------------- GEMM, waves split K --
 // For grids too small to fill the CUs (short prompts): a block's 4 waves take
 // the same 64 columns and 32 MT rows and split the block's K range in four.
 // Each wave streams its own operands through a private LDS ring (global ->
@@ -575,21 +415,22 @@ __device__ __forceinline__ float f4_at(const float4& v, int e) {
   return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w;
 }
 
-template <int MT>
+template <int FMT, int MT>
 struct KwLayout {
-  static constexpr int NR = 4;                           // ring stages per wave
+  static constexpr int NR = FMT == WF_Q4 ? 4 : 3;        // ring stages per wave (fp16: two blocks' rings fit a CU)
   static constexpr int NA = 2 * MT;                      // 1 KiB A copies per stage
-  static constexpr int W_OFF = MT * 2048, S_OFF = W_OFF + 1024, STAGE = S_OFF + 256;
+  static constexpr int NW = FMT == WF_Q4 ? 1 : 4;        // 1 KiB weight copies per stage
+  static constexpr int W_OFF = MT * 2048, S_OFF = W_OFF + NW * 1024, STAGE = S_OFF + (FMT == WF_Q4 ? 256 : 0);
   static constexpr int WAVE_BYTES = NR * STAGE;          // one wave's ring
-  static constexpr int LPS = NA + 2;                     // copies per stage
+  static constexpr int LPS = NA + NW + (FMT == WF_Q4);   // copies per stage
   static constexpr int ACC_FLOATS = MT * 2 * 16 * 64;    // one wave's accumulators
   static_assert(4 * ACC_FLOATS * 4 <= 4 * WAVE_BYTES, "accumulator handoff fits in the rings");
   static_assert((NR - 1) * LPS <= 63, "copies in flight within vmcnt's range");
 };
 
-template <int MT>
+template <int FMT, int MT>
 struct KwWave {
-  using KL = KwLayout<MT>;
+  using KL = KwLayout<FMT, MT>;
   const char* abase;
   const char* wbase;
   const char* sbase;
@@ -601,10 +442,14 @@ struct KwWave {
   __device__ __forceinline__ void issue(int stage, int c) {
     const uint32_t sb = lbase + stage * KL::STAGE;
     const char* ab = abase + (size_t)c * 64;
+    const char* wb = wbase + (size_t)c * KL::NW * kTile * 16;
 #pragma unroll
     for (int u = 0; u < KL::NA; u++) lds_dma16(ab, agoff[u], __builtin_amdgcn_readfirstlane(sb + u * 1024));
-    lds_dma16(wbase + (size_t)c * kTile * 16, wgoff, __builtin_amdgcn_readfirstlane(sb + KL::W_OFF));
-    lds_dma4(sbase + (size_t)c * kTile * 2, sgoff, __builtin_amdgcn_readfirstlane(sb + KL::S_OFF));
+#pragma unroll
+    for (int u = 0; u < KL::NW; u++)
+      lds_dma16(wb + u * 1024, wgoff, __builtin_amdgcn_readfirstlane(sb + KL::W_OFF + u * 1024));
+    if constexpr (FMT == WF_Q4)
+      lds_dma4(sbase + (size_t)c * kTile * 2, sgoff, __builtin_amdgcn_readfirstlane(sb + KL::S_OFF));
   }
 
   template <int S>
@@ -621,11 +466,16 @@ struct KwWave {
     half8_t b[2][2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const uint2 wv = *reinterpret_cast<const uint2*>(sb + rd_w[j]);
-      const _Float16 sc = *reinterpret_cast<const _Float16*>(sb + rd_s[j]);
-      const half2_t s2 = {sc, sc};
-      b[j][0] = dequant8(wv.x, s2);
-      b[j][1] = dequant8(wv.y, s2);
+      if constexpr (FMT == WF_Q4) {
+        const uint2 wv = *reinterpret_cast<const uint2*>(sb + rd_w[j]);
+        const _Float16 sc = *reinterpret_cast<const _Float16*>(sb + rd_s[j]);
+        const half2_t s2 = {sc, sc};
+        b[j][0] = dequant8(wv.x, s2);
+        b[j][1] = dequant8(wv.y, s2);
+      } else {
+        b[j][0] = *reinterpret_cast<const half8_t*>(sb + rd_w[j]);
+        b[j][1] = *reinterpret_cast<const half8_t*>(sb + rd_w[j] + 1024);
+      }
     }
 #pragma unroll
     for (int t = 0; t < MT; t++) {
@@ -640,29 +490,51 @@ struct KwWave {
   }
 };
 
-template <int MT, int EPI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_q4_kw_kernel(GemmArgs g) {
-  using KL = KwLayout<MT>;
+// Steps S.. of the wave's ring: full() refills each stage NR - 1 steps ahead,
+// tail() runs what is left after the last full pass.
+template <class KW, int S>
+struct KwSteps {
+  static constexpr int NR = KW::KL::NR;
+  static __device__ __forceinline__ void full(KW& kw, const unsigned char* mine, int i, int n) {
+    if constexpr (S < NR) {
+      kw.template step<S>(mine, min(i + S + NR - 1, n - 1));
+      KwSteps<KW, S + 1>::full(kw, mine, i, n);
+    }
+  }
+  static __device__ __forceinline__ void tail(KW& kw, const unsigned char* mine, int i, int n) {
+    if constexpr (S < NR - 1) {
+      if (i + S < n) kw.template step<S>(mine, n - 1);
+      KwSteps<KW, S + 1>::tail(kw, mine, i, n);
+    }
+  }
+};
+
+template <int FMT, int MT, int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_kw_kernel(GemmArgs g) {
+  using KL = KwLayout<FMT, MT>;
   __shared__ __align__(16) unsigned char lds[4 * KL::WAVE_BYTES];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, kh = lane >> 5;
-  const int m0 = blockIdx.y * 32 * MT, t0 = blockIdx.x, T = (g.N + kTile - 1) / kTile;
+  const int m0 = blockIdx.y * 32 * MT, t0 = blockIdx.x;
   const int cb = blockIdx.z * g.spc, nb = min(g.spc, g.K / 32 - cb);
   const int q = (nb + 3) / 4, c0 = cb + wave * q, n = max(0, min(q, nb - wave * q));
   const unsigned char* mine = lds + wave * KL::WAVE_BYTES;
 
-  KwWave<MT> kw;
+  KwWave<FMT, MT> kw;
   kw.lbase = (uint32_t)(uintptr_t)mine;
-  kw.abase = reinterpret_cast<const char*>(g.A) + (size_t)c0 * 64;
-  kw.wbase = reinterpret_cast<const char*>(g.w) + (size_t)c0 * kTile * 16;
-  kw.sbase = reinterpret_cast<const char*>(g.s) + (size_t)c0 * kTile * 2;
+  kw.abase = reinterpret_cast<const char*>(g.A) + ((size_t)m0 * g.lda + (size_t)c0 * 32) * 2;
+  kw.wbase = reinterpret_cast<const char*>(g.w) + ((size_t)t0 * g.C + (size_t)c0 * KL::NW) * kTile * 16;
+  kw.wgoff = (uint32_t)lane * 16;
 #pragma unroll
   for (int u = 0; u < KL::NA; u++) {
     const int sl = u * 64 + lane, r = sl >> 2;
-    kw.agoff[u] = (uint32_t)(((size_t)min(m0 + r, g.M - 1) * g.lda + 8 * ((sl & 3) ^ a_swz(r))) * 2);
+    kw.agoff[u] = (uint32_t)(((size_t)min(r, g.M - 1 - m0) * g.lda + 8 * ((sl & 3) ^ a_swz(r))) * 2);
   }
-  kw.wgoff = (uint32_t)(((size_t)min(t0, T - 1) * g.C * kTile + lane) * 16);
-  kw.sgoff = (uint32_t)(((size_t)min(t0 + (lane >> 5), T - 1) * g.C * kTile + 2 * (lane & 31)) * 2);
+  if constexpr (FMT == WF_Q4) {  // the copy is two tiles wide: the last tile is copied twice
+    const int T = (g.N + kTile - 1) / kTile;
+    kw.sbase = reinterpret_cast<const char*>(g.s) + ((size_t)t0 * g.C + c0) * kTile * 2;
+    kw.sgoff = (uint32_t)(((size_t)(min(t0 + (lane >> 5), T - 1) - t0) * g.C * kTile + 2 * (lane & 31)) * 2);
+  }
 #pragma unroll
   for (int t = 0; t < MT; t++) {
     kw.rd_a1[t] = a_slot(32 * t + l32, 2 * kh) * 16;
@@ -670,7 +542,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   }
 #pragma unroll
   for (int j = 0; j < 2; j++) {
-    kw.rd_w[j] = KL::W_OFF + (32 * j + l32) * 16 + 8 * kh;
+    kw.rd_w[j] = KL::W_OFF + (FMT == WF_Q4 ? (32 * j + l32) * 16 + 8 * kh : 2 * kh * 1024 + (32 * j + l32) * 16);
     kw.rd_s[j] = KL::S_OFF + (32 * j + l32) * 2;
   }
 #pragma unroll
@@ -707,19 +579,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       }
   }
   if (n > 0) {  // steps relative to c0
-    kw.issue(0, 0);
-    kw.issue(1, min(1, n - 1));
-    kw.issue(2, min(2, n - 1));
+#pragma unroll
+    for (int st = 0; st < KL::NR - 1; st++) kw.issue(st, min(st, n - 1));
     int i = 0;
-    for (; i + 4 <= n; i += 4) {
-      kw.template step<0>(mine, min(i + 3, n - 1));
-      kw.template step<1>(mine, min(i + 4, n - 1));
-      kw.template step<2>(mine, min(i + 5, n - 1));
-      kw.template step<3>(mine, min(i + 6, n - 1));
-    }
-    if (i < n) kw.template step<0>(mine, n - 1);
-    if (i + 1 < n) kw.template step<1>(mine, n - 1);
-    if (i + 2 < n) kw.template step<2>(mine, n - 1);
+    for (; i + KL::NR <= n; i += KL::NR) KwSteps<KwWave<FMT, MT>, 0>::full(kw, mine, i, n);
+    KwSteps<KwWave<FMT, MT>, 0>::tail(kw, mine, i, n);
   }
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // every copy of this wave has landed
   __syncthreads();                           // every wave is done with its ring
@@ -851,11 +715,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   }
 }
 
-// TLM_GEMM_RING=0 selects the register-prefetch kernel for q4 too (comparisons)
-static const bool g_use_ring = [] {
-  const char* e = getenv("TLM_GEMM_RING");
-  return !(e && e[0] == '0');
-}();
 // TLM_GEMM_SPLIT_WAVES=n: split K while the grid holds at most n waves per CU
 // (default 4: with 32-row K-wave tiles, 4 beat 8 by 2-7 % from 127 to 1100
 // rows; every split adds an M x N fp32 slice that the consuming row kernel folds)
@@ -865,68 +724,89 @@ static const int g_split_waves = [] {
   return v > 0 && v <= 64 ? v : 4;
 }();
 
-GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus) {
+// What a GEMM takes, in us: fitted to 120 shapes drawn over 1-2048 rows,
+// 256-16384 columns and K 256-8192, each timed on every tile with 1-32 splits
+// (the fit is within 6-18 % rms, and the tile and split count it picks take
+// 2 % longer than the best ones in the mean, 31 % at most).
+struct GemmCost {
+  int tile;
+  float base;        // the launch and the first operands
+  float one, two;    // a 32-k step of one block on a CU; of the two that share it (0: one fits).
+                     // GT_KW: a step of a block's waves alone on a CU; per block of a shared CU
+  float slice, out;  // 1e6 floats of slices, written and folded; of a result stored unsplit
+};
+static const GemmCost kCostQ4[] = {{GT_KW, 3.7f, 0.15f, 0.22f, 2.6f, 1.6f}, {GT_128x256, 7.7f, 0.37f, 0.67f, 2.1f, 3.0f}};
+static const GemmCost kCostF16[] = {{GT_KW, 3.1f, 0.25f, 0.255f, 4.2f, 3.0f},
+                                    {GT_128x128, 5.6f, 0.19f, 0.40f, 2.6f, 3.0f},
+                                    {GT_256x256, 8.0f, 0.55f, 0.f, 2.0f, 2.7f}};
+constexpr float kFoldLaunch = 2.f;  // us: the second kernel, where the caller folds the slices itself
+
+static float gemm_cost(const GemmCost& c, int M, int N, int steps, int splits, int cus) {
+  const int bm = gemm_tile_rows(c.tile), bn = gemm_tile_cols(c.tile), spc = (steps + splits - 1) / splits;
+  const long blocks = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits;
+  const float mn = (float)M * N * 1e-6f, edge = c.base + (splits > 1 ? splits * c.slice : c.out) * mn;
+  if (c.tile == GT_KW) {
+    const int w = (spc + 3) / 4;
+    const float per_cu = blocks <= 4L * cus ? (float)((blocks + cus - 1) / cus) : (float)blocks / cus;
+    return edge + w * fmaxf(c.one, c.two * per_cu);
+  }
+  const long slots = c.two > 0.f ? 2 * cus : cus, rem = blocks % slots;
+  const float full = c.two > 0.f ? c.two : c.one;
+  return edge + spc * (full * (blocks / slots) + (rem == 0 ? 0.f : rem <= cus ? c.one : c.two));
+}
+
+GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part) {
   GemmShape s;
-  s.ring = fmt == WF_Q4 && g_use_ring;
-  s.wn = 1;
-  s.kw = 0;
   const int steps = K >= 32 ? K / 32 : 1;  // K % 32 != 0 is rejected by launch_gemm
-  int min_steps = 4;                       // 32-k steps per wave, at least
-  int kdiv = 1;                            // waves sharing one block's K range
-  if (s.ring) {
-    s.mt = M > 64 ? 4 : M > 32 ? 2 : 1;
-    s.nb = 2;
-    s.gy = (M + 32 * s.mt - 1) / (32 * s.mt);
-    if (((N + 255) / 256) * s.gy >= cus / 2) {  // four waves side by side over 256 columns
-      s.wn = 4;
-      s.gx = (N + 255) / 256;
-    } else {  // too few tiles to fill the CUs: four waves split K on one tile
-      // of 32 rows: 4x the blocks of 128-row tiles, and three blocks fit a CU
-      // (53 KB of LDS against 151 KB), which the re-read weight tiles (L2 hits)
-      // more than pay for (measured 5-25 % faster from 64 to 1100 rows)
-      s.kw = 1;
-      s.mt = 1;
-      s.gy = (M + 31) / 32;
-      s.gx = (N + kTile - 1) / kTile;
-      kdiv = 4;
-      min_steps = 2;
+  int splits = 1;
+  s.tile = GT_KW;
+  if (fmt == WF_Q4 && epi != GEMM_STORE) {
+    // four waves side by side over 256 columns, unless that leaves half the
+    // CUs idle: then four waves split K on one tile of 32 rows: 4x the blocks
+    // of 128-row tiles, and three blocks fit a CU (53 KB of LDS against
+    // 151 KB), which the re-read weight tiles (L2 hits) more than pay for
+    // (measured 5-25 % faster from 64 to 1100 rows)
+    const int tiles = ((N + 255) / 256) * ((M + 127) / 128);
+    if (M > 64 && tiles >= cus / 2) s.tile = GT_128x256;
+    const int kdiv = s.tile == GT_KW ? 4 : 1, min_steps = s.tile == GT_KW ? 2 : 4;
+    if (epi == GEMM_PART && s.tile != GT_KW) {
+      // two blocks per CU: pick the split count with the least
+      // (rounds of blocks x steps per block) + the split slices' write and read
+      // (M N 8 bytes each at ~6 TB/s, in units of a ~1 us step), the latter
+      // weighted 2x: the slice stores compete with the GEMM's own operand reads
+      // (measured 1-2 % faster 2048-row chunks than at weight 1, none slower)
+      const double slice_steps = 2.0 * (double)M * N * 8.0 / 6e6;
+      double best = 1e30;
+      for (int sp = 1; sp <= 32 && steps / sp >= min_steps; sp *= 2) {
+        const int rounds = (tiles * sp + 2 * cus - 1) / (2 * cus);
+        const double cost = (double)rounds * ((steps + sp - 1) / sp) + sp * slice_steps;
+        if (cost < best) best = cost, splits = sp;
+      }
+    } else if (epi == GEMM_PART) {
+      // split K while the grid stays within about g_split_waves waves per CU:
+      // past one round of blocks a CU streams the same bytes either way and each
+      // split only adds a slice for the next row kernel to fold (Qwen2.5-0.5B
+      // shape, 64 to 300 rows: the down GEMM in 4 splits instead of 8, the chunk
+      // 3-6 % faster)
+      const int target = g_split_waves * cus, waves = 4 * ((N + kTile - 1) / kTile) * ((M + 31) / 32);
+      while (splits < 32 && waves * splits * 2 <= target && steps / (2 * splits * kdiv) >= min_steps) splits *= 2;
     }
   } else {
-    s.mt = M > 64 ? 2 : 1;
-    s.nb = (epi == GEMM_SWIGLU || N > 64) ? 2 : 1;
-    s.gx = (N + 64 * s.nb - 1) / (64 * s.nb);
-    s.gy = (M + 64 * s.mt - 1) / (64 * s.mt);
-    s.wn = 4;
+    const GemmCost* tab = fmt == WF_Q4 ? kCostQ4 : kCostF16;
+    const int nt = fmt == WF_Q4 ? 2 : 3;
+    float best = INFINITY;
+    for (int i = 0; i < nt; i++)
+      for (int sp = 1; sp <= 32; sp *= 2) {
+        if (sp > 1 && (epi == GEMM_STORE ? (size_t)sp * M * N > part : epi != GEMM_PART)) break;
+        if (sp > 1 && steps / sp < (tab[i].tile == GT_KW ? 8 : 4)) break;
+        float c = gemm_cost(tab[i], M, N, steps, sp, cus);
+        if (sp > 1 && epi == GEMM_STORE) c += kFoldLaunch;
+        if (c < best) best = c, s.tile = tab[i].tile, splits = sp;
+      }
   }
-  int splits = 1;
-  if (epi == GEMM_PART && s.ring && !s.kw) {
-    // four-wave ring blocks, two per CU: pick the split count with the least
-    // (rounds of blocks x steps per block) + the split slices' write and read
-    // (M N 8 bytes each at ~6 TB/s, in units of a ~1 us step), the latter
-    // weighted 2x: the slice stores compete with the GEMM's own operand reads
-    // (measured 1-2 % faster 2048-row chunks than at weight 1, none slower)
-    const double slice_steps = 2.0 * (double)M * N * 8.0 / 6e6;
-    double best = 1e30;
-    for (int sp = 1; sp <= 32 && steps / sp >= min_steps; sp *= 2) {
-      const int rounds = (s.gx * s.gy * sp + 2 * cus - 1) / (2 * cus);
-      const double cost = (double)rounds * ((steps + sp - 1) / sp) + sp * slice_steps;
-      if (cost < best) best = cost, splits = sp;
-    }
-  } else if (epi == GEMM_PART) {
-    // split K while the grid stays within about g_split_waves waves per CU:
-    // past one round of blocks a CU streams the same bytes either way and each
-    // split only adds a slice for the next row kernel to fold (Qwen2.5-0.5B
-    // shape, 64 to 300 rows: the down GEMM in 4 splits instead of 8, the chunk
-    // 3-6 % faster; TLM_GEMM_SPLIT_FLOOR=0 splits until the grid reaches that
-    // size instead)
-    const int target = g_split_waves * cus;
-    const int waves = s.gx * s.gy * (s.ring ? (s.kw ? 4 : s.wn) : 4);
-    static const bool floor_rule = [] { const char* e = getenv("TLM_GEMM_SPLIT_FLOOR"); return !(e && e[0] == '0'); }();
-    if (floor_rule)
-      while (splits < 32 && waves * splits * 2 <= target && steps / (2 * splits * kdiv) >= min_steps) splits *= 2;
-    else
-      while (splits < 32 && waves * splits < target && steps / (2 * splits * kdiv) >= min_steps) splits *= 2;
-  }
+  const int bm = gemm_tile_rows(s.tile), bn = gemm_tile_cols(s.tile);
+  s.gx = (N + bn - 1) / bn;
+  s.gy = (M + bm - 1) / bm;
   s.spc = (steps + splits - 1) / splits;
   s.splits = (steps + s.spc - 1) / s.spc;
   return s;
@@ -934,54 +814,66 @@ GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus) {
 
 bool launch_gemm(int fmt, int epi, const GemmShape& sh, const GemmArgs& ga, hipStream_t st) {
   if (ga.K % 32 != 0 || ga.lda % 8 != 0 || ga.M <= 0 || ga.N <= 0) return false;
-  if (epi == GEMM_SWIGLU && (ga.N % kTile != 0 || sh.nb != 2)) return false;
+  if (epi == GEMM_SWIGLU && ga.N % kTile != 0) return false;
   if (epi != GEMM_PART && sh.splits != 1) return false;
-  if (epi == GEMM_ROPE && !(sh.ring && sh.kw && ga.N % kTile == 0)) return false;  // the K-wave kernel only
-  if (epi == GEMM_FOLD && !(sh.ring && sh.kw && ga.N % kTile == 0 && ga.N / kTile <= ga.ss_ld)) return false;
-  if (epi == GEMM_SWIGLU && ga.ss && !(sh.ring && sh.kw && ga.ss_ld <= 32)) return false;
+  const bool kw_q4 = fmt == WF_Q4 && sh.tile == GT_KW;  // RoPE and the fold: epilogues of this kernel only
+  if (epi == GEMM_ROPE && !(kw_q4 && ga.N % kTile == 0)) return false;
+  if (epi == GEMM_FOLD && !(kw_q4 && ga.N % kTile == 0 && ga.N / kTile <= ga.ss_ld)) return false;
+  if (epi == GEMM_SWIGLU && ga.ss && !(kw_q4 && ga.ss_ld <= 32)) return false;
   GemmArgs g = ga;
   g.spc = sh.spc;
   const dim3 grid(sh.gx, sh.gy, sh.splits);
-  const int mt = sh.mt, nb = sh.nb;
-  if (sh.ring && sh.kw) {
-    if (fmt != WF_Q4) return false;
-#define KW_CASE(MTV, E)                                                                          \
-  if (mt == MTV && epi == E) {                                                                   \
-    hipLaunchKernelGGL((gemm_q4_kw_kernel<MTV, E>), grid, dim3(256), 0, st, g);                  \
-    return true;                                                                                 \
+#define KW_CASE(F, E)                                                              \
+  if (fmt == F && sh.tile == GT_KW && epi == E) {                                  \
+    hipLaunchKernelGGL((gemm_kw_kernel<F, 1, E>), grid, dim3(256), 0, st, g);      \
+    return true;                                                                   \
   }
-#define KW_EPIS(MTV) KW_CASE(MTV, GEMM_STORE) KW_CASE(MTV, GEMM_PART) KW_CASE(MTV, GEMM_SWIGLU) KW_CASE(MTV, GEMM_ROPE) \
-  KW_CASE(MTV, GEMM_FOLD)
-    KW_EPIS(1)  // gemm_shape gives the K-wave blocks 32 rows
-#undef KW_EPIS
-#undef KW_CASE
-    return false;
+#define RING_CASE(F, TILE, MT, WM, WN, NS, E)                                                             \
+  if (fmt == F && sh.tile == TILE && epi == E) {                                                          \
+    hipLaunchKernelGGL((gemm_ring_kernel<F, MT, WM, WN, NS, E>), grid, dim3(64 * WM * WN), 0, st, g);     \
+    return true;                                                                                          \
   }
-  if (sh.ring) {
-    if (fmt != WF_Q4) return false;
-#define RING_CASE(MTV, WNV, E)                                                                   \
-  if (mt == MTV && sh.wn == WNV && epi == E) {                                                   \
-    hipLaunchKernelGGL((gemm_q4_ring_kernel<MTV, WNV, E>), grid, dim3(64 * WNV), 0, st, g);      \
-    return true;                                                                                 \
-  }
-#define RING_EPIS(MTV, WNV) RING_CASE(MTV, WNV, GEMM_STORE) RING_CASE(MTV, WNV, GEMM_PART) RING_CASE(MTV, WNV, GEMM_SWIGLU)
-    RING_EPIS(1, 4) RING_EPIS(2, 4) RING_EPIS(4, 4)
+#define RING_EPIS(F, TILE, MT, WM, WN, NS)       \
+  RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_STORE) \
+  RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_PART)  \
+  RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_SWIGLU)
+  KW_CASE(WF_Q4, GEMM_STORE) KW_CASE(WF_Q4, GEMM_PART) KW_CASE(WF_Q4, GEMM_SWIGLU)
+  KW_CASE(WF_Q4, GEMM_ROPE) KW_CASE(WF_Q4, GEMM_FOLD)
+  KW_CASE(WF_F16, GEMM_STORE) KW_CASE(WF_F16, GEMM_PART) KW_CASE(WF_F16, GEMM_SWIGLU)
+  RING_EPIS(WF_Q4, GT_128x256, 4, 1, 4, 4)
+  RING_EPIS(WF_F16, GT_128x128, 2, 2, 2, 4)
+  RING_EPIS(WF_F16, GT_256x256, 4, 2, 4, 4)
 #undef RING_EPIS
 #undef RING_CASE
-    return false;
-  }
-#define GEMM_CASE(F, MTV, NBV, E)                                                         \
-  if (fmt == F && mt == MTV && nb == NBV && epi == E) {                                   \
-    hipLaunchKernelGGL((gemm_kernel<F, MTV, NBV, E>), grid, dim3(256), 0, st, g);         \
-    return true;                                                                          \
-  }
-#define GEMM_EPIS(F, MTV, NBV) \
-  GEMM_CASE(F, MTV, NBV, GEMM_STORE) GEMM_CASE(F, MTV, NBV, GEMM_PART) GEMM_CASE(F, MTV, NBV, GEMM_SWIGLU)
-  GEMM_EPIS(WF_Q4, 1, 1) GEMM_EPIS(WF_Q4, 1, 2) GEMM_EPIS(WF_Q4, 2, 1) GEMM_EPIS(WF_Q4, 2, 2)
-  GEMM_EPIS(WF_F16, 1, 1) GEMM_EPIS(WF_F16, 1, 2) GEMM_EPIS(WF_F16, 2, 1) GEMM_EPIS(WF_F16, 2, 2)
-#undef GEMM_EPIS
-#undef GEMM_CASE
+#undef KW_CASE
   return false;
+}
+
+// y[m][n] = bias[n] + the sum of the split-K slices, in slice order: a
+// streaming pass over (n_part + 1) M N floats.
+template <int V>
+__global__ __launch_bounds__(256) void fold_rows_kernel(const float* part, int n_part, const float* bias, unsigned N,
+                                                        unsigned n, float* y) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  const unsigned i = (blockIdx.x * 256 + threadIdx.x) * V;
+  if (i >= n) return;
+  vec v = {};
+  if (bias) {
+#pragma unroll
+    for (int e = 0; e < V; e++) v[e] = bias[i % N + e];
+  }
+#pragma unroll 4
+  for (int s = 0; s < n_part; s++) v += *reinterpret_cast<const vec*>(part + (size_t)s * n + i);
+  *reinterpret_cast<vec*>(y + i) = v;
+}
+
+// M N < 2^31 (the slices' buffer is far smaller)
+void launch_fold_rows(const float* part, int n_part, const float* bias, int M, int N, float* y, hipStream_t st) {
+  const unsigned n = (unsigned)M * N;
+  if (N % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0)
+    hipLaunchKernelGGL(fold_rows_kernel<4>, dim3((n / 4 + 255) / 256), dim3(256), 0, st, part, n_part, bias, N, n, y);
+  else
+    hipLaunchKernelGGL(fold_rows_kernel<1>, dim3((n + 255) / 256), dim3(256), 0, st, part, n_part, bias, N, n, y);
 }
 
 // ------------------------------------------------------------ row kernels --
