@@ -1,0 +1,88 @@
+"""tlm_op_attention_rows where its kernel can go wrong: key and query tiles that
+end inside a tile, a softmax reference that moves with every tile or never, rows
+with nothing to see in a tile, and the two ways the queries reach the kernel.
+
+No rotation (frequencies of zero) and queries and keys on a coarse grid make
+every score exact in fp32; what is left is fp16 probabilities (2^-10 each,
+rounded toward zero) and the fp16 output, so 2e-3 bounds the error of a
+weighted mean of values of unit scale."""
+import math
+
+import numpy as np
+import pytest
+
+import three_llm_amd.tlm as tlm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = tlm.Context(0)
+    yield c
+    c.close()
+
+
+def inputs(rng, n, heads, kv, D, slope):
+    """Rows whose scores change by about `slope` (log2) per key position."""
+    q = rng.integers(-2, 3, (n, heads, D)) / 8.0
+    k = rng.integers(-8, 9, (n, kv, D)) / 8.0
+    q[:, :, 0] = 1.0
+    k[:, :, 0] = np.round(np.arange(n) * slope * 8)[:, None] / 8.0
+    v = rng.standard_normal((n, kv, D)).astype(np.float16).astype(np.float32)
+    return np.concatenate([x.reshape(n, -1) for x in (q, k, v)], 1).astype(np.float32)
+
+
+def expected(x, p0, heads, kv, D, window):
+    n = x.shape[0]
+    q = x[p0:, :heads * D].astype(np.float64).reshape(n - p0, heads, D)
+    k = x[:, heads * D:(heads + kv) * D].astype(np.float64).reshape(n, kv, D)
+    v = x[:, (heads + kv) * D:].astype(np.float64).reshape(n, kv, D)
+    pos, key = np.arange(p0, n)[:, None], np.arange(n)[None, :]
+    hidden = (key > pos) | ((key <= pos - window) if window else False)
+    out = np.empty((n - p0, heads, D))
+    for h in range(heads):
+        s = np.where(hidden, -np.inf, q[:, h] @ k[:, h // (heads // kv)].T)
+        p = np.exp2(s - s.max(1, keepdims=True))
+        out[:, h] = (p / p.sum(1, keepdims=True)) @ v[:, h // (heads // kv)]
+    return out.reshape(n - p0, heads * D)
+
+
+@pytest.mark.parametrize("heads,kv,D", [(7, 1, 64), (4, 2, 64), (3, 1, 128)])
+@pytest.mark.parametrize("p0,rows,window,slope", [
+    (0, 1, 0, 0.0), (0, 33, 0, 1.0), (31, 34, 0, -1.0), (63, 1, 0, 1.0), (64, 65, 0, 0.5), (1, 127, 0, -0.25),
+    (200, 161, 0, 4.0), (200, 161, 0, -4.0), (190, 100, 30, 1.0), (190, 100, 1, 0.0), (100, 200, 129, -2.0),
+])
+def test_rows_at_tile_edges_and_moving_references(ctx, heads, kv, D, p0, rows, window, slope):
+    print(f"[attention rows] {heads}/{kv} x {D}, {rows} at {p0}, window {window}, slope {slope}", flush=True)
+    rng = np.random.default_rng(heads * 1000 + p0 + rows)
+    n = p0 + rows
+    x = inputs(rng, n, heads, kv, D, slope)
+    A = tlm.Attention(ctx, heads, kv, D, n, np.zeros(D // 2, np.float32), sliding_window=window,
+                      attn_scale=math.log(2.0))
+    if p0:
+        A.rows(ctx.array(x[:p0]), p0, 0, ctx.buffer(2 * p0 * heads * D))
+    got = A.rows(ctx.array(x[p0:]), rows, p0, ctx.buffer(2 * rows * heads * D)).read(np.uint16)
+    A.close()
+    got = got.view(np.float16).astype(np.float64).reshape(rows, heads * D)
+    ref = expected(x, p0, heads, kv, D, window)
+    assert np.abs(got - ref).max() <= 2e-3 * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_rows_written_over_their_projections_equal_rows_apart(ctx, D):
+    """out inside qkv: the queries are staged, with the same result."""
+    heads, kv, rows = 6, 2, 70
+    rng = np.random.default_rng(D)
+    x = rng.standard_normal((rows, (heads + 2 * kv) * D)).astype(np.float32)
+    inv = (1e4 ** (-np.arange(0, D, 2) / D)).astype(np.float32)
+    outs = []
+    for inside in (False, True):
+        A = tlm.Attention(ctx, heads, kv, D, rows, inv)
+        qkv = ctx.array(x)
+        out = A.rows(qkv, rows, 0, qkv if inside else ctx.buffer(2 * rows * heads * D))
+        outs.append(out.read(np.uint16)[:rows * heads * D].copy())
+        A.close()
+    # RoPE of the staged queries may be contracted differently: one fp16 step of a query
+    a, b = (o.view(np.float16).astype(np.float64) for o in outs)
+    assert np.abs(a - b).max() <= 2e-3 * np.abs(a).max()

@@ -920,7 +920,7 @@ int tlm_op_attention(tlm_attn* A, const float* qkv, int position, float* out) {
 
 // RoPE + cache append of `rows` positions from position0, then their causal
 // attention, enqueued on the context's stream; q: fp16 staging of the rotated
-// queries, [rows][heads * head_dim].
+// queries, [rows][heads * head_dim], or null where none is needed.
 static int check_attention_rows(const tlm_attn* A, const float* qkv, int32_t rows, int32_t position0,
                                 const uint16_t* out) {
   if (!A || !qkv || !out || rows <= 0) return fail(TLM_ERR_INVALID, "TLMAttention: invalid argument");
@@ -933,10 +933,22 @@ static int check_attention_rows(const tlm_attn* A, const float* qkv, int32_t row
   return TLM_OK;
 }
 
+// With full rotary the attention kernel forms its queries itself, from qkv,
+// which out may not share an address with (a block writes its rows of out while
+// others still read theirs of qkv); otherwise q stages them.
+static bool rows_need_staging(const tlm_attn* A, const float* qkv, int32_t rows, const uint16_t* out) {
+  const tlm_attn_desc& d = A->d;
+  const uintptr_t x = reinterpret_cast<uintptr_t>(qkv), o = reinterpret_cast<uintptr_t>(out);
+  const size_t nx = sizeof(float) * (size_t)rows * (d.heads + 2 * d.kv_heads) * d.head_dim;
+  const size_t no = sizeof(uint16_t) * (size_t)rows * d.heads * d.head_dim;
+  return d.rotary_dim != d.head_dim || (x < o + no && o < x + nx);
+}
+
 static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, int32_t position0, uint16_t* out,
                                    uint16_t* q) {
   const tlm_attn_desc& d = A->d;
   hipStream_t st = A->ctx->stream;
+  const float qscale = A->scale * 1.4426950408889634f;  // log2 e: the softmax runs in base 2
   RopeKvArgs r;
   memset(&r, 0, sizeof r);
   r.qkv = qkv;
@@ -946,18 +958,26 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   r.p0 = position0;
   r.Hq = d.heads;
   r.Hkv = d.kv_heads;
+  r.h0 = q ? 0 : d.heads;
   r.D = d.head_dim;
   r.rd = d.rotary_dim;
   r.max_tokens = d.max_tokens;
   r.rope_cos = A->rope_cos;
   r.rope_sin = A->rope_sin;
   r.q = q;
+  r.qscale = qscale;
   r.kc = A->kc;
   r.vc = A->vc;
   launch_rope_kv(r, st);
   PrefillAttnArgs pa;
   memset(&pa, 0, sizeof pa);
   pa.q = q;
+  if (!q) {
+    pa.qkv = qkv;
+    pa.rope_cos = A->rope_cos;
+    pa.rope_sin = A->rope_sin;
+    pa.qscale = qscale;
+  }
   pa.kc = A->kc;
   pa.vc = A->vc;
   pa.out = out;
@@ -969,7 +989,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   pa.G = A->G;
   pa.max_tokens = d.max_tokens;
   pa.window = d.sliding_window;
-  pa.scale_log2 = A->scale * 1.4426950408889634f;
   return launch_prefill_attention(pa, st);
 }
 
@@ -977,11 +996,12 @@ int tlm_op_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, int32_t p
   int rc = check_attention_rows(A, qkv, rows, position0, out);
   if (rc) return rc;
   uint16_t* q = nullptr;
-  HIP_TRY(hipMalloc(&q, sizeof(uint16_t) * (size_t)rows * A->d.heads * A->d.head_dim));
+  if (rows_need_staging(A, qkv, rows, out))
+    HIP_TRY(hipMalloc(&q, sizeof(uint16_t) * (size_t)rows * A->d.heads * A->d.head_dim));
   const bool launched = enqueue_attention_rows(A, qkv, rows, position0, out, q);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(A->ctx->stream);
-  hipFree(q);
+  if (q) hipFree(q);
   if (e != hipSuccess) return fail(TLM_ERR_HIP, "TLMAttention: batched rows failed: %s", hipGetErrorString(e));
   if (!launched) return fail(TLM_ERR_STATE, "TLMAttention: no batched attention kernel for this shape");
   return TLM_OK;
@@ -996,7 +1016,8 @@ int tlm_op_attention_rows_noalloc(tlm_attn* A, const float* qkv, int32_t rows, i
                 "entry point holds %zu (at most %zu rows of this shape)", rows, need, kScratchBytes,
                 kScratchBytes / (sizeof(uint16_t) * A->d.heads * A->d.head_dim));
   if (!A->ctx->scratch) return fail(TLM_ERR_STATE, "TLMAttention: the context has no scratch address");
-  if (!enqueue_attention_rows(A, qkv, rows, position0, out, static_cast<uint16_t*>(A->ctx->scratch)))
+  uint16_t* q = rows_need_staging(A, qkv, rows, out) ? static_cast<uint16_t*>(A->ctx->scratch) : nullptr;
+  if (!enqueue_attention_rows(A, qkv, rows, position0, out, q))
     return fail(TLM_ERR_STATE, "TLMAttention: no batched attention kernel for this shape");
   CHECK_LAUNCH("TLMAttention");
   return TLM_OK;
@@ -1927,6 +1948,7 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
   const int H = d.hidden_size, I = d.intermediate_size, D = d.head_dim;
   const int lf = wfmt(d.linear_fmt);
   const size_t rowsH = (size_t)M * H;
+  const float qscale = m->attn.scale * 1.4426950408889634f;  // log2 e: the softmax runs in base 2
   // per layer: two row kernels (one when the O GEMM folds its rows; layer 0's
   // first one also gathers the embedding rows), the QKV GEMM (+ rope_kv unless
   // RoPE runs in its epilogue), attention and three GEMMs; then the last fold
@@ -1952,6 +1974,7 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
       g.rope_cos = m->attn.rope_cos;
       g.rope_sin = m->attn.rope_sin;
       g.ctrl = m->ctrl;
+      g.qscale = qscale;
       g.Hq = d.num_heads;
       g.Hkv = d.num_kv_heads;
       g.max_tokens = d.max_tokens;
@@ -1978,6 +2001,7 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
       r.rope_cos = m->attn.rope_cos;
       r.rope_sin = m->attn.rope_sin;
       r.q = m->pf_q;
+      r.qscale = qscale;
       r.kc = L.kc;
       r.vc = L.vc;
       r.kv_f32 = 0;
@@ -1998,7 +2022,6 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
     pa.G = m->attn.G;
     pa.max_tokens = d.max_tokens;
     pa.window = m->windows[l];
-    pa.scale_log2 = m->attn.scale * 1.4426950408889634f;
     ok = ok && launch_prefill_attention(pa, st);
     g = gemm_args(L.o, m->pf_att, m->QS, M);
     g.ldc = H;

@@ -664,8 +664,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         if (kind == 0) {
           uint16_t* qr = g.Ch + (size_t)row * g.ldc + t0 * kTile;
-          qr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0));
-          qr[d + 32] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y1));
+          qr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0 * g.qscale));
+          qr[d + 32] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y1 * g.qscale));
         } else {
           uint16_t* cr = (kind == 1 ? g.kc : g.vc) + ((size_t)hk * g.max_tokens + pos) * kTile;
           cr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0));
@@ -953,7 +953,7 @@ __device__ __forceinline__ float fold_slices(const float* row, const float* bias
 __device__ __forceinline__ void rope_store(const RopeKvArgs& a, int m, int pos, int i, float y) {
   const int nq = a.Hq * a.D, nk = a.Hkv * a.D;
   if (i < nq) {
-    a.q[(size_t)m * nq + i] = __builtin_bit_cast(uint16_t, f16_guard(a.ovf, y));
+    a.q[(size_t)m * nq + i] = __builtin_bit_cast(uint16_t, f16_guard(a.ovf, y * a.qscale));
     return;
   }
   const bool isv = i >= nq + nk;
@@ -990,7 +990,7 @@ __device__ __forceinline__ void rope_pair(const RopeKvArgs& a, int pi, int& i0, 
 constexpr int RKV_ROWS = 2;
 __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
   const int D = a.D, width = (a.Hq + 2 * a.Hkv) * D;
-  const int pi = blockIdx.y * 256 + threadIdx.x;
+  const int pi = a.h0 * (D / 2) + blockIdx.y * blockDim.x + threadIdx.x;
   if (pi >= width / 2) return;
   int i0, i1, dr;
   bool rot;
@@ -1035,6 +1035,7 @@ __device__ __forceinline__ float4 fold_slices4(const float* row, const float* bi
 
 __device__ __forceinline__ void rope_store4(const RopeKvArgs& a, int m, int pos, int i, float4 y) {
   const int nq = a.Hq * a.D, nk = a.Hkv * a.D;
+  if (i < nq) y.x *= a.qscale, y.y *= a.qscale, y.z *= a.qscale, y.w *= a.qscale;
   const half4_t h = {f16_guard(a.ovf, y.x), f16_guard(a.ovf, y.y), f16_guard(a.ovf, y.z), f16_guard(a.ovf, y.w)};
   uint16_t* dst;
   if (i < nq) {
@@ -1049,7 +1050,7 @@ __device__ __forceinline__ void rope_store4(const RopeKvArgs& a, int m, int pos,
 
 __global__ __launch_bounds__(256) void rope_kv4_kernel(RopeKvArgs a) {
   const int D = a.D, g8 = D / 8, groups = (a.Hq + 2 * a.Hkv) * g8, half = D / 2;
-  const int g = blockIdx.y * 256 + threadIdx.x;
+  const int g = a.h0 * g8 + blockIdx.y * blockDim.x + threadIdx.x;
   if (g >= groups) return;
   const int h = g / g8, j = g - h * g8;
   const bool rot = h < a.Hq + a.Hkv;
@@ -1090,14 +1091,13 @@ static const bool g_rope_vec = [] {
 
 void launch_rope_kv(const RopeKvArgs& a, hipStream_t st) {
   const bool vec = g_rope_vec && !a.kv_f32 && a.rd == a.D && a.D % 8 == 0 && a.pstride % 4 == 0;
-  if (vec) {
-    const int groups = (a.Hq + 2 * a.Hkv) * a.D / 8;
-    hipLaunchKernelGGL(rope_kv4_kernel, dim3((a.M + RKV_ROWS - 1) / RKV_ROWS, (groups + 255) / 256), dim3(256), 0, st,
-                       a);
-    return;
-  }
-  const int pairs = (a.Hq + 2 * a.Hkv) * a.D / 2;
-  hipLaunchKernelGGL(rope_kv_kernel, dim3((a.M + RKV_ROWS - 1) / RKV_ROWS, (pairs + 255) / 256), dim3(256), 0, st, a);
+  const int work = (a.Hq + 2 * a.Hkv - a.h0) * a.D / (vec ? 8 : 2);  // threads per row
+  const int bt = min(256, (work + 63) / 64 * 64);
+  const dim3 grid((a.M + RKV_ROWS - 1) / RKV_ROWS, (work + bt - 1) / bt);
+  if (vec)
+    hipLaunchKernelGGL(rope_kv4_kernel, grid, dim3(bt), 0, st, a);
+  else
+    hipLaunchKernelGGL(rope_kv_kernel, grid, dim3(bt), 0, st, a);
 }
 
 // ------------------------------------------------------- flash attention --
@@ -1106,25 +1106,42 @@ void launch_rope_kv(const RopeKvArgs& a, hipStream_t st) {
 // query heads of the group (one wave each), times NG key groups: group z
 // takes key tiles z, z + NG, ... and the groups merge their (max, sum, O) at
 // the end, which halves the serial chain of the long (late) query tiles.
-// Per tile of 64 keys: K rows and V^T sit in LDS (double buffered; the next
-// tiles' rows are loaded into registers while this one is computed, one
+// Per tile of 64 keys: K and V rows sit in LDS (double buffered; the next
+// tile's rows are copied there, global -> LDS, while this one is computed, one
 // barrier per tile); S^T = K Q^T (lane = query, registers = keys), an online
 // softmax in registers (the two half-waves of a query exchange one value;
-// masks only on tiles that cross the causal diagonal or the window start; O
-// is rescaled only when some row's max moved), then O^T += V^T P^T with P^T
-// taken straight from the S^T registers: the key order of the contraction is
-// permuted to match that register layout.  P is rounded to fp16 toward zero.
-template <int DT, int NG>
+// masks only on tiles that cross the causal diagonal or the window start),
+// then O^T += V^T P^T with P^T taken straight from the S^T registers: the key
+// order of the contraction is permuted to match that register layout.
+// The vector ALU's share per score bounds it (a tile's 32 scores a lane
+// against 16 MFMAs), so that is kept to an exponential, half a max3, half a
+// conversion and half a dot product: the queries carry scale * log2 e, the
+// score accumulators start at minus the softmax's reference, the reference
+// moves only when a score passes it by kRefSlack (O is rescaled then; fp16 P
+// stays below 2^9), and the sum adds the pairs of P as the matrix cores see
+// them, rounded toward zero to fp16.  2048 rows of the Llama-3.2-1B heads: 38
+// -> 30 us from position 0, 90 -> 66 us from 2048, of which the copies that
+// stay in flight across the math (register staging was sunk below it) gave
+// about 8; four waves per SIMD need <= 128 registers, hence the copies.
+template <int DT>
 struct AttnTile {
-  static constexpr int KT = 64;            // keys per tile
-  static constexpr int KS = DT + 8;        // halves per K row in LDS
-  // halves per V row: the four rows a half-wave's transposing reads touch fall
-  // on different banks (row strides of 40 and 80 dwords)
-  static constexpr int VS = DT + (DT == 64 ? 16 : 32);
-  static constexpr int PIECES = KT * DT / 8;  // 16-byte pieces of K (or V) per tile
-  static constexpr int PPT = PIECES / 256;    // pieces per thread (256 threads per key group)
-  static constexpr int TILE_HALVES = KT * KS + KT * VS;
+  static constexpr int KT = 64;             // keys per tile
+  static constexpr int P = DT / 8;          // 16-byte pieces of a K or V row
+  static constexpr int ROWB = DT * 2;       // bytes of a row
+  static constexpr int HALF = KT * ROWB;    // bytes of the tile's K (and of its V, which follows)
+  static constexpr int BYTES = 2 * HALF;
+  static constexpr int CPW = HALF / 4096;   // 1 KiB copies of K (and of V) per wave of a key group
 };
+
+// Position (16-byte piece) in LDS of piece q of row r: q ^ f(r).  The 64 banks
+// hold 16 pieces (two rows of head_dim 64, one of 128): f puts the same piece
+// of 16 consecutive rows (the K reads) and the four pieces of a 32-dim tile of
+// 4 consecutive rows (a half-wave's transposing V read) on distinct banks.
+template <int DT>
+__device__ __forceinline__ int kv_swz(int r) {
+  const int b0 = r & 1, b1 = (r >> 1) & 1, b2 = (r >> 2) & 1, b3 = (r >> 3) & 1;
+  return DT == 64 ? (b0 ^ b3) | (b2 << 1) | (b1 << 2) : b2 | (b3 << 1) | (b0 << 2) | (b1 << 3);
+}
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 // ds_read_b64_tr_b16 (gfx950): in each group of 16 lanes, lane j names 4
@@ -1132,47 +1149,28 @@ typedef short short4_t __attribute__((ext_vector_type(4)));
 // With lane j at V[key0 + j / 4][d0 + 4 (j % 4)], lane i receives
 // V[key0 + k][d0 + i]: four consecutive keys of one dim (checked on the
 // device with an index-valued LDS probe).
-__device__ __forceinline__ half4_t lds_read_tr4(const _Float16* p) {
+__device__ __forceinline__ half4_t lds_read_tr4(const unsigned char* p) {
   const short4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (short4_t __attribute__((address_space(3)))*)(p));
   return __builtin_bit_cast(half4_t, v);
 }
 
-// K and V pieces of one tile in registers: piece i is row i / (DT / 8), dims
-// 8 (i % (DT / 8)) .. + 7; rows past qhi repeat row qhi (their keys are masked).
-template <int DT, int NG>
-struct AttnStage {
-  using AT = AttnTile<DT, NG>;
-  uint4 kr[AT::PPT], vr[AT::PPT];
-  __device__ __forceinline__ void load(const _Float16* kb, const _Float16* vb, int kt0, int qhi, int t) {
-#pragma unroll
-    for (int u = 0; u < AT::PPT; u++) {
-      const int i = t + 256 * u;
-      const size_t src = (size_t)min(kt0 + i / (DT / 8), qhi) * DT + 8 * (i % (DT / 8));
-      kr[u] = *reinterpret_cast<const uint4*>(kb + src);
-      vr[u] = *reinterpret_cast<const uint4*>(vb + src);
-    }
-  }
-  // K and V rows as they are (V is read transposed, lds_read_tr4)
-  __device__ __forceinline__ void store(_Float16* tile, int t) const {
-    _Float16* ks = tile;
-    _Float16* vs = tile + AT::KT * AT::KS;
-#pragma unroll
-    for (int u = 0; u < AT::PPT; u++) {
-      const int i = t + 256 * u, r = i / (DT / 8), c8 = i % (DT / 8);
-      *reinterpret_cast<uint4*>(&ks[r * AT::KS + 8 * c8]) = kr[u];
-      *reinterpret_cast<uint4*>(&vs[r * AT::VS + 8 * c8]) = vr[u];
-    }
-  }
-};
+// v_maximum3_f32: unlike fmaxf it takes its inputs as they are (no
+// canonicalising copies); a NaN wins and stays in the output
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
+}
+// A score may exceed the reference by this much (log2) before it moves
+constexpr float kRefSlack = 8.f;
 
-template <int DT, int NG>
-__global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) void prefill_attn_kernel(PrefillAttnArgs a) {
-  using AT = AttnTile<DT, NG>;
-  constexpr int KT = AT::KT, KS = AT::KS, VS = AT::VS, NDT = DT / 32;
-  __shared__ __align__(16) _Float16 lds[2 * NG * AT::TILE_HALVES];
+template <int DT, int NG, bool QF>
+__global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 64 ? 4 : 2))) void prefill_attn_kernel(PrefillAttnArgs a) {
+  using AT = AttnTile<DT>;
+  constexpr int KT = AT::KT, NDT = DT / 32;
+  __shared__ __align__(16) unsigned char lds[2 * NG * AT::BYTES];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int grp = __builtin_amdgcn_readfirstlane(tid >> 8), t256 = tid & 255, wave = t256 >> 6;
+  const int grp = __builtin_amdgcn_readfirstlane(tid >> 8), t256 = tid & 255;
+  const int wave = __builtin_amdgcn_readfirstlane(t256 >> 6);
   const int l32 = lane & 31, kh = lane >> 5;
   const int nqt = (a.M + 31) / 32;
   // Longest key ranges first in the lower half of the (head, group) blocks and
@@ -1192,41 +1190,96 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) v
   const int QW = a.Hq * DT;
 
   half8_t qb[DT / 16];
-  const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)min(qr, a.M - 1) * QW + h * DT;
+  if constexpr (QF) {  // the lane's query row from its fp32 projection: RoPE pairs (d, d + DT / 2)
+    const int m = min(qr, a.M - 1);
+    const float* x = a.qkv + (size_t)m * (a.Hq + 2 * a.Hkv) * DT + h * DT;
+    const float* ct = a.rope_cos + (size_t)(p0 + m) * (DT / 2);
+    const float* st = a.rope_sin + (size_t)(p0 + m) * (DT / 2);
 #pragma unroll
-  for (int j = 0; j < DT / 16; j++) qb[j] = *reinterpret_cast<const half8_t*>(qrow + 16 * j + 8 * kh);
+    for (int j = 0; j < DT / 32; j++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const int d = 16 * j + 8 * kh + e;
+        const float4 u = *reinterpret_cast<const float4*>(x + d), v = *reinterpret_cast<const float4*>(x + d + DT / 2);
+        const float4 c = *reinterpret_cast<const float4*>(ct + d), s = *reinterpret_cast<const float4*>(st + d);
+        half8_t &lo = qb[j], &hi = qb[j + DT / 32];
+        lo[e] = (_Float16)((u.x * c.x - v.x * s.x) * a.qscale), hi[e] = (_Float16)((v.x * c.x + u.x * s.x) * a.qscale);
+        lo[e + 1] = (_Float16)((u.y * c.y - v.y * s.y) * a.qscale), hi[e + 1] = (_Float16)((v.y * c.y + u.y * s.y) * a.qscale);
+        lo[e + 2] = (_Float16)((u.z * c.z - v.z * s.z) * a.qscale), hi[e + 2] = (_Float16)((v.z * c.z + u.z * s.z) * a.qscale);
+        lo[e + 3] = (_Float16)((u.w * c.w - v.w * s.w) * a.qscale), hi[e + 3] = (_Float16)((v.w * c.w + u.w * s.w) * a.qscale);
+      }
+  } else {
+    const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)min(qr, a.M - 1) * QW + h * DT;
+#pragma unroll
+    for (int j = 0; j < DT / 16; j++) qb[j] = *reinterpret_cast<const half8_t*>(qrow + 16 * j + 8 * kh);
+  }
 
+  // this wave's copies of a tile: slot 64 u + lane of its K (and V) holds piece
+  // cq[u] of row cr[u] (rows past qhi repeat row qhi: their keys are masked)
   const _Float16* kb = reinterpret_cast<const _Float16*>(a.kc) + (size_t)hk * a.max_tokens * DT;
   const _Float16* vb = reinterpret_cast<const _Float16*>(a.vc) + (size_t)hk * a.max_tokens * DT;
-  AttnStage<DT, NG> sg;
+  int cr[AT::CPW], cq[AT::CPW];
+#pragma unroll
+  for (int u = 0; u < AT::CPW; u++) {
+    const int slot = (wave * AT::CPW + u) * 64 + lane;
+    cr[u] = slot / AT::P;
+    cq[u] = ((slot % AT::P) ^ kv_swz<DT>(cr[u])) * 16;
+  }
+  const uint32_t gbase = (uint32_t)(uintptr_t)lds + grp * AT::BYTES + wave * AT::CPW * 1024;
+  auto stage = [&](int buf, int kt0) {
+#pragma unroll
+    for (int u = 0; u < AT::CPW; u++) {
+      const uint32_t off = (uint32_t)(min(kt0 + cr[u], qhi) * AT::ROWB + cq[u]);
+      const uint32_t dst = gbase + buf * NG * AT::BYTES + u * 1024;
+      lds_dma16(kb, off, __builtin_amdgcn_readfirstlane(dst));
+      lds_dma16(vb, off, __builtin_amdgcn_readfirstlane(dst + AT::HALF));
+    }
+  };
+  // every wave's copies have landed and its LDS reads are complete
+  auto landed = [] {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+    asm volatile("s_barrier" ::: "memory");
+  };
+  // LDS offsets of this lane's K pieces (of 32 keys; 32 keys further the
+  // swizzle is the same) and V pieces
+  int rk[DT / 16], rv[NDT][4];
+#pragma unroll
+  for (int j = 0; j < DT / 16; j++) rk[j] = l32 * AT::ROWB + ((2 * j + kh) ^ kv_swz<DT>(l32)) * 16;
+#pragma unroll
+  for (int i = 0; i < NDT; i++)
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int r = 4 * kh + (lane & 15) / 4 + 8 * s, d = 32 * i + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+      rv[i][s] = r * AT::ROWB + ((d / 8) ^ kv_swz<DT>(r)) * 16 + (d % 8) * 2;
+    }
 
   float16_t o[NDT];
 #pragma unroll
   for (int i = 0; i < NDT; i++) o[i] = (float16_t){};
-  float mrun = -INFINITY, lrun = 0.f;  // running max (log2 units) and this half-wave's sum
+  // the reference of the exponents (log2 units, -inf before the first key) and
+  // this half-wave's sum
+  float mrun = -INFINITY, lrun = 0.f;
+  float16_t neg_ref = {};
   const int kbeg = kfirst & ~(KT - 1);
   const int ntiles = (qhi - kbeg) / KT + 1;
   const int nsteps = (ntiles + NG - 1) / NG;
-  _Float16* const mytile = lds + grp * AT::TILE_HALVES;  // buffer b at + b NG TILE_HALVES
-  sg.load(kb, vb, kbeg + grp * KT, qhi, t256);
-  sg.store(mytile, t256);
-  __syncthreads();
+  stage(0, kbeg + grp * KT);
+  landed();
   for (int it = 0; it < nsteps; it++) {
     const int buf = it & 1, tile = it * NG + grp, kt0 = kbeg + tile * KT;
-    sg.load(kb, vb, kt0 + NG * KT, qhi, t256);  // this group's next tile, in flight during the math
-    if (tile < ntiles) {
-      const _Float16* kbuf = mytile + buf * NG * AT::TILE_HALVES;
-      const _Float16* vbuf = kbuf + KT * KS;
+    if (tile + NG < ntiles) stage(buf ^ 1, kt0 + NG * KT);  // this group's next tile, in flight during the math
+    if (tile < ntiles && active) {
+      const unsigned char* kbuf = lds + (buf * NG + grp) * AT::BYTES;
+      const unsigned char* vbuf = kbuf + AT::HALF;
+      // scores less the reference: the accumulators start at -mref
       float16_t s[2];
 #pragma unroll
-      for (int b2 = 0; b2 < 2; b2++) {
-        s[b2] = (float16_t){};
+      for (int j = 0; j < DT / 16; j++)
 #pragma unroll
-        for (int j = 0; j < DT / 16; j++) {
-          const half8_t ak = *reinterpret_cast<const half8_t*>(kbuf + (32 * b2 + l32) * KS + 16 * j + 8 * kh);
-          s[b2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qb[j], s[b2], 0, 0, 0);
+        for (int b2 = 0; b2 < 2; b2++) {
+          const half8_t ak = *reinterpret_cast<const half8_t*>(kbuf + 32 * b2 * AT::ROWB + rk[j]);
+          s[b2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qb[j], j == 0 ? neg_ref : s[b2], 0, 0, 0);
         }
-      }
       if (kt0 + KT - 1 > qlo || (a.window > 0 && kt0 < qhi - a.window + 1)) {
 #pragma unroll
         for (int b2 = 0; b2 < 2; b2++)
@@ -1236,34 +1289,37 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) v
             if (key > qpos || key < qfirst) s[b2][v] = -INFINITY;
           }
       }
-      float mv[16];  // max over the 32 scores as a tree, not a chain
+      float m0 = max3(s[0][0], s[0][1], s[0][2]), m1 = max3(s[1][0], s[1][1], s[1][2]);
 #pragma unroll
-      for (int v = 0; v < 16; v++) mv[v] = fmaxf(s[0][v], s[1][v]);
+      for (int v = 3; v < 15; v += 2) {
+        m0 = max3(m0, s[0][v], s[0][v + 1]);
+        m1 = max3(m1, s[1][v], s[1][v + 1]);
+      }
+      m0 = max3(m0, s[0][15], s[1][15]);
+      m0 = max3(m0, m1, m1);
+      const float mx = __builtin_elementwise_maximum(m0, swap32(m0));
+      const bool first = mrun == -INFINITY, move = mx > kRefSlack || (first && mx > -INFINITY);
+      if (__builtin_amdgcn_ballot_w64(move)) {
+        const float d = move ? mx : 0.f, corr = move && first ? 0.f : __builtin_amdgcn_exp2f(-d);
+        if (move) mrun = (first ? 0.f : mrun) + d;
+        const float nr = mrun == -INFINITY ? 0.f : -mrun;
 #pragma unroll
-      for (int w = 8; w > 0; w >>= 1)
+        for (int v = 0; v < 16; v++) s[0][v] -= d, s[1][v] -= d, neg_ref[v] = nr;
+        lrun *= corr;
 #pragma unroll
-        for (int v = 0; v < w; v++) mv[v] = fmaxf(mv[v], mv[v + w]);
-      float mx = fmaxf(mv[0], swap32(mv[0])) * a.scale_log2;
-      const float mn = fmaxf(mrun, mx);
-      const float mu = mn == -INFINITY ? 0.f : mn;
-      const float corr = __builtin_amdgcn_exp2f(mrun - mu);
-      float ps = 0.f;
+        for (int i = 0; i < NDT; i++) o[i] *= corr;
+      }
+      float ps[2] = {0.f, 0.f};
       uint32_t pk[2][8];
 #pragma unroll
       for (int b2 = 0; b2 < 2; b2++)
 #pragma unroll
         for (int v = 0; v < 16; v += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[b2][v], a.scale_log2, -mu));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[b2][v + 1], a.scale_log2, -mu));
-          ps += p0 + p1;
-          pk[b2][v >> 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+          const auto pr = __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(s[b2][v]), __builtin_amdgcn_exp2f(s[b2][v + 1]));
+          ps[b2] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pr), (half2_t){(_Float16)1.f, (_Float16)1.f}, ps[b2], false);
+          pk[b2][v >> 1] = __builtin_bit_cast(uint32_t, pr);
         }
-      lrun = lrun * corr + ps;
-      mrun = mn;
-      if (__builtin_amdgcn_ballot_w64(corr != 1.f)) {
-#pragma unroll
-        for (int i = 0; i < NDT; i++) o[i] *= corr;
-      }
+      lrun += ps[0] + ps[1];
 #pragma unroll
       for (int b2 = 0; b2 < 2; b2++) {
         const half8_t pb0 = __builtin_bit_cast(half8_t, make_uint4(pk[b2][0], pk[b2][1], pk[b2][2], pk[b2][3]));
@@ -1272,12 +1328,9 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int i = 0; i < NDT; i++) {
           // lane (16 g + j) names V[32 b2 + 4 kh + j / 4 + 8 s][32 i + 16 (g % 2) + 4 (j % 4)]
           // and receives keys 32 b2 + 4 kh + 8 s + 0..3 of dim 32 i + l32
-          const _Float16* vr0 = vbuf + (32 * b2 + 4 * kh + (lane & 15) / 4) * VS + 32 * i + 16 * ((lane >> 4) & 1) +
-                                4 * (lane & 3);
-          const half4_t x0 = lds_read_tr4(vr0);
-          const half4_t x1 = lds_read_tr4(vr0 + 8 * VS);
-          const half4_t x2 = lds_read_tr4(vr0 + 16 * VS);
-          const half4_t x3 = lds_read_tr4(vr0 + 24 * VS);
+          const unsigned char* vr = vbuf + 32 * b2 * AT::ROWB;
+          const half4_t x0 = lds_read_tr4(vr + rv[i][0]), x1 = lds_read_tr4(vr + rv[i][1]);
+          const half4_t x2 = lds_read_tr4(vr + rv[i][2]), x3 = lds_read_tr4(vr + rv[i][3]);
           const half8_t a1 = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
           const half8_t a2 = {x2[0], x2[1], x2[2], x2[3], x3[0], x3[1], x3[2], x3[3]};
           o[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, pb0, o[i], 0, 0, 0);
@@ -1285,8 +1338,7 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) v
         }
       }
     }
-    sg.store(mytile + (buf ^ 1) * NG * AT::TILE_HALVES, t256);
-    __syncthreads();
+    landed();
   }
   lrun += swap32(lrun);
   if (NG > 1) {  // group 1 hands (max, sum, O) to group 0 through LDS (the tiles are free now)
@@ -1327,12 +1379,15 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(2))) v
 bool launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st) {
   // four query heads per block (waves past the group's heads only stage K/V)
   const dim3 grid((a.M + 31) / 32, a.Hkv, (a.G + 3) / 4);
-  if (a.D == 64)
-    hipLaunchKernelGGL((prefill_attn_kernel<64, 2>), grid, dim3(512), 0, st, a);
-  else if (a.D == 128)
-    hipLaunchKernelGGL((prefill_attn_kernel<128, 1>), grid, dim3(256), 0, st, a);
+  if (a.D != 64 && a.D != 128) return false;
+  if (a.D == 64 && a.qkv)
+    hipLaunchKernelGGL((prefill_attn_kernel<64, 2, true>), grid, dim3(512), 0, st, a);
+  else if (a.D == 64)
+    hipLaunchKernelGGL((prefill_attn_kernel<64, 2, false>), grid, dim3(512), 0, st, a);
+  else if (a.qkv)
+    hipLaunchKernelGGL((prefill_attn_kernel<128, 1, true>), grid, dim3(256), 0, st, a);
   else
-    return false;
+    hipLaunchKernelGGL((prefill_attn_kernel<128, 1, false>), grid, dim3(256), 0, st, a);
   return true;
 }
 
