@@ -115,6 +115,7 @@ struct GemvArgs {
   // staged), then clears the key and the count.  Null: greedy_pick_kernel.
   unsigned* arrived;
   int* mctrl;
+  int* token;  // with mctrl null: the token alone goes here (tlm_op_logits)
   // PRO_RMSF input of the persistent schedule: acc_in holds kRep partials of
   // published words (fp32 value in bits 0..31), summed as floats
   int ps_words;
@@ -200,12 +201,9 @@ void launch_rmsnorm(const float* x, const float* w, int n, float eps, int offset
 void launch_silu_mul(const float* g, const float* u, int n, float* out, hipStream_t st);
 void launch_reduce(const float* part, int n_part, int stride, const float* bias, int n, float* y, hipStream_t st);
 void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* token, int blocks, hipStream_t st);
-// second pass of the greedy sampler; `ctrl` receives the token at ctrl[C_TOKEN]
-// ps: the token came from the persistent schedule; advance its token number (C_SEQ)
-void launch_argmax_merge(const float* pval, const int* pidx, int n, int* ctrl, int* tokens_out, int advance,
-                         int max_steps, const EmbStage& es, hipStream_t st, int ps = 0);
-// The merge of an LM head launch that folded into key (greedy_key order),
-// with argmax_merge_kernel's control-word updates; clears key.
+// The merge of an LM head launch that folded into key (greedy_key order):
+// token, position and step of the control words (ps: the token came from the
+// persistent schedule, its token number advances too); clears key.
 void launch_greedy_pick(unsigned long long* key, int* ctrl, int* tokens_out, int advance, int max_steps,
                         const EmbStage& es, hipStream_t st, int ps);
 void launch_set_ctrl(int* ctrl, int token, int pos, int step, int base, int len, const EmbStage& es,

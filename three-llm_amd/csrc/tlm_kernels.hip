@@ -520,16 +520,19 @@ __global__ __launch_bounds__(W * 64) void lm_head_kernel(GemvArgs a) {
           asm volatile("" ::"v"((unsigned)prev), "v"((unsigned)(prev >> 32)) : "memory");
           const unsigned n = __hip_atomic_fetch_add(a.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           if (n == gridDim.x - 1) {
-            int* ctrl = a.mctrl;
-            const int step = ctrl[C_STEP], posv = ctrl[C_POS], seqv = ctrl[C_SEQ];
             const unsigned long long k = __hip_atomic_load(a.arg_key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // nothing above LOWEST (or nothing folded) -> token 0, as the merge
             const int token = k != 0 && greedy_key_value(k) > kLowest ? greedy_key_id(k) : 0;
-            if (a.tokens_out && step >= 0 && step < a.max_steps) a.tokens_out[step] = token;
-            ctrl[C_TOKEN] = token;
-            ctrl[C_POS] = posv + 1;
-            ctrl[C_STEP] = step + 1;
-            ctrl[C_SEQ] = ps_next_seq(seqv);
+            if (int* ctrl = a.mctrl) {
+              const int step = ctrl[C_STEP], posv = ctrl[C_POS], seqv = ctrl[C_SEQ];
+              if (a.tokens_out && step >= 0 && step < a.max_steps) a.tokens_out[step] = token;
+              ctrl[C_TOKEN] = token;
+              ctrl[C_POS] = posv + 1;
+              ctrl[C_STEP] = step + 1;
+              ctrl[C_SEQ] = ps_next_seq(seqv);
+            } else {
+              *a.token = token;
+            }
             __hip_atomic_store(a.arg_key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(a.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
@@ -539,10 +542,6 @@ __global__ __launch_bounds__(W * 64) void lm_head_kernel(GemvArgs a) {
   }
 }
 
-// Second pass of the greedy sampler (createGreedyMergeNode, TSLLogits.ts:250-274):
-// one block reduces the per-block partials; a separate launch, so the kernel
-// boundary (not a device-scope fence per block) publishes the partials.  In the
-// decode graph it also advances the token/position state for the next step.
 // Writes the embedding row of `token`, in fixed point, to replica 0 of es.x0
 // (all threads of the block take part).
 __device__ __forceinline__ void stage_embedding(const EmbStage& es, int token) {
@@ -554,21 +553,13 @@ __device__ __forceinline__ void stage_embedding(const EmbStage& es, int token) {
 
 __device__ __forceinline__ void ps_next_token(int* ctrl) { ctrl[C_SEQ] = ps_next_seq(ctrl[C_SEQ]); }
 
-__global__ __launch_bounds__(1024) void argmax_merge_kernel(const float* pval, const int* pidx, int n, int* ctrl,
-                                                            int* tokens_out, int advance, int max_steps,
-                                                            EmbStage es, int ps) {
+// Second pass of the greedy sampler (createGreedyMergeNode, TSLLogits.ts:250-274):
+// one block reduces the per-block partials; a separate launch, so the kernel
+// boundary (not a device-scope fence per block) publishes the partials.
+__global__ __launch_bounds__(1024) void argmax_merge_kernel(const float* pval, const int* pidx, int n, int* token) {
   __shared__ float sv[16];
   __shared__ int si[16];
-  __shared__ int tok_s;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  // the control words this block updates, requested with the partials (no
-  // other kernel of the step writes them)
-  int step = 0, posv = 0, seqv = 0;
-  if (threadIdx.x == 0) {
-    step = ctrl[C_STEP];
-    posv = ctrl[C_POS];
-    seqv = ctrl[C_SEQ];
-  }
   float bv = kLowest;
   int bi = 0x7fffffff;
   for (int i = threadIdx.x; i < n; i += blockDim.x)
@@ -589,29 +580,13 @@ __global__ __launch_bounds__(1024) void argmax_merge_kernel(const float* pval, c
         bi = si[w];
       }
     // the merge starts from (LOWEST, 0): nothing above LOWEST -> token 0
-    const int token = bv > kLowest ? bi : 0;
-    if (tokens_out && step >= 0 && step < max_steps) tokens_out[step] = token;
-    ctrl[C_TOKEN] = token;
-    if (advance) {
-      ctrl[C_POS] = posv + 1;
-      ctrl[C_STEP] = step + 1;
-    }
-    if (ps) ctrl[C_SEQ] = ps_next_seq(seqv);
-    tok_s = token;
+    *token = bv > kLowest ? bi : 0;
   }
-  __syncthreads();
-  stage_embedding(es, tok_s);
 }
 
-void launch_argmax_merge(const float* pval, const int* pidx, int n, int* ctrl, int* tokens_out, int advance,
-                         int max_steps, const EmbStage& es, hipStream_t st, int ps) {
-  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(1024), 0, st, pval, pidx, n, ctrl, tokens_out, advance,
-                     max_steps, es, ps);
-}
-
-// argmax_merge_kernel's work when the LM head blocks already folded their
-// partials into one key (greedy_key): decode it, advance the control words,
-// clear the key for the next launch.
+// The merge where the LM head's blocks already folded their partials into one
+// key (greedy_key): decode it, advance the control words, clear the key for the
+// next launch.
 __global__ __launch_bounds__(256) void greedy_pick_kernel(unsigned long long* key, int* ctrl, int* tokens_out,
                                                           int advance, int max_steps, EmbStage es, int ps) {
   __shared__ int tok_s;
@@ -1318,7 +1293,7 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float* logits
 
 void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* token, int blocks, hipStream_t st) {
   hipLaunchKernelGGL(argmax_partial_kernel, dim3(blocks), dim3(256), 0, st, logits, n, pval, pidx);
-  launch_argmax_merge(pval, pidx, blocks, token, nullptr, 0, 0, EmbStage{}, st);
+  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(1024), 0, st, pval, pidx, blocks, token);
 }
 
 // ---------------------------------------------------------------- top-k --
