@@ -1,0 +1,41 @@
+"""Batched chunks whose GEMMs pick 128-row tiles with K slices (q4) or the fp16
+ring tiles, at ragged row counts, against the replayed decode graph: an
+independent path with the tolerances of the batched prefill (fp16 activations)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from bridge import close
+import three_llm_amd.runner as R
+import three_llm_amd.tlm as tlm
+import three_llm_amd.weights as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage,n", [(None, 1001), (None, 1901), ("f16", 65), ("f16", 700)])
+def test_ragged_chunks_match_replay(storage, n):
+    print(f"[prefill slices] {storage or 'q4'} linears, {n} rows", flush=True)
+    layers, base = 2, W.WORKLOADS["llama-3.2-1b"]
+    store = base.storage if storage is None else dataclasses.replace(base.storage, linear=storage)
+    cfg = dict(base.config, num_hidden_layers=layers, vocab_size=4096)
+    wl = W.Workload(base.name + "-2l", cfg, store, n + 1, 6, n + 8, qkv_bias=base.qkv_bias)
+    ctx = tlm.Context(0)
+    runner = R.DecoderHIPRunner(W.synthetic(wl), {"maxTokens": n + 8, "prefillChunkSize": 2048}, ctx=ctx)
+    m = runner.model
+    prompt = [int(t) for t in np.random.default_rng(n).integers(0, 4096, n + 1)]
+    res = []
+    for least in (0, 64):  # no batched chunk, then one
+        m.reset_cache()
+        m.set_prefill(least, 2048)
+        m.prefill(prompt, 0, n)
+        m.compute_token(prompt[-1], n, True)
+        res.append((m.read_logits(), [a.view(np.float16).astype(np.float32) for l in range(layers)
+                                      for a in m.kv_read(l, 0, n)]))
+    (ref, ref_kv), (got, got_kv) = res
+    for a, b in zip(got_kv, ref_kv):
+        close(a, b, 2e-2, 1e-2)
+    close(got, ref, 2e-2, 1e-2)
+    runner.close()
+    ctx.close()

@@ -768,28 +768,30 @@ GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part
     // (measured 5-25 % faster from 64 to 1100 rows)
     const int tiles = ((N + 255) / 256) * ((M + 127) / 128);
     if (M > 64 && tiles >= cus / 2) s.tile = GT_128x256;
-    const int kdiv = s.tile == GT_KW ? 4 : 1, min_steps = s.tile == GT_KW ? 2 : 4;
-    if (epi == GEMM_PART && s.tile != GT_KW) {
-      // two blocks per CU: pick the split count with the least
-      // (rounds of blocks x steps per block) + the split slices' write and read
-      // (M N 8 bytes each at ~6 TB/s, in units of a ~1 us step), the latter
-      // weighted 2x: the slice stores compete with the GEMM's own operand reads
-      // (measured 1-2 % faster 2048-row chunks than at weight 1, none slower)
-      const double slice_steps = 2.0 * (double)M * N * 8.0 / 6e6;
-      double best = 1e30;
-      for (int sp = 1; sp <= 32 && steps / sp >= min_steps; sp *= 2) {
-        const int rounds = (tiles * sp + 2 * cus - 1) / (2 * cus);
-        const double cost = (double)rounds * ((steps + sp - 1) / sp) + sp * slice_steps;
-        if (cost < best) best = cost, splits = sp;
+    if (epi == GEMM_PART && M > 64) {
+      // sums in slices keep the CUs busy with 128-row tiles too: the cheaper of
+      // the two.  128 tiles of K 8192 (2048 rows, the Llama-3.2-1B down
+      // projection) go in 2 slices, one block per CU, and not in 4, two per CU,
+      // whose slices cost more than the shared CU gains.  Prompts of the
+      // Llama-3.2-1B shape, against whole rounds of two blocks per CU and the
+      // rule above: 1000 ids 4066 -> 3765 us, 1900 6664 -> 5736, 4096 12216 -> 11888
+      const float whole = gemm_cost(kCostQ4[0], M, N, steps, 1, cus);
+      float best = INFINITY;
+      for (int sp = 1; sp <= 32 && steps / sp >= 4; sp *= 2) {
+        const float c = gemm_cost(kCostQ4[1], M, N, steps, sp, cus);
+        if (c < best) best = c, splits = sp;
       }
-    } else if (epi == GEMM_PART) {
+      s.tile = best < whole ? GT_128x256 : GT_KW;
+    }
+    if (epi == GEMM_PART && s.tile == GT_KW) {
       // split K while the grid stays within about g_split_waves waves per CU:
       // past one round of blocks a CU streams the same bytes either way and each
       // split only adds a slice for the next row kernel to fold (Qwen2.5-0.5B
       // shape, 64 to 300 rows: the down GEMM in 4 splits instead of 8, the chunk
       // 3-6 % faster)
       const int target = g_split_waves * cus, waves = 4 * ((N + kTile - 1) / kTile) * ((M + 31) / 32);
-      while (splits < 32 && waves * splits * 2 <= target && steps / (2 * splits * kdiv) >= min_steps) splits *= 2;
+      splits = 1;
+      while (splits < 32 && waves * splits * 2 <= target && steps / (2 * splits * 4) >= 2) splits *= 2;
     }
   } else {
     const GemmCost* tab = fmt == WF_Q4 ? kCostQ4 : kCostF16;
