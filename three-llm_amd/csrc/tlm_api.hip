@@ -87,6 +87,7 @@ struct tlm_ctx {
   // tlm_op_logits: the blocks' folded best and their count (zero between launches)
   unsigned long long* arg_key = nullptr;
   unsigned* arg_arrived = nullptr;
+  unsigned* topk_arrived = nullptr;  // tlm_op_topk's blocks done (zero between launches)
   // top-k levels: two levels of kTopkWork (score, id) pairs
   float* topk_v = nullptr;
   int* topk_i = nullptr;
@@ -96,6 +97,10 @@ struct tlm_ctx {
 };
 constexpr size_t kPartFloats = (size_t)8 << 20;  // 32 MiB
 constexpr size_t kTopkWork = 32768;
+// the keys share the first level's ids: a call uses one or the other
+static TopkWork topk_work(tlm_ctx* c) {
+  return TopkWork{c->topk_v, c->topk_i, kTopkWork, reinterpret_cast<unsigned long long*>(c->topk_i), c->topk_arrived};
+}
 
 struct GemvPlan {
   int waves = 4, cps = 1, splits = 1, gx = 1;
@@ -507,6 +512,8 @@ int tlm_open(int device, tlm_ctx** out) {
   if (e == hipSuccess) e = hipMalloc(&c->part, kPartFloats * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&c->arg_key, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMalloc(&c->arg_arrived, sizeof(unsigned));
+  if (e == hipSuccess) e = hipMalloc(&c->topk_arrived, sizeof(unsigned));
+  if (e == hipSuccess) e = hipMemset(c->topk_arrived, 0, sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(c->arg_key, 0, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(c->arg_arrived, 0, sizeof(unsigned));
   if (e == hipSuccess) e = hipDeviceSynchronize();  // the fills are on another stream than the context's
@@ -533,6 +540,7 @@ void tlm_close(tlm_ctx* ctx) {
   hipFree(ctx->part);
   hipFree(ctx->arg_key);
   hipFree(ctx->arg_arrived);
+  hipFree(ctx->topk_arrived);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -1137,8 +1145,7 @@ int tlm_op_topk(tlm_ctx* ctx, const float* logits, int n, int k, double softcap,
   if (!ctx || !logits || !tokens || !scores || n <= 0) return fail(TLM_ERR_INVALID, "TLMLogitSampler: invalid argument");
   if (k < 1 || k > kTopkMax)
     return fail(TLM_ERR_INVALID, "TLMLogitSampler: candidate count %d outside [1, %d]", k, kTopkMax);
-  if (!launch_topk(logits, n, k, (float)(softcap > 0 ? softcap : 0), ctx->topk_v, ctx->topk_i, kTopkWork, scores,
-                   tokens, ctx->stream))
+  if (!launch_topk(logits, n, k, (float)(softcap > 0 ? softcap : 0), topk_work(ctx), scores, tokens, ctx->stream))
     return fail(TLM_ERR_INVALID, "TLMLogitSampler: %d logits exceed the candidate workspace", n);
   CHECK_LAUNCH("TLMLogitSampler");
   return TLM_OK;
@@ -2636,8 +2643,7 @@ int tlm_time_kernel(tlm_model* m, int which, int iters, double* avg_ms) {
   HIP_TRY(hipEventCreate(&e1));
   auto one = [&]() {
     if (which == 6)  // top-8 candidates over the logits
-      return launch_topk(m->logits, m->d.vocab_size, 8, 0.f, m->ctx->topk_v, m->ctx->topk_i, kTopkWork, m->cand_v,
-                         m->cand_i, st);
+      return launch_topk(m->logits, m->d.vocab_size, 8, 0.f, topk_work(m->ctx), m->cand_v, m->cand_i, st);
     return which == 0 ? enqueue_head(m, st, false)
                       : enqueue_layer(m, 0, st, which, long_window(&m->attn, m->host_pos));
   };

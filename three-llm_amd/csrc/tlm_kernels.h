@@ -222,8 +222,15 @@ int attn_lpp(int D, bool kv_f32);
 // top-k candidates (k <= kTopkMax) of an fp32 vector in the greedy order; the
 // workspace holds two levels of wcap (score, id) pairs each
 constexpr int kTopkMax = 16;
-bool launch_topk(const float* logits, int n, int k, float softcap, float* wv, int* wi, size_t wcap, float* out_v,
-                 int* out_i, hipStream_t st);
+struct TopkWork {
+  float* v;                  // two levels of cap (score, id) pairs
+  int* i;
+  size_t cap;
+  unsigned long long* keys;  // the one-launch selection: the blocks' keys (kTopkSlice of them at most)
+  unsigned* arrived;         // and their count (zero between launches)
+};
+bool launch_topk(const float* logits, int n, int k, float softcap, const TopkWork& w, float* out_v, int* out_i,
+                 hipStream_t st);
 
 // --------------------------------------------- persistent per-token schedule --
 // One launch computes every layer of one token on one 1024-thread block per

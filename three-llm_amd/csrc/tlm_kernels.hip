@@ -1310,9 +1310,9 @@ void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* toke
 // k best, nor one below the largest such bound of the four waves.  The few keys
 // that remain (k to about 2 k of random scores; at most 32 k per wave) go to
 // LDS, and each one's rank is the number of larger ones.  All keys differ, so
-// ranks do too and the result does not depend on the order in LDS.  Levels of
-// blocks until one remains.  151936 scores, k = 8 (two levels): 16.5 us with k
-// passes per wave and k for the merge, 7.7 us so.
+// ranks do too and the result does not depend on the order in LDS.  151936
+// scores, k = 8: 16.5 us with k passes per wave and k for the merge, 7.5 us so
+// in two levels of blocks.
 constexpr int kTopkPer = 8;
 constexpr int kTopkSlice = 256 * kTopkPer;
 
@@ -1337,35 +1337,21 @@ __device__ __forceinline__ void max_u64_step(uint32_t& lo, uint32_t& hi) {
     hi = ohi;
   }
 }
-// IDS: the entries are (vals[e], ids[e]) (a merge level) instead of (vals[e], e).
-template <bool IDS>
-__global__ __launch_bounds__(256) void topk_select_kernel(const float* __restrict__ vals, const int* __restrict__ ids,
-                                                          int n, int k, float softcap, float* out_v, int* out_i) {
-  __shared__ unsigned long long cand[kTopkSlice];
-  __shared__ unsigned long long bound[4];
-  __shared__ int count;
+struct TopkShared {
+  unsigned long long cand[kTopkSlice];
+  unsigned long long bound[4];
+  int count;
+};
+
+// The k best of a block's keys (kTopkPer per thread, 0: none): put(rank, key),
+// and put(slot, 0) for the slots past the last candidate.
+template <class Put>
+__device__ __forceinline__ void topk_pick(const unsigned long long (&key)[kTopkPer], int k, TopkShared& sh, Put put) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const size_t base = (size_t)blockIdx.x * kTopkSlice + wave * 64 * kTopkPer;
-  // every load issued before the first use (clamped indices: no branches)
-  float x[kTopkPer];
-  int xi[kTopkPer];
+  if (tid == 0) sh.count = 0;
+  unsigned long long top = 0;
 #pragma unroll
-  for (int u = 0; u < kTopkPer; u++) x[u] = vals[min(base + lane + 64 * u, (size_t)n - 1)];
-#pragma unroll
-  for (int u = 0; u < kTopkPer; u++)
-    xi[u] = IDS ? ids[min(base + lane + 64 * u, (size_t)n - 1)] : (int)(base + lane + 64 * u);
-  if (tid == 0) count = 0;
-  if (softcap > 0.f) {
-#pragma unroll
-    for (int u = 0; u < kTopkPer; u++) x[u] = softcap * tanhf(x[u] / softcap);
-  }
-  unsigned long long key[kTopkPer], top = 0;
-#pragma unroll
-  for (int u = 0; u < kTopkPer; u++) {
-    const bool ok = base + lane + 64 * u < (size_t)n && x[u] > kLowest;  // LOWEST, -inf, NaN: never a candidate
-    key[u] = ok ? topk_key(x[u], xi[u]) : 0ull;
-    top = key[u] > top ? key[u] : top;
-  }
+  for (int u = 0; u < kTopkPer; u++) top = key[u] > top ? key[u] : top;
   // the wave's bound: the k-th largest quad maximum (0 while fewer quads hold a candidate)
   static_assert(kTopkMax <= 16, "one of a wave's 16 quads for each of the k best");
   uint32_t lo = (uint32_t)top, hi = (uint32_t)(top >> 32);
@@ -1387,41 +1373,115 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const float* __restric
   } else {
     top = 0;
   }
-  if (lane == 0) bound[wave] = top;
+  if (lane == 0) sh.bound[wave] = top;
   __syncthreads();
-  unsigned long long b = bound[0];
+  unsigned long long b = sh.bound[0];
 #pragma unroll
-  for (int w = 1; w < 4; w++) b = bound[w] > b ? bound[w] : b;
+  for (int w = 1; w < 4; w++) b = sh.bound[w] > b ? sh.bound[w] : b;
 #pragma unroll
   for (int u = 0; u < kTopkPer; u++)
-    if (key[u] != 0 && key[u] >= b) cand[atomicAdd(&count, 1)] = key[u];
+    if (key[u] != 0 && key[u] >= b) sh.cand[atomicAdd(&sh.count, 1)] = key[u];
   __syncthreads();
-  const int m = count;
+  const int m = sh.count;
   for (int i = tid; i < m; i += 256) {
-    const unsigned long long mine = cand[i];
+    const unsigned long long mine = sh.cand[i];
     int rank = 0;
-    for (int j = 0; j < m; j++) rank += cand[j] > mine ? 1 : 0;
-    if (rank < k) {
-      out_v[(size_t)blockIdx.x * k + rank] = topk_score(mine);
-      out_i[(size_t)blockIdx.x * k + rank] = (int)~(uint32_t)mine;
-    }
+    for (int j = 0; j < m; j++) rank += sh.cand[j] > mine ? 1 : 0;
+    if (rank < k) put(rank, mine);
   }
-  if (tid >= m && tid < k) {  // fewer candidates than slots
-    out_v[(size_t)blockIdx.x * k + tid] = kLowest;
-    out_i[(size_t)blockIdx.x * k + tid] = 0;
+  if (tid >= m && tid < k) put(tid, 0ull);  // fewer candidates than slots
+}
+
+// IDS: the entries are (vals[e], ids[e]) (a merge level) instead of (vals[e], e).
+template <bool IDS>
+__device__ __forceinline__ void topk_keys(const float* __restrict__ vals, const int* __restrict__ ids, int n,
+                                          float softcap, unsigned long long (&key)[kTopkPer]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t base = (size_t)blockIdx.x * kTopkSlice + wave * 64 * kTopkPer;
+  // every load issued before the first use (clamped indices: no branches)
+  float x[kTopkPer];
+  int xi[kTopkPer];
+#pragma unroll
+  for (int u = 0; u < kTopkPer; u++) x[u] = vals[min(base + lane + 64 * u, (size_t)n - 1)];
+#pragma unroll
+  for (int u = 0; u < kTopkPer; u++)
+    xi[u] = IDS ? ids[min(base + lane + 64 * u, (size_t)n - 1)] : (int)(base + lane + 64 * u);
+  if (softcap > 0.f) {
+#pragma unroll
+    for (int u = 0; u < kTopkPer; u++) x[u] = softcap * tanhf(x[u] / softcap);
+  }
+#pragma unroll
+  for (int u = 0; u < kTopkPer; u++) {
+    const bool ok = base + lane + 64 * u < (size_t)n && x[u] > kLowest;  // LOWEST, -inf, NaN: never a candidate
+    key[u] = ok ? topk_key(x[u], xi[u]) : 0ull;
   }
 }
 
-bool launch_topk(const float* logits, int n, int k, float softcap, float* wv, int* wi, size_t wcap, float* out_v,
-                 int* out_i, hipStream_t st) {
+__device__ __forceinline__ void topk_store(float* out_v, int* out_i, int at, unsigned long long key) {
+  out_v[at] = key ? topk_score(key) : kLowest;
+  out_i[at] = key ? (int)~(uint32_t)key : 0;
+}
+
+// One level of many: each block writes its k best.
+template <bool IDS>
+__global__ __launch_bounds__(256) void topk_select_kernel(const float* __restrict__ vals, const int* __restrict__ ids,
+                                                          int n, int k, float softcap, float* out_v, int* out_i) {
+  __shared__ TopkShared sh;
+  unsigned long long key[kTopkPer];
+  topk_keys<IDS>(vals, ids, n, softcap, key);
+  topk_pick(key, k, sh, [&](int r, unsigned long long v) { topk_store(out_v, out_i, blockIdx.x * k + r, v); });
+}
+
+// The whole selection in one launch, where the blocks' k best together fit one
+// block: each block publishes its keys past its XCD's L2 and counts itself once
+// they are performed; the block that counts last selects from all of them and
+// clears the count.  No block waits.  151936 scores, k = 8: 7.5 us with the
+// merge as a launch of its own, 7.0 us so.
+__global__ __launch_bounds__(256) void topk_one_kernel(const float* __restrict__ vals, int n, int k, float softcap,
+                                                       unsigned long long* keys, unsigned* arrived, float* out_v,
+                                                       int* out_i) {
+  __shared__ TopkShared sh;
+  __shared__ unsigned before;
+  unsigned long long key[kTopkPer];
+  topk_keys<false>(vals, nullptr, n, softcap, key);
+  if (gridDim.x == 1) {
+    topk_pick(key, k, sh, [&](int r, unsigned long long v) { topk_store(out_v, out_i, r, v); });
+    return;
+  }
+  topk_pick(key, k, sh, [&](int r, unsigned long long v) {
+    __hip_atomic_store(keys + blockIdx.x * k + r, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's keys are performed
+  __syncthreads();                                  // and every wave's
+  if (threadIdx.x == 0)
+    before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (before != gridDim.x - 1) return;
+  const int total = gridDim.x * k;
+#pragma unroll
+  for (int u = 0; u < kTopkPer; u++) {
+    const int i = threadIdx.x + 256 * u;
+    key[u] = i < total ? __hip_atomic_load(keys + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+  }
+  if (threadIdx.x == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  topk_pick(key, k, sh, [&](int r, unsigned long long v) { topk_store(out_v, out_i, r, v); });
+}
+
+bool launch_topk(const float* logits, int n, int k, float softcap, const TopkWork& w, float* out_v, int* out_i,
+                 hipStream_t st) {
   if (n <= 0 || k <= 0 || k > kTopkMax) return false;
   int blocks = (n + kTopkSlice - 1) / kTopkSlice;
-  if ((size_t)blocks * k > wcap) return false;
+  if ((size_t)blocks * k > w.cap) return false;
+  if (blocks * k <= kTopkSlice) {
+    hipLaunchKernelGGL(topk_one_kernel, dim3(blocks), dim3(256), 0, st, logits, n, k, softcap, w.keys, w.arrived, out_v,
+                       out_i);
+    return true;
+  }
   const float* v = logits;
   const int* ids = nullptr;
   float cap = softcap;
-  float* bufv[2] = {wv, wv + wcap};
-  int* bufi[2] = {wi, wi + wcap};
+  float* bufv[2] = {w.v, w.v + w.cap};
+  int* bufi[2] = {w.i, w.i + w.cap};
   for (int level = 0;; level++) {
     const bool last = blocks == 1;
     float* ov = last ? out_v : bufv[level & 1];
