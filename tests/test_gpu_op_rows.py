@@ -37,7 +37,9 @@ def make_linear(ctx, fmt, w):
     # 128 x 128 tiles, whole and in slices
     (tlm.FMT_F16, 1030, 4100, 1024, True), (tlm.FMT_F16, 512, 2048, 4096, False), (tlm.FMT_F16, 700, 10000, 320, True),
     # 256 x 256 tiles: rows and columns past the last whole one, an odd step count
-    (tlm.FMT_F16, 513, 15000, 608, True),
+    (tlm.FMT_F16, 900, 12300, 608, True),
+    # 128 x 256 tiles (q4), whole and in slices
+    (tlm.FMT_Q4, 900, 8200, 256, True), (tlm.FMT_Q4, 257, 4100, 6048, False),
 ])
 def test_rows_at_tile_edges(ctx, fmt, M, N, K, bias):
     print(f"[rows] fmt {fmt}, {M} x {N} x {K}", flush=True)

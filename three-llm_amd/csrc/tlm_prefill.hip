@@ -724,35 +724,41 @@ static const int g_split_waves = [] {
   return v > 0 && v <= 64 ? v : 4;
 }();
 
-// What a GEMM takes, in us: fitted to 120 shapes drawn over 1-2048 rows,
-// 256-16384 columns and K 256-8192, each timed on every tile with 1-32 splits
-// (the fit is within 6-18 % rms, and the tile and split count it picks take
-// 2 % longer than the best ones in the mean, 31 % at most).
+// What a GEMM takes, in us: fitted to 240 shapes over 1-2048 rows, 256-16384
+// columns and K 256-8192, each timed on every tile with 1-32 splits (the fit is
+// within 6-19 % rms; the tile and split count it picks take 0.5 % (q4) and 0.7 %
+// (fp16) longer than the best ones in the mean, 28 % at most).
 struct GemmCost {
   int tile;
   float base;        // the launch and the first operands
   float one, two;    // a 32-k step of one block on a CU; of the two that share it (0: one fits).
                      // GT_KW: a step of a block's waves alone on a CU; per block of a shared CU
   float slice, out;  // 1e6 floats of slices, written and folded; of a result stored unsplit
+  float edge;        // a block's start and end, in steps
 };
-static const GemmCost kCostQ4[] = {{GT_KW, 3.7f, 0.15f, 0.22f, 2.6f, 1.6f}, {GT_128x256, 7.7f, 0.37f, 0.67f, 2.1f, 3.0f}};
-static const GemmCost kCostF16[] = {{GT_KW, 3.1f, 0.25f, 0.255f, 4.2f, 3.0f},
-                                    {GT_128x128, 5.6f, 0.19f, 0.40f, 2.6f, 3.0f},
-                                    {GT_256x256, 8.0f, 0.55f, 0.f, 2.0f, 2.7f}};
-constexpr float kFoldLaunch = 2.f;  // us: the second kernel, where the caller folds the slices itself
+static const GemmCost kCostQ4[] = {{GT_KW, 3.6f, 0.19f, 0.23f, 2.4f, 1.5f, 0.2f},
+                                   {GT_128x256, 4.2f, 0.38f, 0.50f, 2.0f, 2.5f, 9.6f}};
+static const GemmCost kCostF16[] = {{GT_KW, 2.9f, 0.27f, 0.31f, 3.1f, 2.7f, 0.f},
+                                    {GT_128x128, 5.5f, 0.22f, 0.43f, 2.2f, 1.8f, 0.f},
+                                    {GT_256x256, 2.0f, 0.56f, 0.f, 1.8f, 1.8f, 11.f}};
+constexpr float kFoldLaunch = 2.6f;  // us: the second kernel, where the caller folds the slices itself
 
+// INFINITY where the tile is not to be taken: GT_KW where 128 x 256 tiles alone
+// give each CU a block, and its slices where its tiles do (more blocks of a
+// full chip only move more bytes; the fit has no such cases).
 static float gemm_cost(const GemmCost& c, int M, int N, int steps, int splits, int cus) {
   const int bm = gemm_tile_rows(c.tile), bn = gemm_tile_cols(c.tile), spc = (steps + splits - 1) / splits;
-  const long blocks = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits;
-  const float mn = (float)M * N * 1e-6f, edge = c.base + (splits > 1 ? splits * c.slice : c.out) * mn;
+  const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn), blocks = tiles * splits;
+  const float mn = (float)M * N * 1e-6f, fixed = c.base + (splits > 1 ? splits * c.slice : c.out) * mn;
   if (c.tile == GT_KW) {
-    const int w = (spc + 3) / 4;
+    if (M > 64 && (long)((M + 127) / 128) * ((N + 255) / 256) >= cus) return INFINITY;
+    if (splits > 1 && tiles >= cus) return INFINITY;
     const float per_cu = blocks <= 4L * cus ? (float)((blocks + cus - 1) / cus) : (float)blocks / cus;
-    return edge + w * fmaxf(c.one, c.two * per_cu);
+    return fixed + ((spc + 3) / 4 + c.edge) * fmaxf(c.one, c.two * per_cu);
   }
   const long slots = c.two > 0.f ? 2 * cus : cus, rem = blocks % slots;
   const float full = c.two > 0.f ? c.two : c.one;
-  return edge + spc * (full * (blocks / slots) + (rem == 0 ? 0.f : rem <= cus ? c.one : c.two));
+  return fixed + (spc + c.edge) * (full * (blocks / slots) + (rem == 0 ? 0.f : rem <= cus ? c.one : c.two));
 }
 
 GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part) {
