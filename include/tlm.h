@@ -132,7 +132,6 @@ int tlm_op_attention(tlm_attn* attn, const float* qkv, int position, float* out)
  * device [rows][(heads + 2 kv_heads) * head_dim], bias included; RoPE, the K/V
  * rows appended to the cache, causal attention of each row over
  * [max(0, pos - W + 1), pos] on MFMA; out: fp16 bits device [rows][heads * head_dim].
- * The queries enter as fp16, already times the softmax scale and log2 e.
  * Needs an fp16 cache and head_dim 64 or 128.  Waits for the stream. */
 int tlm_op_attention_rows(tlm_attn* attn, const float* qkv, int32_t rows, int32_t position0, uint16_t* out);
 /* Allocation-free tlm_op_attention_rows.  No counterpart in the reference: it

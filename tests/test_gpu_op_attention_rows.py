@@ -4,7 +4,7 @@ with nothing to see in a tile, and the two ways the queries reach the kernel.
 
 No rotation (frequencies of zero) and queries and keys on a coarse grid make
 every score exact in fp32; what is left is fp16 probabilities (2^-10 each,
-rounded toward zero) and the fp16 output, so 2e-3 bounds the error of a
+rounded to nearest) and the fp16 output, so 2e-3 bounds the error of a
 weighted mean of values of unit scale."""
 import math
 
@@ -86,3 +86,30 @@ def test_rows_written_over_their_projections_equal_rows_apart(ctx, D):
     # RoPE of the staged queries may be contracted differently: one fp16 step of a query
     a, b = (o.view(np.float16).astype(np.float64) for o in outs)
     assert np.abs(a - b).max() <= 2e-3 * np.abs(a).max()
+
+
+@pytest.mark.parametrize("scale,q0,unit,dims", [(2.0 ** -24, 1.5, 2.0 ** 12, None), (2.0, 49984.0, 2.0 ** -14, 1)])
+@pytest.mark.parametrize("rotary", [True, False])
+@pytest.mark.parametrize("D", [64, 128])
+def test_queries_round_before_the_softmax_scale(ctx, D, rotary, scale, q0, unit, dims):
+    """The scale multiplies fp32 scores: query values that fp16 holds exactly keep
+    every bit where query * scale is subnormal in fp16 (1.5 steps: 2 once rounded)
+    or past its largest value."""
+    print(f"[attention rows] D {D}, scale {scale}, queries {q0}", flush=True)
+    rng = np.random.default_rng(D)
+    n = 97
+    c = rng.integers(-8, 9, (n, 1, 1)).astype(np.float64)
+    q, k = np.zeros((n, 2, D)), np.zeros((n, 1, D))
+    q[:, :, :dims], k[:, :, :dims] = q0, c * unit
+    v = (c / 8 + 0.1 * rng.standard_normal((n, 1, D))).astype(np.float16)
+    x = np.concatenate([t.reshape(n, -1) for t in (q, k, v)], 1).astype(np.float32)
+    # without rotary dims the queries are staged, with frequencies of zero formed in the kernel
+    A = tlm.Attention(ctx, 2, 1, D, n, np.zeros(D // 2, np.float32) if rotary else None, rotary_dim=None if rotary else 0,
+                      attn_scale=scale * math.log(2.0))
+    got = A.rows(ctx.array(x), n, 0, ctx.buffer(2 * n * 2 * D)).read(np.uint16)
+    A.close()
+    got = got.view(np.float16).astype(np.float64).reshape(n, 2 * D)
+    x64 = x.astype(np.float64)
+    x64[:, :2 * D] *= scale
+    ref = expected(x64, 0, 2, 1, D, 0)
+    assert np.abs(got - ref).max() <= 2e-3 * max(1.0, np.abs(ref).max())

@@ -966,7 +966,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
                                    uint16_t* q) {
   const tlm_attn_desc& d = A->d;
   hipStream_t st = A->ctx->stream;
-  const float qscale = A->scale * 1.4426950408889634f;  // log2 e: the softmax runs in base 2
   RopeKvArgs r;
   memset(&r, 0, sizeof r);
   r.qkv = qkv;
@@ -983,7 +982,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   r.rope_cos = A->rope_cos;
   r.rope_sin = A->rope_sin;
   r.q = q;
-  r.qscale = qscale;
   r.kc = A->kc;
   r.vc = A->vc;
   launch_rope_kv(r, st);
@@ -994,7 +992,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
     pa.qkv = qkv;
     pa.rope_cos = A->rope_cos;
     pa.rope_sin = A->rope_sin;
-    pa.qscale = qscale;
   }
   pa.kc = A->kc;
   pa.vc = A->vc;
@@ -1007,6 +1004,7 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   pa.G = A->G;
   pa.max_tokens = d.max_tokens;
   pa.window = d.sliding_window;
+  pa.scale_log2 = A->scale * 1.4426950408889634f;  // log2 e: the softmax runs in base 2
   return launch_prefill_attention(pa, st);
 }
 
@@ -1968,7 +1966,6 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
   const int H = d.hidden_size, I = d.intermediate_size, D = d.head_dim;
   const int lf = wfmt(d.linear_fmt);
   const size_t rowsH = (size_t)M * H;
-  const float qscale = m->attn.scale * 1.4426950408889634f;  // log2 e: the softmax runs in base 2
   // per layer: two row kernels (one when the O GEMM folds its rows; layer 0's
   // first one also gathers the embedding rows), the QKV GEMM (+ rope_kv unless
   // RoPE runs in its epilogue), attention and three GEMMs; then the last fold
@@ -1994,7 +1991,6 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
       g.rope_cos = m->attn.rope_cos;
       g.rope_sin = m->attn.rope_sin;
       g.ctrl = m->ctrl;
-      g.qscale = qscale;
       g.Hq = d.num_heads;
       g.Hkv = d.num_kv_heads;
       g.max_tokens = d.max_tokens;
@@ -2021,7 +2017,6 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
       r.rope_cos = m->attn.rope_cos;
       r.rope_sin = m->attn.rope_sin;
       r.q = m->pf_q;
-      r.qscale = qscale;
       r.kc = L.kc;
       r.vc = L.vc;
       r.kv_f32 = 0;
@@ -2042,6 +2037,7 @@ static int prefill_enqueue(tlm_model* m, const PfPlan& pp, int M, hipStream_t st
     pa.G = m->attn.G;
     pa.max_tokens = d.max_tokens;
     pa.window = m->windows[l];
+    pa.scale_log2 = m->attn.scale * 1.4426950408889634f;
     ok = ok && launch_prefill_attention(pa, st);
     g = gemm_args(L.o, m->pf_att, m->QS, M);
     g.ldc = H;

@@ -377,7 +377,6 @@ struct GemmArgs {
   const float* rope_cos;  // [max_tokens][32], attention factor folded in
   const float* rope_sin;
   int p0, Hq, Hkv, max_tokens;
-  float qscale;        // softmax scale * log2(e), applied to q
   uint16_t* kc;        // fp16 [Hkv][max_tokens][64] (this layer)
   uint16_t* vc;
   int* ovf;            // set to 1 when an fp16 output (h, q, k, v) is not finite; may be null
@@ -427,17 +426,17 @@ struct RowsArgs {
   const int* ctrl;
 };
 struct PrefillAttnArgs {
-  const uint16_t* q;    // fp16 [M][Hq D], RoPE applied, times softmax scale * log2(e)
+  const uint16_t* q;    // fp16 [M][Hq D], RoPE applied
   // non-null qkv (full rotary; out apart from it): the queries come from the
-  // fp32 projected rows [M][(Hq + 2 Hkv) D] instead, rotated and scaled in the kernel
+  // fp32 projected rows [M][(Hq + 2 Hkv) D] instead, rotated in the kernel
   const float* qkv;
   const float* rope_cos;  // [max_tokens][D / 2]
   const float* rope_sin;
-  float qscale;
   const void* kc;       // fp16 [Hkv][max_tokens][D] (this layer)
   const void* vc;
   uint16_t* out;        // fp16 [M][Hq D]
   int M, p0, Hq, Hkv, D, G, max_tokens, window;
+  float scale_log2;     // softmax scale * log2(e)
   const int* ctrl;      // non-null: the first row's position is ctrl[C_POS] instead of p0
 };
 struct RopeKvArgs {
@@ -449,8 +448,7 @@ struct RopeKvArgs {
   int h0;               // first head of a row taken (q heads, then k, then v): Hq leaves the queries alone
   const float* rope_cos;  // [max_tokens][rd / 2]
   const float* rope_sin;
-  uint16_t* q;          // fp16 [M][Hq D], times qscale
-  float qscale;         // softmax scale * log2(e)
+  uint16_t* q;          // fp16 [M][Hq D]
   void* kc;             // [Hkv][max_tokens][D]
   void* vc;
   int kv_f32;

@@ -664,8 +664,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         if (kind == 0) {
           uint16_t* qr = g.Ch + (size_t)row * g.ldc + t0 * kTile;
-          qr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0 * g.qscale));
-          qr[d + 32] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y1 * g.qscale));
+          qr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0));
+          qr[d + 32] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y1));
         } else {
           uint16_t* cr = (kind == 1 ? g.kc : g.vc) + ((size_t)hk * g.max_tokens + pos) * kTile;
           cr[d] = __builtin_bit_cast(uint16_t, f16_guard(g.ovf, y0));
@@ -964,7 +964,7 @@ __device__ __forceinline__ float fold_slices(const float* row, const float* bias
 __device__ __forceinline__ void rope_store(const RopeKvArgs& a, int m, int pos, int i, float y) {
   const int nq = a.Hq * a.D, nk = a.Hkv * a.D;
   if (i < nq) {
-    a.q[(size_t)m * nq + i] = __builtin_bit_cast(uint16_t, f16_guard(a.ovf, y * a.qscale));
+    a.q[(size_t)m * nq + i] = __builtin_bit_cast(uint16_t, f16_guard(a.ovf, y));
     return;
   }
   const bool isv = i >= nq + nk;
@@ -1046,7 +1046,6 @@ __device__ __forceinline__ float4 fold_slices4(const float* row, const float* bi
 
 __device__ __forceinline__ void rope_store4(const RopeKvArgs& a, int m, int pos, int i, float4 y) {
   const int nq = a.Hq * a.D, nk = a.Hkv * a.D;
-  if (i < nq) y.x *= a.qscale, y.y *= a.qscale, y.z *= a.qscale, y.w *= a.qscale;
   const half4_t h = {f16_guard(a.ovf, y.x), f16_guard(a.ovf, y.y), f16_guard(a.ovf, y.z), f16_guard(a.ovf, y.w)};
   uint16_t* dst;
   if (i < nq) {
@@ -1125,15 +1124,18 @@ void launch_rope_kv(const RopeKvArgs& a, hipStream_t st) {
 // then O^T += V^T P^T with P^T taken straight from the S^T registers: the key
 // order of the contraction is permuted to match that register layout.
 // The vector ALU's share per score bounds it (a tile's 32 scores a lane
-// against 16 MFMAs), so that is kept to an exponential, half a max3, half a
-// conversion and half a dot product: the queries carry scale * log2 e, the
-// score accumulators start at minus the softmax's reference, the reference
-// moves only when a score passes it by kRefSlack (O is rescaled then; fp16 P
-// stays below 2^9), and the sum adds the pairs of P as the matrix cores see
-// them, rounded toward zero to fp16.  2048 rows of the Llama-3.2-1B heads: 38
-// -> 30 us from position 0, 90 -> 66 us from 2048, of which the copies that
-// stay in flight across the math (register staging was sunk below it) gave
-// about 8; four waves per SIMD need <= 128 registers, hence the copies.
+// against 16 MFMAs), so that is kept to an fma, an exponential, half a max3, an
+// addition and half a conversion: the softmax's reference moves only when a
+// score passes it by kRefSlack (O is rescaled then; fp16 P stays below 2^9).
+// Queries are fp16 as rotated and the scale multiplies the fp32 scores: scaled
+// before the rounding they would run into fp16's subnormals or past its largest
+// value sooner.  P is rounded to nearest for the product with V, and its sum
+// adds the 32-bit values: 3.0e-4 from 64 bits at 2048 rows, 3.4e-4 with both from
+// P rounded toward zero and the queries scaled first, at the same speed (36.8
+// and 36.9 us).  rocprofv3, 2048 rows, registers staging the tiles and O
+// rescaled with every new maximum against this: Llama-3.2-1B heads 39.0 -> 36.8
+// us from position 0, 88.0 -> 75.2 from 2048; Llama-3.2-3B heads 67.4 -> 54.5.
+// Four waves per SIMD need <= 128 registers, hence the copies.
 template <int DT>
 struct AttnTile {
   static constexpr int KT = 64;             // keys per tile
@@ -1171,7 +1173,7 @@ __device__ __forceinline__ half4_t lds_read_tr4(const unsigned char* p) {
 __device__ __forceinline__ float max3(float a, float b, float c) {
   return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
-// A score may exceed the reference by this much (log2) before it moves
+// A score may exceed the softmax's reference by this much (log2) before it moves
 constexpr float kRefSlack = 8.f;
 
 template <int DT, int NG, bool QF>
@@ -1214,10 +1216,10 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
         const float4 u = *reinterpret_cast<const float4*>(x + d), v = *reinterpret_cast<const float4*>(x + d + DT / 2);
         const float4 c = *reinterpret_cast<const float4*>(ct + d), s = *reinterpret_cast<const float4*>(st + d);
         half8_t &lo = qb[j], &hi = qb[j + DT / 32];
-        lo[e] = (_Float16)((u.x * c.x - v.x * s.x) * a.qscale), hi[e] = (_Float16)((v.x * c.x + u.x * s.x) * a.qscale);
-        lo[e + 1] = (_Float16)((u.y * c.y - v.y * s.y) * a.qscale), hi[e + 1] = (_Float16)((v.y * c.y + u.y * s.y) * a.qscale);
-        lo[e + 2] = (_Float16)((u.z * c.z - v.z * s.z) * a.qscale), hi[e + 2] = (_Float16)((v.z * c.z + u.z * s.z) * a.qscale);
-        lo[e + 3] = (_Float16)((u.w * c.w - v.w * s.w) * a.qscale), hi[e + 3] = (_Float16)((v.w * c.w + u.w * s.w) * a.qscale);
+        lo[e] = (_Float16)(u.x * c.x - v.x * s.x), hi[e] = (_Float16)(v.x * c.x + u.x * s.x);
+        lo[e + 1] = (_Float16)(u.y * c.y - v.y * s.y), hi[e + 1] = (_Float16)(v.y * c.y + u.y * s.y);
+        lo[e + 2] = (_Float16)(u.z * c.z - v.z * s.z), hi[e + 2] = (_Float16)(v.z * c.z + u.z * s.z);
+        lo[e + 3] = (_Float16)(u.w * c.w - v.w * s.w), hi[e + 3] = (_Float16)(v.w * c.w + u.w * s.w);
       }
   } else {
     const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)min(qr, a.M - 1) * QW + h * DT;
@@ -1270,7 +1272,6 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
   // the reference of the exponents (log2 units, -inf before the first key) and
   // this half-wave's sum
   float mrun = -INFINITY, lrun = 0.f;
-  float16_t neg_ref = {};
   const int kbeg = kfirst & ~(KT - 1);
   const int ntiles = (qhi - kbeg) / KT + 1;
   const int nsteps = (ntiles + NG - 1) / NG;
@@ -1282,14 +1283,13 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
     if (tile < ntiles && active) {
       const unsigned char* kbuf = lds + (buf * NG + grp) * AT::BYTES;
       const unsigned char* vbuf = kbuf + AT::HALF;
-      // scores less the reference: the accumulators start at -mref
-      float16_t s[2];
+      float16_t s[2] = {};
 #pragma unroll
       for (int j = 0; j < DT / 16; j++)
 #pragma unroll
         for (int b2 = 0; b2 < 2; b2++) {
           const half8_t ak = *reinterpret_cast<const half8_t*>(kbuf + 32 * b2 * AT::ROWB + rk[j]);
-          s[b2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qb[j], j == 0 ? neg_ref : s[b2], 0, 0, 0);
+          s[b2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ak, qb[j], s[b2], 0, 0, 0);
         }
       if (kt0 + KT - 1 > qlo || (a.window > 0 && kt0 < qhi - a.window + 1)) {
 #pragma unroll
@@ -1308,27 +1308,26 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
       }
       m0 = max3(m0, s[0][15], s[1][15]);
       m0 = max3(m0, m1, m1);
-      const float mx = __builtin_elementwise_maximum(m0, swap32(m0));
-      const bool first = mrun == -INFINITY, move = mx > kRefSlack || (first && mx > -INFINITY);
+      const float mx = __builtin_elementwise_maximum(m0, swap32(m0)) * a.scale_log2;
+      const bool move = mx - mrun > kRefSlack;  // not for -inf or NaN
       if (__builtin_amdgcn_ballot_w64(move)) {
-        const float d = move ? mx : 0.f, corr = move && first ? 0.f : __builtin_amdgcn_exp2f(-d);
-        if (move) mrun = (first ? 0.f : mrun) + d;
-        const float nr = mrun == -INFINITY ? 0.f : -mrun;
-#pragma unroll
-        for (int v = 0; v < 16; v++) s[0][v] -= d, s[1][v] -= d, neg_ref[v] = nr;
+        const float corr = move ? __builtin_amdgcn_exp2f(mrun - mx) : 1.f;
+        if (move) mrun = mx;
         lrun *= corr;
 #pragma unroll
         for (int i = 0; i < NDT; i++) o[i] *= corr;
       }
+      const float ref = mrun == -INFINITY ? 0.f : mrun;
       float ps[2] = {0.f, 0.f};
       uint32_t pk[2][8];
 #pragma unroll
       for (int b2 = 0; b2 < 2; b2++)
 #pragma unroll
         for (int v = 0; v < 16; v += 2) {
-          const auto pr = __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(s[b2][v]), __builtin_amdgcn_exp2f(s[b2][v + 1]));
-          ps[b2] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pr), (half2_t){(_Float16)1.f, (_Float16)1.f}, ps[b2], false);
-          pk[b2][v >> 1] = __builtin_bit_cast(uint32_t, pr);
+          const float e0 = __builtin_amdgcn_exp2f(fmaf(s[b2][v], a.scale_log2, -ref));
+          const float e1 = __builtin_amdgcn_exp2f(fmaf(s[b2][v + 1], a.scale_log2, -ref));
+          ps[b2] += e0 + e1;
+          pk[b2][v >> 1] = __builtin_bit_cast(uint32_t, (half2_t){(_Float16)e0, (_Float16)e1});
         }
       lrun += ps[0] + ps[1];
 #pragma unroll
