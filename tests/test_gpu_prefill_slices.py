@@ -39,3 +39,36 @@ def test_ragged_chunks_match_replay(storage, n):
     close(got, ref, 2e-2, 1e-2)
     runner.close()
     ctx.close()
+
+
+def test_chunks_of_several_sizes_on_one_model_equal_fresh_models():
+    """A captured chunk goes when a later one has the row buffers replaced: sizes
+    in turn and again, over a first set of buffers for chunks of 128 rows and a
+    second for 2048, give a fresh model's cache rows bit for bit."""
+    layers, base, longest = 2, W.WORKLOADS["llama-3.2-1b"], 2048
+    cfg = dict(base.config, num_hidden_layers=layers, vocab_size=4096)
+    wl = W.Workload(base.name + "-2l", cfg, base.storage, longest + 1, 6, longest + 8, qkv_bias=base.qkv_bias)
+    hw = W.synthetic(wl)
+    hw.keep = True
+    ctx = tlm.Context(0)
+    prompt = [int(t) for t in np.random.default_rng(9).integers(0, 4096, longest)]
+
+    def rows(m, n):
+        print(f"[prefill sizes] {n} rows", flush=True)
+        m.reset_cache()
+        m.prefill(prompt, 0, n)
+        return [a.copy() for l in range(layers) for a in m.kv_read(l, 0, n)]
+
+    fresh = {}
+    for n in (127, 1000, 1500, 2048):
+        runner = R.DecoderHIPRunner(hw, {"maxTokens": longest + 8, "prefillChunkSize": 2048}, ctx=ctx)
+        fresh[n] = rows(runner.model, n)
+        runner.close()
+    runner = R.DecoderHIPRunner(hw, {"maxTokens": longest + 8, "prefillChunkSize": 128}, ctx=ctx)
+    for chunk, sizes in ((128, (127,)), (2048, (127, 1000, 127, 2048, 1500, 2048, 1000, 127))):
+        runner.model.set_prefill(64, chunk)
+        for n in sizes:
+            for a, b in zip(rows(runner.model, n), fresh[n]):
+                assert np.array_equal(a, b), f"{n} rows in chunks of up to {chunk}"
+    runner.close()
+    ctx.close()

@@ -224,7 +224,6 @@ struct tlm_model {
   // device (asynchronous copies: the host does not wait for a staging copy)
   int* host_pin = nullptr;
   int pf_replayed = 0;     // batched chunks replayed on the decode graph after such a flag
-  size_t pf_part_n = 0;
   uint16_t *pf_xn = nullptr, *pf_q = nullptr, *pf_att = nullptr, *pf_h = nullptr;
   int* pf_ex = nullptr;      // per row: the exponent of the attention norm's scale (GEMM_FOLD)
   float* pf_ss = nullptr;    // per row and 64-column tile: sums of squares of the residual (GEMM_FOLD)
@@ -1159,6 +1158,14 @@ static int model_alloc(void** p, size_t bytes) {
   return TLM_OK;
 }
 
+static void drop_graphs(std::map<int, std::pair<hipGraph_t, hipGraphExec_t>>& graphs) {
+  for (auto& kv : graphs) {
+    hipGraphExecDestroy(kv.second.second);
+    hipGraphDestroy(kv.second.first);
+  }
+  graphs.clear();
+}
+
 void tlm_model_destroy(tlm_model* m);
 
 // Replicas of the fixed-point residual for a hidden size: the MLP's down
@@ -1435,11 +1442,8 @@ void tlm_model_destroy(tlm_model* m) {
   if (!m) return;
   hipStreamSynchronize(m->ctx->stream);
   ps_register(m, false);
-  for (auto* gm : {&m->pf_graphs, &m->replay_graphs})
-    for (auto& kv : *gm) {
-      hipGraphExecDestroy(kv.second.second);
-      hipGraphDestroy(kv.second.first);
-    }
+  drop_graphs(m->pf_graphs);
+  drop_graphs(m->replay_graphs);
   for (int i = 0; i < 2; i++) {
     if (m->g_logits[i]) hipGraphExecDestroy(m->g_logits[i]);
     if (m->g_prefill[i]) hipGraphExecDestroy(m->g_prefill[i]);
@@ -1837,33 +1841,47 @@ static const char* prefill_unsupported(const tlm_model* m) {
   return nullptr;
 }
 
-// Row buffers for `rows` positions and `part` floats of split-K slices.
-static int prefill_alloc(tlm_model* m, int rows, size_t part) {
+// The partial-sum GEMMs of a batched chunk of M rows (QKV, O, down) and the
+// floats of split-K slices that they need.  Not monotonic in M: a Llama-3.2-1B
+// chunk of 1500 rows has 46.9 MiB of slices, one of 2048 rows 32.0.
+struct PfPartial {
+  GemmShape q, o, d;
+  size_t floats;
+};
+static PfPartial prefill_partial(const tlm_model* m, int M) {
+  const int lf = wfmt(m->d.linear_fmt), cus = m->ctx->cus, H = m->d.hidden_size;
+  PfPartial p;
+  p.q = gemm_shape(lf, GEMM_PART, M, m->Nqkv, H, cus);
+  p.o = gemm_shape(lf, GEMM_PART, M, H, m->QS, cus);
+  p.d = gemm_shape(lf, GEMM_PART, M, H, m->d.intermediate_size, cus);
+  p.floats = std::max({(size_t)p.q.splits * M * m->Nqkv, (size_t)p.o.splits * M * H, (size_t)p.d.splits * M * H});
+  return p;
+}
+
+// Row buffers for `rows` positions and the split-K slices of every chunk up to
+// that size.  The captured chunks hold the buffers' addresses, so they go with
+// the buffers that a larger set replaces.
+static int prefill_alloc(tlm_model* m, int rows) {
   if (!m->pf_ovf) {
     int rc = model_alloc((void**)&m->pf_ovf, sizeof(int));
     if (rc) return rc;
   }
-  if (m->pf_cap >= rows && m->pf_part_n >= part) return TLM_OK;
-  HIP_TRY(hipStreamSynchronize(m->ctx->stream));
-  if (m->pf_part_n < part) {
-    hipFree(m->pf_part);
-    m->pf_part = nullptr;
-    m->pf_part_n = 0;
-    int rc = model_alloc((void**)&m->pf_part, sizeof(float) * part);
-    if (rc) return rc;
-    m->pf_part_n = part;
-  }
   if (m->pf_cap >= rows) return TLM_OK;
   rows = std::max(rows, m->pf_chunk);  // one allocation serves every later chunk
-  void* bufs[] = {m->pf_x, m->pf_xn, m->pf_q, m->pf_att, m->pf_h, m->pf_ex, m->pf_ss};
+  size_t part = 0;
+  for (int M = 1; M <= rows; M++) part = std::max(part, prefill_partial(m, M).floats);
+  HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+  drop_graphs(m->pf_graphs);
+  void* bufs[] = {m->pf_x, m->pf_xn, m->pf_q, m->pf_att, m->pf_h, m->pf_ex, m->pf_ss, m->pf_part};
   for (void* q : bufs) hipFree(q);
-  m->pf_x = nullptr;
+  m->pf_x = m->pf_part = nullptr;
   m->pf_xn = m->pf_q = m->pf_att = m->pf_h = nullptr;
   m->pf_ex = nullptr;
   m->pf_ss = nullptr;
   m->pf_cap = 0;
   const size_t R = (size_t)rows, H = m->d.hidden_size, I = m->d.intermediate_size;
   int rc = TLM_OK;
+  if (!rc) rc = model_alloc((void**)&m->pf_part, sizeof(float) * part);
   if (!rc) rc = model_alloc((void**)&m->pf_x, sizeof(float) * R * H);
   if (!rc) rc = model_alloc((void**)&m->pf_xn, 2 * R * H);
   if (!rc) rc = model_alloc((void**)&m->pf_q, 2 * R * m->QS);
@@ -1930,17 +1948,18 @@ static const bool g_pf_fold = [] {
 }();
 static int prefill_plan(tlm_model* m, int M, PfPlan* pp) {
   const tlm_model_desc& d = m->d;
-  const int H = d.hidden_size, I = d.intermediate_size, D = d.head_dim;
+  const int H = d.hidden_size, D = d.head_dim;
   const int lf = wfmt(d.linear_fmt), cus = m->ctx->cus;
   const Layer& L0 = m->layers[0];
-  pp->sq = gemm_shape(lf, GEMM_PART, M, m->Nqkv, H, cus);
+  const PfPartial partial = prefill_partial(m, M);
+  pp->sq = partial.q;
+  pp->so = partial.o;
+  pp->sd = partial.d;
   // small chunks (the K-wave QKV GEMM), head_dim 64, full rotary: RoPE and the
   // cache append run in the QKV GEMM's epilogue (no split-K slices, no rope_kv)
   pp->sr = gemm_shape(lf, GEMM_ROPE, M, m->Nqkv, H, cus);
   pp->rope_epi = lf == WF_Q4 && pp->sr.tile == GT_KW && D == 64 && d.rotary_dim == 64;
-  pp->so = gemm_shape(lf, GEMM_PART, M, H, m->QS, cus);
   pp->sg = gemm_shape(lf, GEMM_SWIGLU, M, L0.gu->T * kTile, H, cus);
-  pp->sd = gemm_shape(lf, GEMM_PART, M, H, I, cus);
   // small chunks (K-wave O and gate|up GEMMs): the O GEMM, unsplit, adds its
   // rows to the residual and writes the FFN norm's operand as fp16(x w 2^e),
   // e from the attention norm of the same rows (which keeps it near unit
@@ -1951,9 +1970,7 @@ static int prefill_plan(tlm_model* m, int M, PfPlan* pp) {
   pp->sf = gemm_shape(lf, GEMM_FOLD, M, H, m->QS, cus);
   pp->fold = g_pf_fold && lf == WF_Q4 && pp->sf.tile == GT_KW && pp->sg.tile == GT_KW && H % kTile == 0 &&
              H / kTile <= 32;
-  const size_t part = std::max({(size_t)pp->sq.splits * M * m->Nqkv, (size_t)pp->so.splits * M * H,
-                                (size_t)pp->sd.splits * M * H});
-  return prefill_alloc(m, M, part);
+  return prefill_alloc(m, M);
 }
 
 // Kernels of one batched chunk of M rows (the counterpart of the reference's
