@@ -113,3 +113,18 @@ def test_queries_round_before_the_softmax_scale(ctx, D, rotary, scale, q0, unit,
     x64[:, :2 * D] *= scale
     ref = expected(x64, 0, 2, 1, D, 0)
     assert np.abs(got - ref).max() <= 2e-3 * max(1.0, np.abs(ref).max())
+
+
+def test_rows_written_right_after_creation_stay(ctx):
+    """The cache's first fill ends before its attention is handed out: 512 MiB
+    each of K and V, and the rows of the first calls are there afterwards."""
+    heads, kv, D, rows = 8, 8, 128, 64
+    x = np.random.default_rng(5).standard_normal((rows, (heads + 2 * kv) * D)).astype(np.float16).astype(np.float32)
+    qkv, out = ctx.array(x), ctx.buffer(2 * rows * heads * D)
+    ctx.sync()
+    for _ in range(3):
+        A = tlm.Attention(ctx, heads, kv, D, 1 << 18)  # no rotary dims: the rows are the projection's
+        A.rows_noalloc(qkv, rows, 0, out)
+        k, v = A.read_cache(rows)
+        A.close()
+        assert np.array_equal(np.concatenate([k, v], 1), x[:, heads * D:])

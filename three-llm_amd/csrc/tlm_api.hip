@@ -832,6 +832,7 @@ static int attn_init(tlm_ctx* ctx, const tlm_attn_desc* d, tlm_attn* A, bool own
     if (!attention_one_prepare(d->kv_fmt == TLM_FMT_F32, D))
       return fail(TLM_ERR_HIP, "TLMAttention: the one-call kernel's LDS was refused");
   }
+  HIP_TRY(hipStreamSynchronize(nullptr));  // the fills are on another stream than the context's
   return TLM_OK;
 }
 
@@ -1150,10 +1151,12 @@ int tlm_op_topk(tlm_ctx* ctx, const float* logits, int n, int k, double softcap,
 
 // -------------------------------------------------------------------- model --
 
+// Zeroed device memory, ready for the context's stream (which does not wait for
+// the fill's by itself).
 static int model_alloc(void** p, size_t bytes) {
   if (hipMalloc(p, std::max<size_t>(bytes, 4)) != hipSuccess)
     return fail(TLM_ERR_OOM, "TLMModel: device allocation of %zu bytes failed", bytes);
-  if (hipMemset(*p, 0, std::max<size_t>(bytes, 4)) != hipSuccess)
+  if (hipMemset(*p, 0, std::max<size_t>(bytes, 4)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
     return fail(TLM_ERR_HIP, "TLMModel: memset failed");
   return TLM_OK;
 }
