@@ -1,16 +1,15 @@
 """One decode attention call at the window lengths where its route changes: the
-block per head (a wave per pass of 8 to 64 positions), the block per kv head
-(32-position tiles, up to 512 or 768 positions) and the chunks with their combine,
-each one position short of, at and past its edge, as prefix lengths and as sliding
-windows.
+block per head (a wave per pass of 8 to 64 positions, 12 of them), the chunks with
+their combine and, past 1024 positions, the matrix-core kernel, each one position
+short of, at and past its edge, as prefix lengths and as sliding windows.
 
 Inputs of unit scale, so the scores' softmax is neither flat nor a single row.
 The reference attends to the cache rows that the device holds: a K element whose
 fp32 rotation falls across an fp16 tie from the 64-bit one moves its score by up to
 2^-10 |k| |q| scale, about 1e-3, which would hide what is tested; the rows
 themselves are checked to one rounding of their own.  What is left is fp32 sums
-and exponentials (q enters the matrix cores as hi + lo fp16 pairs): 2e-5 of the
-output's scale, and 5e-6 with fp32 rows."""
+and exponentials (past 1024 positions q enters the matrix cores as hi + lo fp16
+pairs): 2e-5 of the output's scale, and 5e-6 with fp32 rows."""
 import numpy as np
 import pytest
 
@@ -72,10 +71,10 @@ def run(ctx, hq, hkv, d, kv_fmt, positions, window=0, rotary=None):
 
 @pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (4, 4, 64), (24, 8, 128), (3, 1, 128), (16, 1, 64)])
 def test_fp16_cache_routes(ctx, hq, hkv, d):
-    # 64 | 65: per head -> per kv head; 256 | 257: one tile a wave -> two; 512 | 513 and
-    # 768 | 769 (prefix lengths): chunks; 1024 | 1025: a window the model calls long
-    run(ctx, hq, hkv, d, tlm.FMT_F16, [0, 1, 15, 16, 31, 32, 62, 63, 64, 65, 127, 255, 256, 511, 512, 513, 767, 768, 769,
-                                       1023, 1024, 1025])
+    # 192 | 193 (head_dim 128) and 384 | 385 (64): block per head -> chunks; 1024 | 1025
+    # (prefix lengths): the matrix-core kernel
+    run(ctx, hq, hkv, d, tlm.FMT_F16, [0, 1, 15, 16, 31, 32, 62, 63, 64, 65, 127, 190, 191, 192, 255, 256, 382, 383, 384,
+                                       511, 512, 513, 767, 768, 769, 1023, 1024, 1025])
 
 
 @pytest.mark.parametrize("d,positions", [(64, [0, 15, 16, 63, 190, 191, 192, 193, 300]), (128, [0, 7, 8, 94, 95, 96, 97, 200]),
@@ -92,3 +91,29 @@ def test_sliding_windows(ctx, window):
 def test_without_the_matrix_core_kernel_and_partial_rotary(ctx):
     run(ctx, 4, 2, 32, tlm.FMT_F16, [0, 63, 64, 767, 768, 769, 1030], rotary=16)
     run(ctx, 8, 4, 64, tlm.FMT_F16, [0, 63, 64, 700], rotary=32)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("position", [70, 300, 500, 800, 1023])
+def test_queries_past_the_fp16_range(ctx, d, position):
+    """Windows up to 1024 positions keep q in 32 bits: q * attn_scale * log2 e is past
+    fp16's largest value here, over cache rows small enough for scores of order ten.
+    Their 32-bit sums of d terms are off by at most d 2^-24 of the terms' magnitudes
+    (51 in all at d 64): 2e-4 of a probability."""
+    hq, hkv = 4, 2
+    rng = np.random.default_rng(d + position)
+    n = position + 1
+    x = np.zeros((n, hq + 2 * hkv, d), np.float32)
+    x[:, hq:hq + hkv] = rng.integers(-32, 33, (n, hkv, d)) * 2.0 ** -20 * (64 / d)
+    x[:, hq + hkv:] = rng.standard_normal((n, hkv, d)).astype(np.float16)
+    a = tlm.Attention(ctx, hq, hkv, d, n, attn_scale=1.0)  # no rotary dims
+    a.rows(ctx.array(x), n, 0, ctx.buffer(2 * n * hq * d))
+    x[position, :hq] = rng.standard_normal((hq, d)) * 2.0 ** 16
+    got = a(ctx.array(x[position]), position, ctx.buffer(4 * hq * d)).read().reshape(hq, d)
+    kc, vc = (c.reshape(n, hkv, d).astype(np.float64) for c in a.read_cache(n))
+    a.close()
+    for h in range(hq):
+        s = kc[:, h // 2] @ x[position, h].astype(np.float64)
+        e = np.exp(s - s.max())
+        ref = (e / e.sum()) @ vc[:, h // 2]
+        assert np.abs(got[h] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), f"head {h}"

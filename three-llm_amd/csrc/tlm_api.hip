@@ -910,27 +910,20 @@ int tlm_op_attention(tlm_attn* A, const float* qkv, int position, float* out) {
   if (position < 0 || position >= A->d.max_tokens)
     return fail(TLM_ERR_RANGE, "TLMAttention: position %d outside [0, %d)", position, A->d.max_tokens);
   hipStream_t st = A->ctx->stream;
-  const int total = (A->d.heads + 2 * A->d.kv_heads) * A->d.head_dim, D = A->d.head_dim;
+  const int total = (A->d.heads + 2 * A->d.kv_heads) * A->d.head_dim;
   const bool f32 = A->d.kv_fmt == TLM_FMT_F32;
   const int n = A->d.sliding_window > 0 ? std::min(position + 1, A->d.sliding_window) : position + 1;
-  // One launch as long as one block per head (or per kv head, on the matrix
-  // cores) is faster than chunks and the kernel that combines them.  us a call,
-  // Llama-3.2-1B heads (head_dim 64) / Llama-3.2-3B (128), with the position in
-  // the launch instead of in a control word that a kernel of its own writes:
-  //   block per head        32 positions 3.4 / 4.9   101 4.8 / 6.5   512 7.7 / 10.5
-  //   block per kv head     32 positions 4.4 / 5.9   101 4.5 / 6.1   512 5.7 / 8.6   701 7.3 / 11.2   1001 8.5 / 14.0
-  //   chunks and a combine  1501 positions 8.3 / 9.7 (as many up to 4 chunks fewer)
-  // Without the matrix-core kernel (fp32 cache, other head_dims) the block per
-  // head serves windows of one pass per wave.
-  const bool per_head = n <= (A->gqa ? 64 : attention_one_positions(f32, D));
-  const bool per_kv_head = !per_head && A->gqa && n <= (D == 64 ? 768 : 512);
-  const bool lw = A->gqa || long_window(A, position);
+  // One launch where the window is one pass for each of a block's waves: past
+  // that, chunks and the kernel that combines them are faster.  Both keep the
+  // queries and probabilities of windows up to kLongWindow in 32 bits.  us a call,
+  // Qwen2.5-0.5B heads (head_dim 64) / Llama-3.2-3B (128):
+  //   block per head        32 positions 3.9 / 4.8   192 5.2 / 7.7   384 6.6 / 8.8   501 8.0 / 9.8    1024 9.5 / 13.3
+  //   chunks and a combine  32 positions 6.7 / 7.5   192 7.1 / 7.8   384 7.1 / 8.0   501 7.1 / 8.0    1024 7.4 / 8.2
+  const bool one = n <= attention_one_positions(f32, A->d.head_dim), lw = long_window(A, position);
   AttnArgs a = attn_args(A, qkv, 1, total, nullptr, nullptr, A->kc, A->vc, out, lw);
   a.pos = position;
-  if (per_head || per_kv_head) a.nsplit = 1;
-  if (!(per_head      ? launch_attention_one(f32, a, st)
-        : per_kv_head ? launch_gqa_attention_one(a, st)
-                      : launch_attention(f32, A->gmax, a, true, lw, st)))
+  if (one) a.nsplit = 1;
+  if (!(one ? launch_attention_one(f32, a, st) : launch_attention(f32, A->gmax, a, true, lw, st)))
     return fail(TLM_ERR_STATE, "TLMAttention: no kernel variant for this shape");
   CHECK_LAUNCH("TLMAttention");
   return TLM_OK;

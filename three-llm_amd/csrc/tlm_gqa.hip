@@ -101,9 +101,7 @@ struct GqaV {
   }
 };
 
-// ONE (one call over a short window): one block per kv head takes the whole
-// window and writes the output itself; q|k|v come as one vector.
-template <int DT, bool ONE>
+template <int DT>
 __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
   using S = GqaShape<DT>;
   __shared__ __align__(16) _Float16 lds[S::LDS_HALVES];
@@ -115,7 +113,7 @@ __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
 
   const int G = a.G, Hkv = a.Hkv;
   const int hk = blockIdx.x % Hkv, c = blockIdx.x / Hkv;
-  const int pos = ONE ? a.pos : a.ctrl ? a.ctrl[C_POS] : a.pos;
+  const int pos = a.ctrl ? a.ctrl[C_POS] : a.pos;
   if (pos < 0 || pos >= a.max_tokens) return;
   const ChunkPlan cp = chunk_plan(pos, a.window, a.nsplit, a.chmin);
   if (c >= cp.nact) return;  // block-uniform, before any barrier
@@ -140,13 +138,12 @@ __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
     const int r = e / DT, d = e % DT;
     return r < G ? (hk * G + r) * DT + d : (r == G ? QW : QW + KW) + hk * DT + d;
   };
-  constexpr int NSRC = ONE ? 1 : kMaxPart;
-  float gp[kGqaPro][NSRC], gb[kGqaPro];
+  float gp[kGqaPro][kMaxPart], gb[kGqaPro];
 #pragma unroll
   for (int x = 0; x < kGqaPro; x++) {
     const int col = col_of(min(tid + 64 * kGqaWaves * x, E - 1));
 #pragma unroll
-    for (int j = 0; j < NSRC; j++) gp[x][j] = a.src[(size_t)max(min(j, a.n_src - 1), 0) * a.src_stride + col];
+    for (int j = 0; j < kMaxPart; j++) gp[x][j] = a.src[(size_t)max(min(j, a.n_src - 1), 0) * a.src_stride + col];
     gb[x] = a.bias[col];
   }
   // every element this thread rotates has dim d = tid % DT (64 kGqaWaves is a multiple of DT)
@@ -167,7 +164,7 @@ __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
   for (int x = 0; x < kGqaPro; x++) {
     float sum = gb[x];
 #pragma unroll
-    for (int j = 0; j < NSRC; j++) sum = fmaf(gp[x][j], j < a.n_src ? 1.f : 0.f, sum);
+    for (int j = 0; j < kMaxPart; j++) sum = fmaf(gp[x][j], j < a.n_src ? 1.f : 0.f, sum);
     raw[tid + 64 * kGqaWaves * x] = sum;
   }
   lds_barrier();
@@ -357,10 +354,6 @@ __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
       L = fmaf(rec[1], sc, L);
       O = fmaf(rec[2 + d], sc, O);
     }
-    if (ONE) {
-      a.out[(size_t)(hk * G + j) * DT + d] = O / L;
-      continue;
-    }
     const size_t row = (size_t)(hk * G + j) * a.nsplit + c;
     a.pacc[row * DT + d] = O;
     if (d == 0) {
@@ -375,16 +368,8 @@ __global__ __launch_bounds__(64 * kGqaWaves) void gqa_attn_kernel(AttnArgs a) {
 bool launch_gqa_attention(const AttnArgs& a, hipStream_t st) {
   if (!gqa_attention_fits(a.G, a.D)) return false;
   const dim3 grid((unsigned)(a.Hkv * a.nsplit)), block(64 * kGqaWaves);
-  if (a.D == 64) hipLaunchKernelGGL((gqa_attn_kernel<64, false>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((gqa_attn_kernel<128, false>), grid, block, 0, st, a);
-  return true;
-}
-
-bool launch_gqa_attention_one(const AttnArgs& a, hipStream_t st) {
-  if (!gqa_attention_fits(a.G, a.D)) return false;
-  const dim3 grid((unsigned)a.Hkv), block(64 * kGqaWaves);
-  if (a.D == 64) hipLaunchKernelGGL((gqa_attn_kernel<64, true>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((gqa_attn_kernel<128, true>), grid, block, 0, st, a);
+  if (a.D == 64) hipLaunchKernelGGL(gqa_attn_kernel<64>, grid, block, 0, st, a);
+  else hipLaunchKernelGGL(gqa_attn_kernel<128>, grid, block, 0, st, a);
   return true;
 }
 

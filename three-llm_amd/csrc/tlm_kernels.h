@@ -192,8 +192,6 @@ bool launch_attention(bool kv_f32, int gmax, const AttnArgs& a, bool combine, bo
 int attention_one_positions(bool kv_f32, int D);
 bool attention_one_prepare(bool kv_f32, int D);
 bool launch_attention_one(bool kv_f32, const AttnArgs& a, hipStream_t st);
-// the same on the matrix cores, one block per kv head (what gqa_attention_fits covers)
-bool launch_gqa_attention_one(const AttnArgs& a, hipStream_t st);
 // long windows, fp16 cache, head_dim 64 or 128, G <= 16: grid Hkv x nsplit
 bool launch_gqa_attention(const AttnArgs& a, hipStream_t st);
 size_t gemv_smem_bytes(int fmt, int cps, int waves);
