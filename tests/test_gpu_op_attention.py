@@ -10,6 +10,8 @@ fp32 rotation falls across an fp16 tie from the 64-bit one moves its score by up
 themselves are checked to one rounding of their own.  What is left is fp32 sums
 and exponentials (past 1024 positions q enters the matrix cores as hi + lo fp16
 pairs): 2e-5 of the output's scale, and 5e-6 with fp32 rows."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -117,3 +119,24 @@ def test_queries_past_the_fp16_range(ctx, d, position):
         e = np.exp(s - s.max())
         ref = (e / e.sum()) @ vc[:, h // 2]
         assert np.abs(got[h] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), f"head {h}"
+
+
+@pytest.mark.parametrize("kv_fmt", [tlm.FMT_F16, tlm.FMT_F32])
+@pytest.mark.parametrize("d,position", [(64, 0), (64, 40), (64, 150), (128, 90), (20, 60)])
+def test_out_inside_qkv(ctx, d, position, kv_fmt):
+    """out over any part of qkv: over the queries alone, half over the keys, over the
+    keys and values.  The sums may be taken in another order than with out apart."""
+    hq, hkv = 16, 8
+    rng = np.random.default_rng(d + position)
+    x = rng.standard_normal((position + 1, (hq + 2 * hkv) * d)).astype(np.float32)
+    a = tlm.Attention(ctx, hq, hkv, d, position + 1, kv_fmt=kv_fmt)
+    qkv, out = ctx.buffer(x[0].nbytes), ctx.buffer(4 * hq * d)
+    for p in range(position + 1):
+        a(qkv.write(x[p]), p, out)
+    ref = out.read().reshape(hq * d)
+    for at in (0, hq * d // 2 + 1, hq * d):
+        qkv.write(x[position])
+        tlm.check(tlm.lib().tlm_op_attention(a.ptr, qkv.ptr, position, ctypes.c_void_p(qkv.ptr.value + 4 * at)))
+        got = qkv.read().reshape(-1)[at:at + hq * d]
+        assert np.abs(got - ref).max() <= 2e-6 * max(1.0, np.abs(ref).max()), f"out at {at}"
+    a.close()

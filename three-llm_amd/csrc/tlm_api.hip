@@ -919,7 +919,11 @@ int tlm_op_attention(tlm_attn* A, const float* qkv, int position, float* out) {
   // Qwen2.5-0.5B heads (head_dim 64) / Llama-3.2-3B (128):
   //   block per head        32 positions 3.9 / 4.8   192 5.2 / 7.7   384 6.6 / 8.8   501 8.0 / 9.8    1024 9.5 / 13.3
   //   chunks and a combine  32 positions 6.7 / 7.5   192 7.1 / 7.8   384 7.1 / 8.0   501 7.1 / 8.0    1024 7.4 / 8.2
-  const bool one = n <= attention_one_positions(f32, A->d.head_dim), lw = long_window(A, position);
+  // Its blocks write their heads of out while others still read qkv.  out over
+  // qkv from the start on is fine (a block writes where only it reads); any other
+  // overlap takes the chunks, whose out a kernel of its own writes.
+  const bool apart = out == qkv || !overlap(qkv, total, out, (size_t)A->d.heads * A->d.head_dim);
+  const bool one = apart && n <= attention_one_positions(f32, A->d.head_dim), lw = long_window(A, position);
   AttnArgs a = attn_args(A, qkv, 1, total, nullptr, nullptr, A->kc, A->vc, out, lw);
   a.pos = position;
   if (one) a.nsplit = 1;
