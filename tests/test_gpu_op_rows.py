@@ -2,6 +2,8 @@
 float64 product of the fp16 operands the matrix cores see (weights rounded to
 fp16 once, activations fp16).  fp32 sums of K products: an error bound of
 2e-6 of the sum of magnitudes, as for any order of the same additions."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -59,3 +61,28 @@ def test_rows_at_tile_edges(ctx, fmt, M, N, K, bias):
         ref, mag = ref + b, mag + np.abs(b)
     excess = np.abs(y - ref) - (2e-6 * mag + 1e-7)
     assert excess.max() <= 0, f"max excess {excess.max()}"
+
+
+@pytest.mark.parametrize("fmt", [tlm.FMT_F16, tlm.FMT_Q4])
+@pytest.mark.parametrize("M,N,K", [(3, 100, 96), (130, 4200, 512), (40, 64, 1 << 19)])
+def test_rows_from_any_alignment_of_x(ctx, fmt, M, N, K):
+    """x at 2, 4 and 8 bytes past a 16-byte boundary: the rows are staged (the last
+    shape in two parts) and give the aligned call's sums, of unsplit products."""
+    print(f"[rows] unaligned x, fmt {fmt}, {M} x {N} x {K}", flush=True)
+    rng = np.random.default_rng(M + N)
+    w = (rng.standard_normal((N, K), dtype=np.float32) * 0.02).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32).astype(np.float16)
+    b = (rng.standard_normal(N) * 0.1).astype(np.float32)
+    L, wd = make_linear(ctx, fmt, w)
+    xh, wh = x.astype(np.float32), wd.astype(np.float16).astype(np.float32)
+    ref, mag = xh.astype(np.float64) @ wh.T.astype(np.float64) + b, np.abs(xh) @ np.abs(wh).T + np.abs(b)
+    bias, out = ctx.array(b), ctx.buffer(4 * M * N)
+    for halves in (1, 2, 4):
+        buf = ctx.array(np.concatenate([np.zeros(halves, np.uint16), x.view(np.uint16).reshape(-1)]))
+        assert buf.ptr.value % 16 == 0
+        out.write(np.full(M * N, np.nan, np.float32))
+        tlm.check(tlm.lib().tlm_op_linear_rows(L.ptr, ctypes.c_void_p(buf.ptr.value + 2 * halves), M, bias.ptr, out.ptr))
+        excess = np.abs(out.read().reshape(M, N) - ref) - (2e-6 * mag + 1e-7)
+        assert excess.max() <= 0, f"{halves} halves: max excess {excess.max()}"
+        buf.free()
+    L.close()

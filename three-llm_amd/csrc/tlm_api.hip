@@ -92,7 +92,7 @@ struct tlm_ctx {
   float* topk_v = nullptr;
   int* topk_i = nullptr;
   void* scratch = nullptr;  // this device's copy of `scratch` (device address)
-  float* part = nullptr;    // split-K slices of tlm_op_linear_rows (kPartFloats)
+  float* part = nullptr;    // split-K slices (or unaligned rows) of tlm_op_linear_rows (kPartFloats)
   std::mutex part_mu;
 };
 constexpr size_t kPartFloats = (size_t)8 << 20;  // 32 MiB
@@ -699,6 +699,25 @@ int tlm_op_linear_rows(tlm_linear* L, const uint16_t* x, int32_t rows, const flo
   if (L->fmt == TLM_FMT_Q4 && L->smax > 0x6FFF)
     return fail(TLM_ERR_INVALID, "TLMLinear: q4 scale above 8188 overflows the fp16 GEMM operand");
   tlm_ctx* ctx = L->ctx;
+  // The kernels copy 16-byte pieces of x to LDS: rows from another alignment go
+  // through the slices' buffer, as many at a time as it holds, unsplit.
+  if (reinterpret_cast<uintptr_t>(x) % 16) {
+    const int most = (int)std::min<size_t>(rows, kPartFloats * sizeof(float) / (sizeof(uint16_t) * L->K));
+    if (most < 1) return fail(TLM_ERR_INVALID, "TLMLinear: a row of %d from an unaligned x", L->K);
+    std::lock_guard<std::mutex> lock(ctx->part_mu);
+    uint16_t* staged = reinterpret_cast<uint16_t*>(ctx->part);
+    g.A = staged;
+    for (int r = 0; r < rows; r += most) {
+      g.M = std::min(most, rows - r);
+      g.Cf = y + (size_t)r * L->N;
+      launch_copy_f16(x + (size_t)r * L->K, (size_t)g.M * L->K, staged, ctx->stream);
+      const GemmShape sh = gemm_shape(wfmt(L->fmt), GEMM_STORE, g.M, L->N, L->K, ctx->cus);
+      if (!launch_gemm(wfmt(L->fmt), GEMM_STORE, sh, g, ctx->stream))
+        return fail(TLM_ERR_STATE, "TLMLinear: no batched kernel variant for %d x %d", L->N, L->K);
+    }
+    CHECK_LAUNCH("TLMLinear");
+    return TLM_OK;
+  }
   const GemmShape sh = gemm_shape(wfmt(L->fmt), GEMM_STORE, rows, L->N, L->K, ctx->cus, kPartFloats);
   const bool split = sh.splits > 1;
   // the slices live in the context's buffer from the GEMM to the fold: another

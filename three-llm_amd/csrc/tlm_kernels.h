@@ -459,6 +459,7 @@ GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part
 bool launch_gemm(int fmt, int epi, const GemmShape& sh, const GemmArgs& g, hipStream_t st);
 // y[m][n] = bias[n] + the sum of n_part slices part[s][m][n]
 void launch_fold_rows(const float* part, int n_part, const float* bias, int M, int N, float* y, hipStream_t st);
+void launch_copy_f16(const uint16_t* x, size_t n, uint16_t* y, hipStream_t st);
 void launch_rms_rows(const RowsArgs& a, int M, hipStream_t st);
 void launch_rope_kv(const RopeKvArgs& a, hipStream_t st);
 bool launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st);

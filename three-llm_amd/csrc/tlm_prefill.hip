@@ -1401,6 +1401,15 @@ bool launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st) {
   return true;
 }
 
+__global__ void copy_f16_kernel(const uint16_t* x, size_t n, uint16_t* y) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = x[i];
+}
+
+void launch_copy_f16(const uint16_t* x, size_t n, uint16_t* y, hipStream_t st) {
+  hipLaunchKernelGGL(copy_f16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, n, y);
+}
+
 // fp32 -> fp16 (round to nearest even)
 __global__ void rows_to_f16_kernel(const float* x, size_t n, _Float16* y) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
