@@ -96,6 +96,14 @@ int tlm_op_linear(tlm_linear* lin, const float* x, const float* bias, float* y);
  * y: fp32 device [rows][N].  W is dequantised to fp16 ((code - 8) * s rounded
  * once), products accumulate in fp32.  Enqueue only. */
 int tlm_op_linear_rows(tlm_linear* lin, const uint16_t* x, int32_t rows, const float* bias, float* y);
+/* How a batched linear of that size runs on `cus` compute units: plan[0] rows by
+ * plan[1] columns of a block, plan[2] slices of K; us[0] the predicted time of
+ * that choice, us[1] of the best one on another block size (inf: none weighed).
+ * partial: the partial sums of the batched prefill (QKV, O and down GEMM),
+ * else tlm_op_linear_rows.  Host only: needs no device; for tests and reports,
+ * without a counterpart in the reference. */
+int tlm_rows_plan(int fmt, int partial, int32_t rows, int32_t n_out, int32_t k_in, int32_t cus, int32_t* plan,
+                  float* us);
 
 /* ----------------------------------------------------------- element ops */
 /* TSLRMSNorm (tsl/TSLRMSNorm.ts:18-81): y = x * rsqrt(mean(x^2) + eps) * (offset ? 1 + w : w). */

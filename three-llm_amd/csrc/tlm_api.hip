@@ -734,6 +734,21 @@ int tlm_op_linear_rows(tlm_linear* L, const uint16_t* x, int32_t rows, const flo
   return TLM_OK;
 }
 
+int tlm_rows_plan(int fmt, int partial, int32_t rows, int32_t n_out, int32_t k_in, int32_t cus, int32_t* plan,
+                  float* us) {
+  if ((fmt != TLM_FMT_F16 && fmt != TLM_FMT_Q4) || rows < 1 || n_out < 1 || k_in < 32 || k_in % 32 || cus < 1 ||
+      !plan || !us)
+    return fail(TLM_ERR_INVALID, "TLMLinear: invalid argument");
+  const GemmShape sh =
+      gemm_shape(wfmt(fmt), partial ? GEMM_PART : GEMM_STORE, rows, n_out, k_in, cus, partial ? 0 : kPartFloats);
+  plan[0] = gemm_tile_rows(sh.tile);
+  plan[1] = gemm_tile_cols(sh.tile);
+  plan[2] = sh.splits;
+  us[0] = sh.us;
+  us[1] = sh.rejected;
+  return TLM_OK;
+}
+
 // -------------------------------------------------------------- element ops --
 
 int tlm_op_rmsnorm(tlm_ctx* ctx, const float* x, const float* w, int n, double eps, int offset, float* y) {

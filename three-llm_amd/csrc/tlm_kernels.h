@@ -400,6 +400,7 @@ inline int gemm_tile_cols(int t) { return t == GT_KW ? 64 : t == GT_128x128 ? 12
 // host sizes the slice buffers from the same numbers the launch uses).
 struct GemmShape {
   int tile, gx, gy, spc, splits;
+  float us, rejected;  // gemm_cost of this choice and of the best on another tile (INFINITY: no other was weighed)
 };
 // Rows of the residual stream: X[m] += sum of n_part slices part[s][m]
 // (slice stride pstride floats, rows of H), then Y[m] = fp16(rmsnorm(X[m]) w)

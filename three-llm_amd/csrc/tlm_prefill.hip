@@ -769,6 +769,7 @@ GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part
   const int steps = K >= 32 ? K / 32 : 1;  // K % 32 != 0 is rejected by launch_gemm
   int splits = 1;
   s.tile = GT_KW;
+  s.us = s.rejected = INFINITY;
   if (fmt == WF_Q4 && epi != GEMM_STORE) {
     // four waves side by side over 256 columns, unless that leaves half the
     // CUs idle: then four waves split K on one tile of 32 rows: 4x the blocks
@@ -777,43 +778,54 @@ GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part
     // (measured 5-25 % faster from 64 to 1100 rows)
     const int tiles = ((N + 255) / 256) * ((M + 127) / 128);
     if (M > 64 && tiles >= cus / 2) s.tile = GT_128x256;
-    if (epi == GEMM_PART && M > 64) {
-      // sums in slices keep the CUs busy with 128-row tiles too: the cheaper of
-      // the two.  128 tiles of K 8192 (2048 rows, the Llama-3.2-1B down
-      // projection) go in 2 slices, one block per CU, and not in 4, two per CU,
-      // whose slices cost more than the shared CU gains.  Prompts of the
-      // Llama-3.2-1B shape, against whole rounds of two blocks per CU and the
-      // rule above: 1000 ids 4066 -> 3765 us, 1900 6664 -> 5736, 4096 12216 -> 11888
-      const float whole = gemm_cost(kCostQ4[0], M, N, steps, 1, cus);
-      float best = INFINITY;
-      for (int sp = 1; sp <= 32 && steps / sp >= 4; sp *= 2) {
-        const float c = gemm_cost(kCostQ4[1], M, N, steps, sp, cus);
-        if (c < best) best = c, splits = sp;
-      }
-      s.tile = best < whole ? GT_128x256 : GT_KW;
-    }
-    if (epi == GEMM_PART && s.tile == GT_KW) {
+    if (epi == GEMM_PART) {
       // split K while the grid stays within about g_split_waves waves per CU:
       // past one round of blocks a CU streams the same bytes either way and each
       // split only adds a slice for the next row kernel to fold (Qwen2.5-0.5B
       // shape, 64 to 300 rows: the down GEMM in 4 splits instead of 8, the chunk
       // 3-6 % faster)
       const int target = g_split_waves * cus, waves = 4 * ((N + kTile - 1) / kTile) * ((M + 31) / 32);
-      splits = 1;
+      s.tile = GT_KW;
       while (splits < 32 && waves * splits * 2 <= target && steps / (2 * splits * 4) >= 2) splits *= 2;
+      s.us = gemm_cost(kCostQ4[0], M, N, steps, splits, cus);
+    }
+    if (epi == GEMM_PART && M > 64) {
+      // sums in slices keep the CUs busy with 128-row tiles too: the cheaper of
+      // the two, each with its own slices.  128 tiles of K 8192 (2048 rows, the Llama-3.2-1B down
+      // projection) go in 2 slices, one block per CU, and not in 4, two per CU,
+      // whose slices cost more than the shared CU gains.  Chunks of the
+      // Llama-3.2-1B shape against whole rounds of two blocks per CU: 300 rows
+      // 1755 -> 1686 us; with the 32-row tiles weighed unsplit, 66 rows took
+      // 128-row tiles in 16 slices, 1028 us, and 940 now (947 in whole rounds)
+      float best = INFINITY;
+      int best_splits = 1;
+      for (int sp = 1; sp <= 32 && steps / sp >= 4; sp *= 2) {
+        const float c = gemm_cost(kCostQ4[1], M, N, steps, sp, cus);
+        if (c < best) best = c, best_splits = sp;
+      }
+      s.rejected = best;
+      if (best < s.us) {
+        std::swap(s.us, s.rejected);
+        s.tile = GT_128x256;
+        splits = best_splits;
+      }
     }
   } else {
     const GemmCost* tab = fmt == WF_Q4 ? kCostQ4 : kCostF16;
     const int nt = fmt == WF_Q4 ? 2 : 3;
-    float best = INFINITY;
-    for (int i = 0; i < nt; i++)
+    for (int i = 0; i < nt; i++) {
+      float tile_us = INFINITY;
+      int tile_splits = 1;
       for (int sp = 1; sp <= 32; sp *= 2) {
         if (sp > 1 && (epi == GEMM_STORE ? (size_t)sp * M * N > part : epi != GEMM_PART)) break;
         if (sp > 1 && steps / sp < (tab[i].tile == GT_KW ? 8 : 4)) break;
         float c = gemm_cost(tab[i], M, N, steps, sp, cus);
         if (sp > 1 && epi == GEMM_STORE) c += fmt == WF_Q4 ? kFoldLaunchQ4 : kFoldLaunchF16;
-        if (c < best) best = c, s.tile = tab[i].tile, splits = sp;
+        if (c < tile_us) tile_us = c, tile_splits = sp;
       }
+      s.rejected = fminf(s.rejected, fmaxf(s.us, tile_us));
+      if (tile_us < s.us) s.us = tile_us, s.tile = tab[i].tile, splits = tile_splits;
+    }
   }
   const int bm = gemm_tile_rows(s.tile), bn = gemm_tile_cols(s.tile);
   s.gx = (N + bn - 1) / bn;

@@ -26,7 +26,7 @@ EXPORTS = [
     "tlm_abi_version", "tlm_last_error", "tlm_open", "tlm_close", "tlm_sync", "tlm_device_info", "tlm_device_memory",
     "tlm_alloc",
     "tlm_free", "tlm_upload", "tlm_download", "tlm_copy", "tlm_linear_create", "tlm_linear_destroy", "tlm_linear_dequant",
-    "tlm_op_linear", "tlm_op_linear_rows", "tlm_op_rmsnorm", "tlm_op_silu_mul", "tlm_op_gated_mlp", "tlm_attn_create", "tlm_attn_destroy",
+    "tlm_op_linear", "tlm_op_linear_rows", "tlm_rows_plan", "tlm_op_rmsnorm", "tlm_op_silu_mul", "tlm_op_gated_mlp", "tlm_attn_create", "tlm_attn_destroy",
     "tlm_op_attention", "tlm_op_attention_rows", "tlm_op_attention_rows_noalloc", "tlm_attn_reset", "tlm_attn_read_cache", "tlm_op_logits", "tlm_op_argmax",
     "tlm_op_topk", "tlm_read_candidates",
     "tlm_model_create", "tlm_model_destroy", "tlm_model_upload", "tlm_model_finalize", "tlm_model_set_prefill",
@@ -100,6 +100,7 @@ def lib():
             "tlm_linear_dequant": ([VP, VP], ctypes.c_int),
             "tlm_op_linear": ([VP, VP, VP, VP], ctypes.c_int),
             "tlm_op_linear_rows": ([VP, VP, i32, VP, VP], ctypes.c_int),
+            "tlm_rows_plan": ([ctypes.c_int, ctypes.c_int, i32, i32, i32, i32, VP, VP], ctypes.c_int),
             "tlm_op_rmsnorm": ([VP, VP, VP, ctypes.c_int, dbl, ctypes.c_int, VP], ctypes.c_int),
             "tlm_op_silu_mul": ([VP, VP, VP, ctypes.c_int, VP], ctypes.c_int),
             "tlm_op_gated_mlp": ([VP, VP, VP, VP], ctypes.c_int),
@@ -190,6 +191,13 @@ def f32_to_f16(a: np.ndarray) -> np.ndarray:
 
 
 # ------------------------------------------------------------------ context --
+
+def rows_plan(fmt: int, rows: int, n_out: int, k_in: int, cus: int, partial: bool = False):
+    """((block rows, block columns, K slices), predicted us, predicted us of the best other block size)."""
+    plan, us = np.empty(3, np.int32), np.empty(2, np.float32)
+    check(lib().tlm_rows_plan(fmt, int(partial), rows, n_out, k_in, cus, _ptr(plan), _ptr(us)))
+    return tuple(int(v) for v in plan), float(us[0]), float(us[1])
+
 
 class Buffer:
     """A device allocation owned by a Context."""
