@@ -28,21 +28,31 @@ def make_linear(ctx, fmt, w):
     return tlm.Linear(ctx, fmt, np.ascontiguousarray(h.view(np.uint16))), h.astype(np.float32)
 
 
-@pytest.mark.parametrize("fmt,M,N,K,bias", [
+# (format, rows, N, K, bias, the block's rows x columns, whether K goes in slices);
+# test_rows_plan.py holds the planner to the last two without a GPU
+CASES = [
     # four waves splitting K on 32 x 64 tiles: a wave without steps, a ring that
     # is never full, ragged rows and columns
-    (tlm.FMT_F16, 1, 256, 32, True), (tlm.FMT_F16, 31, 65, 96, False), (tlm.FMT_F16, 33, 64, 416, True),
-    (tlm.FMT_F16, 129, 1000, 1056, True),
+    (tlm.FMT_F16, 1, 256, 32, True, (32, 64), False), (tlm.FMT_F16, 31, 65, 96, False, (32, 64), False),
+    (tlm.FMT_F16, 33, 64, 416, True, (32, 64), False), (tlm.FMT_F16, 129, 1000, 1056, True, (32, 64), False),
     # the same in K slices that a second kernel adds; N % 4 != 0 there too
-    (tlm.FMT_F16, 33, 192, 4096, True), (tlm.FMT_F16, 33, 195, 2080, True), (tlm.FMT_Q4, 31, 130, 4096, False),
-    (tlm.FMT_Q4, 257, 300, 8192, True),
+    (tlm.FMT_F16, 33, 192, 4096, True, (32, 64), True), (tlm.FMT_F16, 33, 195, 2080, True, (32, 64), True),
+    (tlm.FMT_Q4, 31, 130, 4096, False, (32, 64), True), (tlm.FMT_Q4, 257, 300, 8192, True, (32, 64), True),
     # 128 x 128 tiles, whole and in slices
-    (tlm.FMT_F16, 1030, 4100, 1024, True), (tlm.FMT_F16, 512, 2048, 4096, False), (tlm.FMT_F16, 700, 10000, 320, True),
+    (tlm.FMT_F16, 1030, 4100, 1024, True, (128, 128), False), (tlm.FMT_F16, 512, 2048, 4096, False, (128, 128), True),
+    (tlm.FMT_F16, 700, 10000, 320, True, (128, 128), False),
     # 256 x 256 tiles: rows and columns past the last whole one, an odd step count
-    (tlm.FMT_F16, 900, 12300, 608, True),
+    (tlm.FMT_F16, 900, 12300, 608, True, (256, 256), False),
     # 128 x 256 tiles (q4), whole and in slices
-    (tlm.FMT_Q4, 900, 8200, 256, True), (tlm.FMT_Q4, 257, 4100, 6048, False),
-])
+    (tlm.FMT_Q4, 900, 8200, 256, True, (128, 256), False), (tlm.FMT_Q4, 257, 4100, 6048, False, (128, 256), True),
+    # few rows over many columns: 64 x 256, 32 x 256 (one and two row tiles) and, fp16, 64 x 128
+    (tlm.FMT_Q4, 61, 65600, 544, True, (64, 256), False), (tlm.FMT_Q4, 63, 65541, 64, False, (32, 256), False),
+    (tlm.FMT_Q4, 17, 131100, 96, True, (32, 256), False), (tlm.FMT_F16, 50, 16450, 160, True, (64, 128), False),
+    (tlm.FMT_F16, 32, 49200, 1056, False, (64, 128), False),
+]
+
+
+@pytest.mark.parametrize("fmt,M,N,K,bias", [c[:5] for c in CASES])
 def test_rows_at_tile_edges(ctx, fmt, M, N, K, bias):
     print(f"[rows] fmt {fmt}, {M} x {N} x {K}", flush=True)
     rng = np.random.default_rng(M * 7 + N + K)

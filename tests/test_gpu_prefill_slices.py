@@ -41,6 +41,32 @@ def test_ragged_chunks_match_replay(storage, n):
     ctx.close()
 
 
+@pytest.mark.parametrize("storage,hidden", [(None, 1024), (None, 512), ("f16", 1024)])
+def test_short_chunk_of_a_wide_mlp_matches_replay(storage, hidden):
+    """64 rows through gate|up of 2 x 32768: the tiles for few rows over many columns, with SwiGLU."""
+    base, n = W.WORKLOADS["llama-3.2-1b"], 64
+    store = base.storage if storage is None else dataclasses.replace(base.storage, linear=storage)
+    cfg = dict(base.config, num_hidden_layers=2, vocab_size=512, hidden_size=hidden, intermediate_size=32768,
+               num_attention_heads=hidden // 64, num_key_value_heads=4, head_dim=64)
+    wl = W.Workload("wide-mlp", cfg, store, n + 1, 6, n + 8, qkv_bias=False)
+    ctx = tlm.Context(0)
+    runner = R.DecoderHIPRunner(W.synthetic(wl), {"maxTokens": n + 8, "prefillChunkSize": 2048}, ctx=ctx)
+    m = runner.model
+    prompt = [int(t) for t in np.random.default_rng(n).integers(0, 512, n + 1)]
+    res = []
+    for least in (0, 64):
+        m.reset_cache()
+        m.set_prefill(least, 2048)
+        m.prefill(prompt, 0, n)
+        m.compute_token(prompt[-1], n, True)
+        # the second layer's cache rows come from the first one's MLP
+        res.append([m.read_logits()] + [a.view(np.float16).astype(np.float32) for a in m.kv_read(1, 0, n)])
+    for a, b in zip(res[1], res[0]):
+        close(a, b, 2e-2, 1e-2)
+    runner.close()
+    ctx.close()
+
+
 def test_chunks_of_several_sizes_on_one_model_equal_fresh_models():
     """A captured chunk goes when a later one has the row buffers replaced: sizes
     in turn and again, over a first set of buffers for chunks of 128 rows and a

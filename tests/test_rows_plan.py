@@ -4,6 +4,7 @@ import pytest
 
 import three_llm_amd.tlm as tlm
 import three_llm_amd.weights as W
+from test_gpu_op_rows import CASES
 
 CUS = 256
 
@@ -32,6 +33,28 @@ def test_short_prompts_keep_the_small_tile_in_slices(rows, n, k):
     (tile_rows, _, slices), us, rejected = tlm.rows_plan(tlm.FMT_Q4, rows, n, k, CUS, partial=True)
     assert tile_rows == 32 and slices > 1
     assert us < 0.75 * rejected
+
+
+@pytest.mark.parametrize("fmt,rows,n,k,tile,sliced", [(c[0], *c[1:4], c[5], c[6]) for c in CASES])
+def test_cases_of_the_op_reach_the_tiles_that_they_are_for(fmt, rows, n, k, tile, sliced):
+    plan, _, _ = tlm.rows_plan(fmt, rows, n, k, CUS)
+    assert plan[:2] == tile and (plan[2] > 1) == sliced
+
+
+@pytest.mark.parametrize("fmt,rows,n,k,tile", [
+    # the edges of the tiles for few rows over many columns
+    (tlm.FMT_Q4, 33, 49153, 896, (64, 256)), (tlm.FMT_Q4, 33, 49152, 896, (32, 64)),
+    (tlm.FMT_Q4, 64, 98304, 512, (32, 256)), (tlm.FMT_Q4, 64, 98305, 512, (64, 256)),
+    (tlm.FMT_Q4, 32, 130817, 1024, (32, 256)), (tlm.FMT_Q4, 32, 130816, 1024, (32, 64)),
+    (tlm.FMT_Q4, 16, 131072, 1056, (32, 64)), (tlm.FMT_Q4, 17, 131072, 1056, (32, 256)),
+    (tlm.FMT_F16, 33, 16385, 896, (64, 128)), (tlm.FMT_F16, 33, 16384, 896, (32, 64)),
+    (tlm.FMT_F16, 33, 16384, 4096, (64, 128)), (tlm.FMT_F16, 32, 49152, 1024, (64, 128)),
+    (tlm.FMT_F16, 32, 49024, 1024, (32, 64)), (tlm.FMT_F16, 8, 98304, 4096, (64, 128)),
+    (tlm.FMT_F16, 8, 98305, 4096, (32, 64)), (tlm.FMT_F16, 1, 151936, 8192, (32, 64)),
+])
+def test_few_rows_over_many_columns(fmt, rows, n, k, tile):
+    plan, _, _ = tlm.rows_plan(fmt, rows, n, k, CUS)
+    assert plan == (*tile, 1)
 
 
 def test_plan_refuses_what_the_op_refuses():

@@ -393,9 +393,15 @@ struct GemmArgs {
 // Tile of a GEMM block: GT_KW one 64-column weight tile and 32 rows whose K
 // range the block's four waves share; the others rows x columns of a block
 // whose waves share its K steps.
-enum GemmTile { GT_KW = 0, GT_128x256, GT_128x128, GT_256x256 };
-inline int gemm_tile_rows(int t) { return t == GT_KW ? 32 : t == GT_256x256 ? 256 : 128; }
-inline int gemm_tile_cols(int t) { return t == GT_KW ? 64 : t == GT_128x128 ? 128 : 256; }
+enum GemmTile { GT_KW = 0, GT_128x256, GT_128x128, GT_256x256, GT_64x256, GT_32x256, GT_64x128 };
+inline int gemm_tile_rows(int t) {
+  constexpr int rows[] = {32, 128, 128, 256, 64, 32, 64};
+  return rows[t];
+}
+inline int gemm_tile_cols(int t) {
+  constexpr int cols[] = {64, 256, 128, 256, 256, 256, 128};
+  return cols[t];
+}
 // Tile and split-K choice of one GEMM (gemm_shape is the only planner, so the
 // host sizes the slice buffers from the same numbers the launch uses).
 struct GemmShape {

@@ -764,13 +764,38 @@ static float gemm_cost(const GemmCost& c, int M, int N, int steps, int splits, i
   return fixed + (spc + c.edge) * (full * (blocks / slots) + (rem == 0 ? 0.f : rem <= cus ? c.one : c.two));
 }
 
+// At most 64 rows over more columns than the fit has: there the K-wave blocks are
+// several rounds of the chip, each with its own handoff, and one wave over all of
+// K on a wider tile is faster.  us, K-wave blocks (or the fit's choice) against:
+//   64 x 256 q4   64 x 65536 x 896    21.9 -> 20.8   64 x 151936 x 896 45.9 -> 31.9   64 x 151936 x 2048 82 -> 56
+//                 (64 x 49152 x 896   17.0 -> 20.1: not there)
+//   32 x 256 q4   64 x 65536 x 512    15.9 -> 15.5   16 x 131072 x 512 16.2 -> 13.7   32 x 131072 x 4096 92 -> 73
+//                 (8 x 151936 x 2048  39.6 -> 43.1, 32 x 98304 x 896 17.9 -> 18.9: not there)
+//   64 x 128 fp16 64 x 17000 x 2048   28.9 -> 22.6   64 x 151936 x 896 82 -> 64       32 x 65536 x 4096 111 -> 98
+//                 (64 x 16384 x 896   9.1 -> 11.6, 16 x 65536 x 896 20.8 -> 20.5, 8 x 128256 x 2048 96 -> 108: not there)
+// -1: not one of these.
+static int wide_tile(int fmt, int M, int N, int K, int cus) {
+  if (M > 64) return -1;
+  if (fmt == WF_Q4) {
+    const int tiles = (N + 255) / 256;
+    if (M > 32) return 4 * tiles <= 3 * cus ? -1 : K <= 512 && 2 * tiles <= 3 * cus ? GT_32x256 : GT_64x256;
+    return tiles >= 2 * cus && (K <= 1024 || M > 16) ? GT_32x256 : -1;
+  }
+  const int tiles = (N + 127) / 128;  // three to a CU
+  if (M > 32) return 2 * tiles > cus || (2 * tiles == cus && K >= 4096) ? GT_64x128 : -1;
+  return 2 * tiles >= 3 * cus && (long)M * K >= 32768 && (M >= 16 || tiles <= 3 * cus) ? GT_64x128 : -1;
+}
+
 GemmShape gemm_shape(int fmt, int epi, int M, int N, int K, int cus, size_t part) {
   GemmShape s;
   const int steps = K >= 32 ? K / 32 : 1;  // K % 32 != 0 is rejected by launch_gemm
   int splits = 1;
   s.tile = GT_KW;
   s.us = s.rejected = INFINITY;
-  if (fmt == WF_Q4 && epi != GEMM_STORE) {
+  const int wide = epi == GEMM_STORE || epi == GEMM_SWIGLU ? wide_tile(fmt, M, N, K, cus) : -1;
+  if (wide >= 0) {
+    s.tile = wide;
+  } else if (fmt == WF_Q4 && epi != GEMM_STORE) {
     // four waves side by side over 256 columns, unless that leaves half the
     // CUs idle: then four waves split K on one tile of 32 rows: 4x the blocks
     // of 128-row tiles, and three blocks fit a CU (53 KB of LDS against
@@ -856,6 +881,9 @@ bool launch_gemm(int fmt, int epi, const GemmShape& sh, const GemmArgs& ga, hipS
     hipLaunchKernelGGL((gemm_ring_kernel<F, MT, WM, WN, NS, E>), grid, dim3(64 * WM * WN), 0, st, g);     \
     return true;                                                                                          \
   }
+#define RING_WIDE(F, TILE, MT, WM, WN, NS)       \
+  RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_STORE) \
+  RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_SWIGLU)
 #define RING_EPIS(F, TILE, MT, WM, WN, NS)       \
   RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_STORE) \
   RING_CASE(F, TILE, MT, WM, WN, NS, GEMM_PART)  \
@@ -866,7 +894,9 @@ bool launch_gemm(int fmt, int epi, const GemmShape& sh, const GemmArgs& ga, hipS
   RING_EPIS(WF_Q4, GT_128x256, 4, 1, 4, 4)
   RING_EPIS(WF_F16, GT_128x128, 2, 2, 2, 4)
   RING_EPIS(WF_F16, GT_256x256, 4, 2, 4, 4)
+  RING_WIDE(WF_Q4, GT_64x256, 2, 1, 4, 4) RING_WIDE(WF_Q4, GT_32x256, 1, 1, 4, 4) RING_WIDE(WF_F16, GT_64x128, 1, 2, 2, 4)
 #undef RING_EPIS
+#undef RING_WIDE
 #undef RING_CASE
 #undef KW_CASE
   return false;
