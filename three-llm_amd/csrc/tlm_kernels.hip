@@ -1308,11 +1308,12 @@ void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* toke
 // steps, so there are no k passes: the k-th largest of a wave's 16 quad maxima
 // is a bound that at least k of its keys reach, so no key below it is among the
 // k best, nor one below the largest such bound of the four waves.  The few keys
-// that remain (k to about 2 k of random scores; at most 32 k per wave) go to
-// LDS, and each one's rank is the number of larger ones.  All keys differ, so
-// ranks do too and the result does not depend on the order in LDS.  151936
-// scores, k = 8: 16.5 us with k passes per wave and k for the merge, 7.5 us so
-// in two levels of blocks.
+// that remain (k to about 3 k of a wave's random scores; at most 8 k, see
+// below) go to LDS, and each one's rank is the number of larger ones.  All keys
+// differ, so ranks do too and the result does not depend on the order in LDS.
+// 151936 scores: k = 8 16.5 us with k passes per wave and k for the merge, 6.6
+// so; k = 16 28.8, 9.6; 9.3 where 15 of the 16 quads hold every score, 19.8
+// where 15 lanes do.
 constexpr int kTopkPer = 8;
 constexpr int kTopkSlice = 256 * kTopkPer;
 
@@ -1337,6 +1338,10 @@ __device__ __forceinline__ void max_u64_step(uint32_t& lo, uint32_t& hi) {
     hi = ohi;
   }
 }
+__device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int l) {
+  return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+}
 struct TopkShared {
   unsigned long long cand[kTopkSlice];
   unsigned long long bound[4];
@@ -1349,29 +1354,35 @@ template <class Put>
 __device__ __forceinline__ void topk_pick(const unsigned long long (&key)[kTopkPer], int k, TopkShared& sh, Put put) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid == 0) sh.count = 0;
-  unsigned long long top = 0;
+  unsigned long long mine = 0;
 #pragma unroll
-  for (int u = 0; u < kTopkPer; u++) top = key[u] > top ? key[u] : top;
+  for (int u = 0; u < kTopkPer; u++) mine = key[u] > mine ? key[u] : mine;
   // the wave's bound: the k-th largest quad maximum (0 while fewer quads hold a candidate)
   static_assert(kTopkMax <= 16, "one of a wave's 16 quads for each of the k best");
-  uint32_t lo = (uint32_t)top, hi = (uint32_t)(top >> 32);
+  uint32_t lo = (uint32_t)mine, hi = (uint32_t)(mine >> 32);
   max_u64_step<kDppXor1>(lo, hi);
   max_u64_step<kDppXor2>(lo, hi);
-  top = ((unsigned long long)hi << 32) | lo;
+  unsigned long long top = ((unsigned long long)hi << 32) | lo;
   int above = 0;
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const unsigned long long o = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)hi, 4 * q) << 32) |
-                                 (uint32_t)__builtin_amdgcn_readlane((int)lo, 4 * q);
-    above += o > top ? 1 : 0;
-  }
+  for (int q = 0; q < 16; q++) above += lane_u64(top, 4 * q) > top ? 1 : 0;
   const unsigned long long at = __builtin_amdgcn_ballot_w64(above == k - 1);
-  if (at) {
-    const int l = __builtin_ctzll(at);
-    top = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)hi, l) << 32) |
-          (uint32_t)__builtin_amdgcn_readlane((int)lo, l);
-  } else {
-    top = 0;
+  top = at ? lane_u64(top, __builtin_ctzll(at)) : 0;
+  // Scores that favour some quads (a mask by position, lists in rank order)
+  // leave many keys above that bound: the k-th largest lane maximum then, which
+  // at most 8 k keys of the wave reach.
+  int reach = 0;
+  if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(mine != 0 && mine >= top)) > k + 6) {
+#pragma unroll
+    for (int u = 0; u < kTopkPer; u++)
+      reach += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[u] != 0 && key[u] >= top));
+  }
+  if (reach > 64) {  // wave-uniform
+    above = 0;
+#pragma unroll 16
+    for (int l = 0; l < 64; l++) above += lane_u64(mine, l) > mine ? 1 : 0;
+    const unsigned long long kth = __builtin_amdgcn_ballot_w64(above == k - 1);
+    if (kth) top = lane_u64(mine, __builtin_ctzll(kth));
   }
   if (lane == 0) sh.bound[wave] = top;
   __syncthreads();
@@ -1384,10 +1395,11 @@ __device__ __forceinline__ void topk_pick(const unsigned long long (&key)[kTopkP
   __syncthreads();
   const int m = sh.count;
   for (int i = tid; i < m; i += 256) {
-    const unsigned long long mine = sh.cand[i];
+    const unsigned long long cand = sh.cand[i];
     int rank = 0;
-    for (int j = 0; j < m; j++) rank += sh.cand[j] > mine ? 1 : 0;
-    if (rank < k) put(rank, mine);
+#pragma unroll 8
+    for (int j = 0; j < m; j++) rank += sh.cand[j] > cand ? 1 : 0;
+    if (rank < k) put(rank, cand);
   }
   if (tid >= m && tid < k) put(tid, 0ull);  // fewer candidates than slots
 }
@@ -1435,8 +1447,11 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const float* __restric
 // The whole selection in one launch, where the blocks' k best together fit one
 // block: each block publishes its keys past its XCD's L2 and counts itself once
 // they are performed; the block that counts last selects from all of them and
-// clears the count.  No block waits.  151936 scores, k = 8: 7.5 us with the
-// merge as a launch of its own, 7.0 us so.
+// clears the count.  No block waits.  The keys lie rank by rank, so that a wave
+// holds every list's best before any list's rest and its bound is a close one
+// (list by list, a quad's four lanes hold neighbouring ranks, and at k = 16 the
+// bound came from ranks 12 to 15: 35.6 us a call, 9.6 so).  151936 scores, k = 8:
+// 7.5 us with the merge as a launch of its own, 6.6 us so.
 __global__ __launch_bounds__(256) void topk_one_kernel(const float* __restrict__ vals, int n, int k, float softcap,
                                                        unsigned long long* keys, unsigned* arrived, float* out_v,
                                                        int* out_i) {
@@ -1449,7 +1464,7 @@ __global__ __launch_bounds__(256) void topk_one_kernel(const float* __restrict__
     return;
   }
   topk_pick(key, k, sh, [&](int r, unsigned long long v) {
-    __hip_atomic_store(keys + blockIdx.x * k + r, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(keys + r * gridDim.x + blockIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   });
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's keys are performed
   __syncthreads();                                  // and every wave's
