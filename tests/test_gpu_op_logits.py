@@ -1,6 +1,6 @@
-"""tlm_op_logits: the token is picked by the last block to finish, so what is
-checked is its choice across blocks (ties, nothing above the lowest score) and
-that one call leaves the next one a clean start."""
+"""tlm_op_logits: the token is picked by the last block to finish or by a merge
+kernel, so what is checked is the choice across blocks (ties, nothing above the
+lowest score) and that one call leaves the next one a clean start."""
 import numpy as np
 import pytest
 
@@ -16,7 +16,8 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("V", [1, 64, 65, 40000])
+# up to 128 blocks and from 128 MiB of weights on: the last block; between: the merge
+@pytest.mark.parametrize("V", [1, 64, 65, 8192, 8193, 40000, 1050000])
 def test_token_across_blocks(ctx, V):
     rng = np.random.default_rng(V)
     K = 64

@@ -1147,17 +1147,26 @@ int tlm_op_logits(tlm_linear* head, const float* x, float* logits, int32_t* toke
   a.cps = p.cps;
   a.in = x;
   a.logits = logits;
-  a.arg_val = ctx->arg_val;
-  a.arg_idx = ctx->arg_idx;
-  // the last block to finish picks the token: a merge kernel of its own took
-  // 4.5 us of 43.4 at 151936 x 896
-  a.arg_key = ctx->arg_key;
-  a.arrived = ctx->arg_arrived;
-  a.token = token;
+  // The last block to finish picks the token, where the blocks are few or end
+  // far enough apart for their atomics on one word: fp16 8192 x 896 7.6 -> 6.8
+  // us, 128256 x 896 35.6 -> 34.6, 151936 x 896 42.0 -> 40.4; 500 blocks that
+  // end together queue for longer than a merge kernel takes: q4 32000 x 512 7.1
+  // -> 10.4, fp16 65536 x 512 12.9 -> 15.0.
+  const size_t bytes = (size_t)head->T * head->C * kTile * (head->fmt == TLM_FMT_Q4 ? 18 : 16);
+  const bool in_head = p.gx <= ctx->cus / 2 || bytes >= (size_t)128 << 20;
+  if (in_head) {
+    a.arg_key = ctx->arg_key;
+    a.arrived = ctx->arg_arrived;
+    a.token = token;
+  } else {
+    a.arg_val = ctx->arg_val;
+    a.arg_idx = ctx->arg_idx;
+  }
   if (gemv_smem_bytes(wfmt(head->fmt), p.cps, p.waves) > 65536)
     return fail(TLM_ERR_INVALID, "TLMLogits: hidden size %d too large for one block", head->K);
   if (!launch_lm_head(wfmt(head->fmt), PRO_COPY, p.waves, p.nch, dim3(p.gx), a, ctx->stream))
     return fail(TLM_ERR_STATE, "TLMLogits: no kernel variant for this shape");
+  if (!in_head) launch_argmax_merge(ctx->arg_val, ctx->arg_idx, p.gx, token, ctx->stream);
   CHECK_LAUNCH("TLMLogits");
   return TLM_OK;
 }

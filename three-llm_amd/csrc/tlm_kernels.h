@@ -198,6 +198,8 @@ size_t gemv_smem_bytes(int fmt, int cps, int waves);
 void launch_rmsnorm(const float* x, const float* w, int n, float eps, int offset, float* y, hipStream_t st);
 void launch_silu_mul(const float* g, const float* u, int n, float* out, hipStream_t st);
 void launch_reduce(const float* part, int n_part, int stride, const float* bias, int n, float* y, hipStream_t st);
+// second pass of the greedy sampler: the best of n (score, id) pairs
+void launch_argmax_merge(const float* pval, const int* pidx, int n, int* token, hipStream_t st);
 void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* token, int blocks, hipStream_t st);
 // The merge of an LM head launch that folded into key (greedy_key order):
 // token, position and step of the control words (ps: the token came from the

@@ -508,10 +508,10 @@ __global__ __launch_bounds__(W * 64) void lm_head_kernel(GemvArgs a) {
   if (wave == 0) {
     wave_argmax(best_v, best_i);
     if (lane == 0) {
-      a.arg_val[blockIdx.x] = best_v;
-      a.arg_idx[blockIdx.x] = best_i;
-      // the merge as it goes: one device-scope atomic max per block
-      if (a.arg_key) {
+      if (!a.arg_key) {  // a second kernel merges the blocks' best
+        a.arg_val[blockIdx.x] = best_v;
+        a.arg_idx[blockIdx.x] = best_i;
+      } else {  // the merge as it goes: one device-scope atomic max per block
         const unsigned long long prev =
             __hip_atomic_fetch_max(a.arg_key, greedy_key(best_v, best_i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a.arrived) {
@@ -1291,9 +1291,13 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float* logits
   }
 }
 
+void launch_argmax_merge(const float* pval, const int* pidx, int n, int* token, hipStream_t st) {
+  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(1024), 0, st, pval, pidx, n, token);
+}
+
 void launch_argmax(const float* logits, int n, float* pval, int* pidx, int* token, int blocks, hipStream_t st) {
   hipLaunchKernelGGL(argmax_partial_kernel, dim3(blocks), dim3(256), 0, st, logits, n, pval, pidx);
-  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(1024), 0, st, pval, pidx, blocks, token);
+  launch_argmax_merge(pval, pidx, blocks, token, st);
 }
 
 // ---------------------------------------------------------------- top-k --
