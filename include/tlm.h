@@ -144,11 +144,10 @@ int tlm_op_attention(tlm_attn* attn, const float* qkv, int position, float* out)
 int tlm_op_attention_rows(tlm_attn* attn, const float* qkv, int32_t rows, int32_t position0, uint16_t* out);
 /* Allocation-free tlm_op_attention_rows.  No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
- * capture, tight serving loops).  The same kernels and results; where the
- * rotated fp16 queries need staging (partial rotary, out inside qkv) they go to
- * a fixed 4 MiB device array of the library (one per device, held until the
- * process ends) instead of a buffer allocated per call, and
- * rows * heads * head_dim * 2 may not exceed 4 MiB in any call (TLM_ERR_RANGE
+ * capture, tight serving loops).  The same kernels and results; the rotated
+ * fp16 queries are staged in a fixed 4 MiB device array of the library (one
+ * per device, held until the process ends) instead of a buffer of the context
+ * or one allocated per call, so rows * heads * head_dim * 2 may not exceed 4 MiB (TLM_ERR_RANGE
  * otherwise).  Enqueue only: no allocation, free or wait.  Every call on one
  * device shares that array, so calls that overlap on one device (other
  * streams or contexts) race. */

@@ -1,9 +1,10 @@
 """tlm_op_attention_rows where its kernel can go wrong: key and query tiles that
 end inside a tile, a softmax reference that moves with every tile or never, rows
-with nothing to see in a tile, and the two ways the queries reach the kernel.
+with nothing to see in a tile, and queries staged in the context's buffer or in one
+of their own.
 
 No rotation (frequencies of zero) and queries and keys on a coarse grid make
-every score exact in fp32; what is left is fp16 probabilities (2^-10 each,
+every score exact in fp32; what is left is fp16 probabilities (2^-11 each,
 rounded to nearest) and the fp16 output, so 2e-3 bounds the error of a
 weighted mean of values of unit scale."""
 import math
@@ -71,7 +72,7 @@ def test_rows_at_tile_edges_and_moving_references(ctx, heads, kv, D, p0, rows, w
 
 @pytest.mark.parametrize("D", [64, 128])
 def test_rows_written_over_their_projections_equal_rows_apart(ctx, D):
-    """out inside qkv: the queries are staged, with the same result."""
+    """out inside qkv: the queries are staged first, so the result is the same."""
     heads, kv, rows = 6, 2, 70
     rng = np.random.default_rng(D)
     x = rng.standard_normal((rows, (heads + 2 * kv) * D)).astype(np.float32)
@@ -83,9 +84,7 @@ def test_rows_written_over_their_projections_equal_rows_apart(ctx, D):
         out = A.rows(qkv, rows, 0, qkv if inside else ctx.buffer(2 * rows * heads * D))
         outs.append(out.read(np.uint16)[:rows * heads * D].copy())
         A.close()
-    # RoPE of the staged queries may be contracted differently: one fp16 step of a query
-    a, b = (o.view(np.float16).astype(np.float64) for o in outs)
-    assert np.abs(a - b).max() <= 2e-3 * np.abs(a).max()
+    assert np.array_equal(*outs)
 
 
 @pytest.mark.parametrize("scale,q0,unit,dims", [(2.0 ** -24, 1.5, 2.0 ** 12, None), (2.0, 49984.0, 2.0 ** -14, 1)])
@@ -103,7 +102,6 @@ def test_queries_round_before_the_softmax_scale(ctx, D, rotary, scale, q0, unit,
     q[:, :, :dims], k[:, :, :dims] = q0, c * unit
     v = (c / 8 + 0.1 * rng.standard_normal((n, 1, D))).astype(np.float16)
     x = np.concatenate([t.reshape(n, -1) for t in (q, k, v)], 1).astype(np.float32)
-    # without rotary dims the queries are staged, with frequencies of zero formed in the kernel
     A = tlm.Attention(ctx, 2, 1, D, n, np.zeros(D // 2, np.float32) if rotary else None, rotary_dim=None if rotary else 0,
                       attn_scale=scale * math.log(2.0))
     got = A.rows(ctx.array(x), n, 0, ctx.buffer(2 * n * 2 * D)).read(np.uint16)
@@ -128,3 +126,23 @@ def test_rows_written_right_after_creation_stay(ctx):
         k, v = A.read_cache(rows)
         A.close()
         assert np.array_equal(np.concatenate([k, v], 1), x[:, heads * D:])
+
+
+def test_queries_past_the_contexts_buffer(ctx):
+    """4100 rows of 32 x 128 queries (33.6 MB) get a buffer of their own: the same
+    rows as in two calls that fit the context's."""
+    heads, kv, D, rows = 32, 2, 128, 4100
+    x = np.random.default_rng(3).standard_normal((rows, (heads + 2 * kv) * D)).astype(np.float32)
+    inv = (1e4 ** (-np.arange(0, D, 2) / D)).astype(np.float32)
+    outs = []
+    for parts in ((rows,), (2048, rows - 2048)):
+        A = tlm.Attention(ctx, heads, kv, D, rows, inv)
+        done = []
+        for n in parts:
+            p = sum(len(d) for d in done)
+            out = ctx.buffer(2 * n * heads * D)
+            done.append(A.rows(ctx.array(x[p:p + n]), n, p, out).read(np.uint16).reshape(n, heads * D))
+        outs.append(np.concatenate(done))
+        A.close()
+    a, b = (o.view(np.float16).astype(np.float64) for o in outs)
+    assert np.abs(a - b).max() <= 2e-3 * np.abs(a).max()

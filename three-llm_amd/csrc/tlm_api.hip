@@ -92,7 +92,9 @@ struct tlm_ctx {
   float* topk_v = nullptr;
   int* topk_i = nullptr;
   void* scratch = nullptr;  // this device's copy of `scratch` (device address)
-  float* part = nullptr;    // split-K slices (or unaligned rows) of tlm_op_linear_rows (kPartFloats)
+  // split-K slices (or unaligned rows) of tlm_op_linear_rows, staged queries of
+  // tlm_op_attention_rows (kPartFloats)
+  float* part = nullptr;
   std::mutex part_mu;
 };
 constexpr size_t kPartFloats = (size_t)8 << 20;  // 32 MiB
@@ -969,7 +971,7 @@ int tlm_op_attention(tlm_attn* A, const float* qkv, int position, float* out) {
 
 // RoPE + cache append of `rows` positions from position0, then their causal
 // attention, enqueued on the context's stream; q: fp16 staging of the rotated
-// queries, [rows][heads * head_dim], or null where none is needed.
+// queries, [rows][heads * head_dim].
 static int check_attention_rows(const tlm_attn* A, const float* qkv, int32_t rows, int32_t position0,
                                 const uint16_t* out) {
   if (!A || !qkv || !out || rows <= 0) return fail(TLM_ERR_INVALID, "TLMAttention: invalid argument");
@@ -980,17 +982,6 @@ static int check_attention_rows(const tlm_attn* A, const float* qkv, int32_t row
   if (d.kv_fmt == TLM_FMT_F32 || (d.head_dim != 64 && d.head_dim != 128))
     return fail(TLM_ERR_INVALID, "TLMAttention: batched rows need an fp16 cache and head_dim 64 or 128");
   return TLM_OK;
-}
-
-// With full rotary the attention kernel forms its queries itself, from qkv,
-// which out may not share an address with (a block writes its rows of out while
-// others still read theirs of qkv); otherwise q stages them.
-static bool rows_need_staging(const tlm_attn* A, const float* qkv, int32_t rows, const uint16_t* out) {
-  const tlm_attn_desc& d = A->d;
-  const uintptr_t x = reinterpret_cast<uintptr_t>(qkv), o = reinterpret_cast<uintptr_t>(out);
-  const size_t nx = sizeof(float) * (size_t)rows * (d.heads + 2 * d.kv_heads) * d.head_dim;
-  const size_t no = sizeof(uint16_t) * (size_t)rows * d.heads * d.head_dim;
-  return d.rotary_dim != d.head_dim || (x < o + no && o < x + nx);
 }
 
 static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, int32_t position0, uint16_t* out,
@@ -1006,7 +997,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   r.p0 = position0;
   r.Hq = d.heads;
   r.Hkv = d.kv_heads;
-  r.h0 = q ? 0 : d.heads;
   r.D = d.head_dim;
   r.rd = d.rotary_dim;
   r.max_tokens = d.max_tokens;
@@ -1019,11 +1009,6 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
   PrefillAttnArgs pa;
   memset(&pa, 0, sizeof pa);
   pa.q = q;
-  if (!q) {
-    pa.qkv = qkv;
-    pa.rope_cos = A->rope_cos;
-    pa.rope_sin = A->rope_sin;
-  }
   pa.kc = A->kc;
   pa.vc = A->vc;
   pa.out = out;
@@ -1042,13 +1027,20 @@ static bool enqueue_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, 
 int tlm_op_attention_rows(tlm_attn* A, const float* qkv, int32_t rows, int32_t position0, uint16_t* out) {
   int rc = check_attention_rows(A, qkv, rows, position0, out);
   if (rc) return rc;
-  uint16_t* q = nullptr;
-  if (rows_need_staging(A, qkv, rows, out))
-    HIP_TRY(hipMalloc(&q, sizeof(uint16_t) * (size_t)rows * A->d.heads * A->d.head_dim));
-  const bool launched = enqueue_attention_rows(A, qkv, rows, position0, out, q);
+  // The queries are staged in the context's slices' buffer (a buffer allocated and
+  // freed per call took 35 us from 2 MiB on); past its size they get their own.
+  const size_t need = sizeof(uint16_t) * (size_t)rows * A->d.heads * A->d.head_dim;
+  uint16_t* own = nullptr;
+  if (need > kPartFloats * sizeof(float)) HIP_TRY(hipMalloc(&own, need));
+  bool launched;
+  {
+    std::lock_guard<std::mutex> lock(A->ctx->part_mu);
+    launched =
+        enqueue_attention_rows(A, qkv, rows, position0, out, own ? own : reinterpret_cast<uint16_t*>(A->ctx->part));
+  }
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(A->ctx->stream);
-  if (q) hipFree(q);
+  if (own) hipFree(own);
   if (e != hipSuccess) return fail(TLM_ERR_HIP, "TLMAttention: batched rows failed: %s", hipGetErrorString(e));
   if (!launched) return fail(TLM_ERR_STATE, "TLMAttention: no batched attention kernel for this shape");
   return TLM_OK;
@@ -1063,8 +1055,7 @@ int tlm_op_attention_rows_noalloc(tlm_attn* A, const float* qkv, int32_t rows, i
                 "entry point holds %zu (at most %zu rows of this shape)", rows, need, kScratchBytes,
                 kScratchBytes / (sizeof(uint16_t) * A->d.heads * A->d.head_dim));
   if (!A->ctx->scratch) return fail(TLM_ERR_STATE, "TLMAttention: the context has no scratch address");
-  uint16_t* q = rows_need_staging(A, qkv, rows, out) ? static_cast<uint16_t*>(A->ctx->scratch) : nullptr;
-  if (!enqueue_attention_rows(A, qkv, rows, position0, out, q))
+  if (!enqueue_attention_rows(A, qkv, rows, position0, out, static_cast<uint16_t*>(A->ctx->scratch)))
     return fail(TLM_ERR_STATE, "TLMAttention: no batched attention kernel for this shape");
   CHECK_LAUNCH("TLMAttention");
   return TLM_OK;

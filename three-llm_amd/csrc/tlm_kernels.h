@@ -434,11 +434,6 @@ struct RowsArgs {
 };
 struct PrefillAttnArgs {
   const uint16_t* q;    // fp16 [M][Hq D], RoPE applied
-  // non-null qkv (full rotary; out apart from it): the queries come from the
-  // fp32 projected rows [M][(Hq + 2 Hkv) D] instead, rotated in the kernel
-  const float* qkv;
-  const float* rope_cos;  // [max_tokens][D / 2]
-  const float* rope_sin;
   const void* kc;       // fp16 [Hkv][max_tokens][D] (this layer)
   const void* vc;
   uint16_t* out;        // fp16 [M][Hq D]
@@ -452,7 +447,6 @@ struct RopeKvArgs {
   size_t pstride;       // floats between slices
   const float* bias;    // [Nqkv] or null
   int M, p0, Hq, Hkv, D, rd, max_tokens;
-  int h0;               // first head of a row taken (q heads, then k, then v): Hq leaves the queries alone
   const float* rope_cos;  // [max_tokens][rd / 2]
   const float* rope_sin;
   uint16_t* q;          // fp16 [M][Hq D]

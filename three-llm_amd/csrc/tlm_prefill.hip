@@ -1043,7 +1043,7 @@ __device__ __forceinline__ void rope_pair(const RopeKvArgs& a, int pi, int& i0, 
 constexpr int RKV_ROWS = 2;
 __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
   const int D = a.D, width = (a.Hq + 2 * a.Hkv) * D;
-  const int pi = a.h0 * (D / 2) + blockIdx.y * blockDim.x + threadIdx.x;
+  const int pi = blockIdx.y * blockDim.x + threadIdx.x;
   if (pi >= width / 2) return;
   int i0, i1, dr;
   bool rot;
@@ -1102,7 +1102,7 @@ __device__ __forceinline__ void rope_store4(const RopeKvArgs& a, int m, int pos,
 
 __global__ __launch_bounds__(256) void rope_kv4_kernel(RopeKvArgs a) {
   const int D = a.D, g8 = D / 8, groups = (a.Hq + 2 * a.Hkv) * g8, half = D / 2;
-  const int g = a.h0 * g8 + blockIdx.y * blockDim.x + threadIdx.x;
+  const int g = blockIdx.y * blockDim.x + threadIdx.x;
   if (g >= groups) return;
   const int h = g / g8, j = g - h * g8;
   const bool rot = h < a.Hq + a.Hkv;
@@ -1143,7 +1143,7 @@ static const bool g_rope_vec = [] {
 
 void launch_rope_kv(const RopeKvArgs& a, hipStream_t st) {
   const bool vec = g_rope_vec && !a.kv_f32 && a.rd == a.D && a.D % 8 == 0 && a.pstride % 4 == 0;
-  const int work = (a.Hq + 2 * a.Hkv - a.h0) * a.D / (vec ? 8 : 2);  // threads per row
+  const int work = (a.Hq + 2 * a.Hkv) * a.D / (vec ? 8 : 2);  // threads per row
   const int bt = min(256, (work + 63) / 64 * 64);
   const dim3 grid((a.M + RKV_ROWS - 1) / RKV_ROWS, (work + bt - 1) / bt);
   if (vec)
@@ -1218,7 +1218,7 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 // A score may exceed the softmax's reference by this much (log2) before it moves
 constexpr float kRefSlack = 8.f;
 
-template <int DT, int NG, bool QF>
+template <int DT, int NG>
 __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 64 ? 4 : 2))) void prefill_attn_kernel(PrefillAttnArgs a) {
   using AT = AttnTile<DT>;
   constexpr int KT = AT::KT, NDT = DT / 32;
@@ -1245,29 +1245,9 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
   const int QW = a.Hq * DT;
 
   half8_t qb[DT / 16];
-  if constexpr (QF) {  // the lane's query row from its fp32 projection: RoPE pairs (d, d + DT / 2)
-    const int m = min(qr, a.M - 1);
-    const float* x = a.qkv + (size_t)m * (a.Hq + 2 * a.Hkv) * DT + h * DT;
-    const float* ct = a.rope_cos + (size_t)(p0 + m) * (DT / 2);
-    const float* st = a.rope_sin + (size_t)(p0 + m) * (DT / 2);
+  const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)min(qr, a.M - 1) * QW + h * DT;
 #pragma unroll
-    for (int j = 0; j < DT / 32; j++)
-#pragma unroll
-      for (int e = 0; e < 8; e += 4) {
-        const int d = 16 * j + 8 * kh + e;
-        const float4 u = *reinterpret_cast<const float4*>(x + d), v = *reinterpret_cast<const float4*>(x + d + DT / 2);
-        const float4 c = *reinterpret_cast<const float4*>(ct + d), s = *reinterpret_cast<const float4*>(st + d);
-        half8_t &lo = qb[j], &hi = qb[j + DT / 32];
-        lo[e] = (_Float16)(u.x * c.x - v.x * s.x), hi[e] = (_Float16)(v.x * c.x + u.x * s.x);
-        lo[e + 1] = (_Float16)(u.y * c.y - v.y * s.y), hi[e + 1] = (_Float16)(v.y * c.y + u.y * s.y);
-        lo[e + 2] = (_Float16)(u.z * c.z - v.z * s.z), hi[e + 2] = (_Float16)(v.z * c.z + u.z * s.z);
-        lo[e + 3] = (_Float16)(u.w * c.w - v.w * s.w), hi[e + 3] = (_Float16)(v.w * c.w + u.w * s.w);
-      }
-  } else {
-    const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)min(qr, a.M - 1) * QW + h * DT;
-#pragma unroll
-    for (int j = 0; j < DT / 16; j++) qb[j] = *reinterpret_cast<const half8_t*>(qrow + 16 * j + 8 * kh);
-  }
+  for (int j = 0; j < DT / 16; j++) qb[j] = *reinterpret_cast<const half8_t*>(qrow + 16 * j + 8 * kh);
 
   // this wave's copies of a tile: slot 64 u + lane of its K (and V) holds piece
   // cq[u] of row cr[u] (rows past qhi repeat row qhi: their keys are masked)
@@ -1431,15 +1411,12 @@ __global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(DT == 
 bool launch_prefill_attention(const PrefillAttnArgs& a, hipStream_t st) {
   // four query heads per block (waves past the group's heads only stage K/V)
   const dim3 grid((a.M + 31) / 32, a.Hkv, (a.G + 3) / 4);
-  if (a.D != 64 && a.D != 128) return false;
-  if (a.D == 64 && a.qkv)
-    hipLaunchKernelGGL((prefill_attn_kernel<64, 2, true>), grid, dim3(512), 0, st, a);
-  else if (a.D == 64)
-    hipLaunchKernelGGL((prefill_attn_kernel<64, 2, false>), grid, dim3(512), 0, st, a);
-  else if (a.qkv)
-    hipLaunchKernelGGL((prefill_attn_kernel<128, 1, true>), grid, dim3(256), 0, st, a);
+  if (a.D == 64)
+    hipLaunchKernelGGL((prefill_attn_kernel<64, 2>), grid, dim3(512), 0, st, a);
+  else if (a.D == 128)
+    hipLaunchKernelGGL((prefill_attn_kernel<128, 1>), grid, dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((prefill_attn_kernel<128, 1, false>), grid, dim3(256), 0, st, a);
+    return false;
   return true;
 }
 
