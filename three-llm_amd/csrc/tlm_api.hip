@@ -206,8 +206,6 @@ struct tlm_model {
   float *pq = nullptr, *po = nullptr;
   int mlp_nch = 1, mlp_ndb = 1;
   float* logits = nullptr;
-  float* arg_val = nullptr;
-  int* arg_idx = nullptr;
   unsigned long long* arg_key = nullptr;  // the LM head's folded argmax (zero between launches)
   unsigned* arg_arrived = nullptr;        // LM head blocks done, for its in-launch merge (zero between launches)
   float* cand_v = nullptr;  // top-k candidates of the last logits (kTopkMax)
@@ -1454,8 +1452,6 @@ int tlm_model_create(tlm_ctx* ctx, const tlm_model_desc* d, tlm_model** out) {
       rc = fail(TLM_ERR_INVALID, "TLMModel: hidden size %d too large for one LM head block", H);
   }
   M_TRY(model_alloc((void**)&m->logits, sizeof(float) * d->vocab_size));
-  M_TRY(model_alloc((void**)&m->arg_val, sizeof(float) * 4096));
-  M_TRY(model_alloc((void**)&m->arg_idx, sizeof(int) * 4096));
   M_TRY(model_alloc((void**)&m->arg_key, sizeof(unsigned long long)));
   M_TRY(model_alloc((void**)&m->arg_arrived, sizeof(unsigned)));
   M_TRY(model_alloc((void**)&m->cand_v, sizeof(float) * kTopkMax));
@@ -1500,7 +1496,7 @@ void tlm_model_destroy(tlm_model* m) {
   tlm_linear_destroy(m->head);
   attn_free(&m->attn, false);
   void* bufs[] = {m->emb, m->final_norm, m->ctrl, m->tokens_out, m->prompt, m->xa, m->x0, m->xf, m->attn_out,
-                  m->pq, m->po, m->rb, m->logits, m->arg_val, m->arg_idx, m->arg_key, m->arg_arrived, m->cand_v, m->cand_i, m->pf_x, m->pf_part, m->pf_xn,
+                  m->pq, m->po, m->rb, m->logits, m->arg_key, m->arg_arrived, m->cand_v, m->cand_i, m->pf_x, m->pf_part, m->pf_xn,
                   m->pf_q, m->pf_att, m->pf_h, m->pf_ex, m->pf_ss, m->pf_ovf, m->ps_layers, m->ps_roles, m->ps_pub_x, m->ps_pub_qkv,
                   m->ps_pub_o, m->ps_pub_xm, m->ps_pub_h, m->ps_args_dev, m->ps_xcc};
   for (void* p : bufs) hipFree(p);
@@ -1697,8 +1693,6 @@ static bool enqueue_head(tlm_model* m, hipStream_t st, bool advance, hipEvent_t*
   a.ctrl = m->ctrl;  // fixed-point range flag of the residual it reads
   a.xnorm = m->xf;
   a.logits = m->logits;
-  a.arg_val = m->arg_val;
-  a.arg_idx = m->arg_idx;
   a.arg_key = m->arg_key;  // the blocks fold their bests as they finish
   // after a persistent step the head's last block also does the merge
   // (TLM_HEAD_MERGE=0: greedy_pick_kernel, comparisons)

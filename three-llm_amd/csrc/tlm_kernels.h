@@ -100,7 +100,7 @@ struct GemvArgs {
   // LM head
   float* xnorm;        // with an RMS prologue: block 0 stores the normalised input here (may be null)
   float* logits;       // full logits (may be null)
-  float* arg_val;      // per-block argmax partials
+  float* arg_val;      // per-block argmax partials (with arg_key null)
   int* arg_idx;
   int* tokens_out;     // greedy stream (indexed by ctrl[C_STEP]), may be null
   int advance;         // 1: the merge advances ctrl (token <- argmax, pos++, step++)
