@@ -46,7 +46,10 @@ Q4, F16 = tlm.FMT_Q4, tlm.FMT_F16
 @pytest.mark.parametrize("fmt,n,k", [(Q4, 1, 32), (Q4, 9, 64), (Q4, 1535, 96), (Q4, 3071, 160), (Q4, 3073, 416),
                                      (Q4, 6145, 384), (Q4, 12289, 224), (Q4, 65, 10624), (Q4, 65, 10656),
                                      (Q4, 12300, 10688), (F16, 1, 1), (F16, 8, 8), (F16, 1537, 30), (F16, 3100, 136),
-                                     (F16, 6200, 97), (F16, 12290, 40), (F16, 33, 10920), (F16, 33, 10931)])
+                                     (F16, 6200, 97), (F16, 12290, 40), (F16, 33, 10920), (F16, 33, 10931),
+                                     # four blocks a CU and more: 4, 8 and 16 waves by the chunks
+                                     (Q4, 65473, 736), (Q4, 65473, 768), (Q4, 65473, 1536), (F16, 65480, 190),
+                                     (F16, 65480, 192), (F16, 65480, 385)])
 def test_linear_at_block_and_slice_edges(ctx, fmt, n, k):
     rng = np.random.default_rng(n * 31 + k)
     lin, w = make(ctx, fmt, n, k, rng)

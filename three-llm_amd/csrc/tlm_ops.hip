@@ -148,7 +148,11 @@ __global__ __launch_bounds__(W * 64) void op_gemv_kernel(OpGemvArgs a) {
 // 3072, SwiGLU: 7.2 us at 32 rows = 256 blocks, 8.5 at 16, 8.1 at 64 = 128; 2048
 // at K 8192: 5.1 at 8 or 16, 7.0 at 32 = 64 blocks).  Waves: one for each chunk
 // group of the block up to 16 (896 x 4864, 19 groups: 3.2 us with 16 waves, 3.4
-// with 8, 4.4 with 4; 1152 x 896, 3.5 groups: 2.35 with 4, 2.65 with 16).
+// with 8, 4.4 with 4; 1152 x 896, 3.5 groups: 2.35 with 4, 2.65 with 16).  From
+// four blocks a CU on the blocks fill the chip by themselves and a wave has at
+// least three groups, as its start and the sum at the end cost more than what
+// it hides: q4 151936 x 256 6.4 -> 5.3 us, x 896 16.2 -> 14.2, 65536 x 896 7.5 ->
+// 6.1, fp16 65536 x 256 5.8 -> 4.3.
 bool launch_op_gemv(int fmt, bool swiglu, const OpGemvArgs& aa, int cus, hipStream_t st) {
   OpGemvArgs a = aa;
   // x and its sums in at most 48 KB of LDS
@@ -158,8 +162,10 @@ bool launch_op_gemv(int fmt, bool swiglu, const OpGemvArgs& aa, int cus, hipStre
   const int rows = swiglu ? a.N / 2 : a.N;
   int R = 64;
   while (R > 8 && (rows + R - 1) / R < 3 * cus / 4) R /= 2;
-  const int groups = (a.cps * R + 63) / 64, W = groups >= 12 ? 16 : groups >= 6 ? 8 : 4;
   const dim3 grid((rows + R - 1) / R);
+  const int groups = (a.cps * R + 63) / 64;
+  const bool many = (int)grid.x >= 4 * cus;
+  const int W = groups >= (many ? 48 : 12) ? 16 : groups >= (many ? 24 : 6) ? 8 : 4;
   const size_t smem = a.cps * per_chunk + sizeof(float) * (swiglu ? 2 : 1) * W * R;
 #define OPG(F, RV, WV)                                                                                       \
   if (fmt == F && R == RV && W == WV) {                                                                      \
