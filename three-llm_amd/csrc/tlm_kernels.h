@@ -64,7 +64,7 @@ __host__ __device__ inline ChunkPlan chunk_plan(int pos, int window, int nsplit,
 enum Ctrl { C_TOKEN = 0, C_POS = 1, C_STEP = 2, C_BASE = 3, C_LEN = 4, C_SEQ = 5, C_FXR = 6, C_ERR = 7 };
 
 // Embedding row staging: the kernels that choose the next token (set_ctrl,
-// prefill_advance, argmax_merge) also write its embedding row, in fixed point,
+// prefill_advance, greedy_pick) also write its embedding row, in fixed point,
 // to replica 0 of x0, the residual accumulator layer 0 reads (replicas 1..3
 // stay zero).  x0 == null disables the copy.
 struct EmbStage {

@@ -820,8 +820,8 @@ bool launch_mlp(int fmt, int nch, int ndb, int blocks, const MlpArgs& m, hipStre
 
 int attn_lpp(int D, bool kv_f32) { return head_tiling(attn_dt(D), kv_f32 ? 4 : 2).lpp; }
 
-// LDS of a head_kernel block: one wave region per wave, then (long windows)
-// the merge area [kAttnWaves][2 + DT] (max, sum, unnormalised output of each wave).
+// LDS of a head_kernel block of nw waves: one region per wave, then (more than
+// one wave) the merge area [nw][2 + DT] (max, sum, unnormalised output of each wave).
 static size_t head_smem_bytes(int D, bool kv_f32, int nw) {
   const int dt = attn_dt(D), esz = kv_f32 ? 4 : 2;
   return sizeof(float) * ((size_t)nw * head_wave_floats(dt, esz) + (nw > 1 ? (size_t)nw * (2 + dt) : 0));
@@ -894,8 +894,9 @@ __global__ __launch_bounds__(64 * (ONE ? kOneWaves : LONG ? kAttnWaves : 1)) voi
   if (pos < 0 || pos >= a.max_tokens) return;
   const ChunkPlan cp = chunk_plan(pos, a.window, a.nsplit, a.chmin);
   if (c >= cp.nact) return;
-  // the block's chunk [b0, b1), split over nwu <= kAttnWaves waves of at least
-  // 32 positions (block-uniform); this wave's part [t0, t1) may be empty
+  // the block's chunk [b0, b1), split over nwu waves (block-uniform): LONG up to
+  // kAttnWaves of at least 32 positions, ONE all of the block's, a pass (SUB
+  // positions) each; this wave's part [t0, t1) may be empty
   const int b0 = cp.first + c * cp.chunk, b1 = min(b0 + cp.chunk, pos + 1);
   const int nwu = ONE ? NW : LONG ? min(NW, (b1 - b0 + 31) / 32) : 1;
   if (nwu == 1 && wv != 0) return;  // one wave does the whole chunk, no merge

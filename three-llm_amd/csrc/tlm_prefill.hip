@@ -1172,11 +1172,12 @@ void launch_rope_kv(const RopeKvArgs& a, hipStream_t st) {
 // Queries are fp16 as rotated and the scale multiplies the fp32 scores: scaled
 // before the rounding they would run into fp16's subnormals or past its largest
 // value sooner.  P is rounded to nearest for the product with V, and its sum
-// adds the 32-bit values: 3.0e-4 from 64 bits at 2048 rows, 3.4e-4 with both from
-// P rounded toward zero and the queries scaled first, at the same speed (36.8
-// and 36.9 us).  rocprofv3, 2048 rows, registers staging the tiles and O
-// rescaled with every new maximum against this: Llama-3.2-1B heads 39.0 -> 36.8
-// us from position 0, 88.0 -> 75.2 from 2048; Llama-3.2-3B heads 67.4 -> 54.5.
+// adds the 32-bit values: 3.1e-4 from 64 bits at 2048 rows, 3.4e-4 with both from
+// P rounded toward zero and the queries scaled first.  rocprofv3, 2048 rows,
+// registers staging the tiles and O rescaled with every new maximum against
+// this: Llama-3.2-1B heads 39.4 -> 31.3 us from position 0, 87.5 -> 70.7 from
+// 2048; Llama-3.2-3B heads 67.8 -> 48.1.  Queries formed here from their fp32
+// projection took 5 us more (rows 12 KB apart: 64 lines a load).
 // Four waves per SIMD need <= 128 registers, hence the copies.
 template <int DT>
 struct AttnTile {
