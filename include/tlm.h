@@ -94,7 +94,8 @@ int tlm_op_linear(tlm_linear* lin, const float* x, const float* bias, float* y);
  * prefill's linear; the reference applies TSLLinear once per replayed token,
  * DecoderTSLRunner.ts:472-480).  x: fp16 bits device [rows][K] (K % 32 == 0),
  * y: fp32 device [rows][N].  W is dequantised to fp16 ((code - 8) * s rounded
- * once), products accumulate in fp32.  Enqueue only. */
+ * once), products accumulate in fp32.  x may start at any address; one that is no
+ * multiple of 16 bytes costs a copy of the rows.  Enqueue only. */
 int tlm_op_linear_rows(tlm_linear* lin, const uint16_t* x, int32_t rows, const float* bias, float* y);
 /* How a batched linear of that size runs on `cus` compute units: plan[0] rows by
  * plan[1] columns of a block, plan[2] slices of K; us[0] the predicted time of
@@ -133,7 +134,9 @@ typedef struct tlm_attn_desc {
 int tlm_attn_create(tlm_ctx* ctx, const tlm_attn_desc* desc, tlm_attn** out);
 void tlm_attn_destroy(tlm_attn* attn);
 /* qkv: fp32 device [(heads + 2 kv_heads) * head_dim] (packed Q|K|V, pre-RoPE);
- * out: fp32 device [heads * head_dim]. */
+ * out: fp32 device [heads * head_dim], anywhere, also over qkv.  q and the
+ * probabilities are fp32, past 1024 positions over an fp16 cache (head_dim 64 or
+ * 128) pairs of fp16 values: |q| * attn_scale * log2 e below 65520 there. */
 int tlm_op_attention(tlm_attn* attn, const float* qkv, int position, float* out);
 /* `rows` consecutive positions position0.. at once (the batched prefill's
  * attention; the reference runs TSLAttention once per replayed token): qkv fp32
